@@ -266,40 +266,6 @@ void appendTask( BatchPlan::Step& s, Task t, int blocks )
 }
 
 template < typename T >
-SweepArgs< T > sweepArgs( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol, int L, const StencilCall& c, int cfg )
-{
-   constexpr bool dbl = std::is_same< T, double >::value;
-   const int      nC  = m.mesh->nC();
-   const int      nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
-   SweepArgs< T > p;
-   p.segs    = g.zSegs[cfg];
-   p.nSegs   = g.nZSegs[cfg];
-   p.nC      = nC;
-   p.L       = L;
-   p.flag    = c.flag;
-   p.stride  = g.stride;
-   p.cellSt  = dbl ? (const T*) ol.cellSt : (const T*) ol.cellStF;
-   p.cfs     = m.cellFaces;
-   p.entryW  = dbl ? (const T*) ol.entryW : (const T*) ol.entryWF;
-   p.primInv = dbl ? (const T*) ol.primInv : (const T*) ol.primInvF;
-   p.part    = dbl ? (T*) ol.facePart : (T*) ol.facePartF;
-   p.x       = (const T*) c.x;
-   p.in1     = (const T*) c.in1;
-   p.out0    = (T*) c.out0;
-   p.out1    = (T*) c.out1;
-   p.a       = T( c.a );
-   p.items   = g.flatItems;
-   p.nItems  = nFace > 0 ? g.nFlatItems : 0;
-   p.chunks  = g.chunks;
-   p.nChunks = nLow;
-   p.prims   = m.prims;
-   p.entries = m.entries;
-   p.gC      = p.nSegs > 0 ? xcdGrid( ( ( p.nSegs + 3 ) / 4 ) * nC ) : 0;
-   p.gF      = p.nItems > 0 ? xcdGrid( ceilDiv( p.nItems, 4 ) ) : 0;
-   return p;
-}
-
-template < typename T >
 void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item >& items, int cfg )
 {
    constexpr bool   dbl = std::is_same< T, double >::value;
@@ -339,13 +305,13 @@ void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item 
       {
          t.kind          = 0;
          t.sw            = sweepArgs< T >( m, g, ol, it.L, c, cfg );
-         const int gL    = nLow > 0 ? xcdGrid( ceilDiv( nLow, kBlock / 64 ) ) : 0;
+         const int gL    = t.sw.nChunks > 0 ? xcdGrid( ceilDiv( t.sw.nChunks, kBlock / 64 ) ) : 0;
          appendTask( st, t, t.sw.gC + t.sw.gF + gL );
          f.kind    = 0;
          f.part    = dbl ? (const T*) ol.facePart : (const T*) ol.facePartF;
          f.primInv = dbl ? (const T*) ol.primInv : (const T*) ol.primInvF;
          f.dinv    = nullptr;
-         appendTask( cb, f, nFace > 0 ? xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) : 0 );
+         appendTask( cb, f, nFace > 0 && t.sw.faces ? xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) : 0 );
       }
       else
       {

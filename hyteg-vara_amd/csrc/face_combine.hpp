@@ -20,18 +20,17 @@ __device__ __forceinline__ void bFaceCombine( int bid, const LowerChunk* __restr
    const int ci = remapXcd( bid, nb ) * ( kBlock / 64 ) + __builtin_amdgcn_readfirstlane( int( threadIdx.x >> 6 ) );
    if ( ci >= nChunks )
       return;
-   const LowerChunk ch = chunks[ci];
-   const LowerPrim  p  = prims[ch.prim];
+   const LowerChunk ch   = chunks[ci];
    const int        lane = int( threadIdx.x & 63 );
-   if ( !( p.bc & flag ) || lane >= ch.n )
+   if ( !( ch.bc & flag ) || lane >= ch.n )
       return;
    const int N = 1 << L, NP = N + 1, w = N + 1;
    const int i = ch.i0 + lane, j = ch.j, f = ch.prim - firstFacePrim;
    T         Ax = T( 0 );
    i64       o[2];
-   for ( int k = 0; k < p.nCells; ++k )
+   for ( int k = 0; k < ch.nCells; ++k )
    {
-      const LowerEntry e = entries[p.entry0 + k];
+      const LowerEntry e = entries[ch.entry0 + k];
       int              qx, qy, qz;
       entryPos( e, N, i, j, qx, qy, qz );
       o[k] = i64( e.cell ) * stride + cidx( w, qx, qy, qz );
@@ -46,7 +45,7 @@ __device__ __forceinline__ void bFaceCombine( int bid, const LowerChunk* __restr
       ov = out0[o[0]];
    const T dinv = dinvArr ? dinvArr[o[0]] : ( primInv ? primInv[ch.prim] : T( 1 ) );
    epilogue< T, MODE >( Ax, xc, i1, ov, dinv, a, r0, r1 );
-   for ( int k = 0; k < p.nCells; ++k )
+   for ( int k = 0; k < ch.nCells; ++k )
    {
       out0[o[k]] = r0;
       if constexpr ( MODE == MODE_CHEB0 || MODE == MODE_CHEBK )
@@ -91,26 +90,25 @@ __global__ __launch_bounds__( kBlock ) void kFaceCombineSor( const LowerChunk* _
    if ( ci >= nChunks )
       return;
    const LowerChunk ch   = chunks[ci];
-   const LowerPrim  p    = prims[ch.prim];
    const int        lane = int( threadIdx.x & 63 );
-   if ( !( p.bc & flag ) || lane >= ch.n )
+   if ( !( ch.bc & flag ) || lane >= ch.n )
       return;
    const int N = 1 << L, NP = N + 1, w = N + 1;
    const int i = ch.i0 + lane, j = ch.j, f = ch.prim - firstFacePrim;
-   if ( sorColour( cinfo, entries[p.entry0], N, i, j, sorM ) != sorK )
+   if ( sorColour( cinfo, entries[ch.entry0], N, i, j, sorM ) != sorK )
       return;
    T   Ax = T( 0 );
    i64 o[2];
-   for ( int k = 0; k < p.nCells; ++k )
+   for ( int k = 0; k < ch.nCells; ++k )
    {
-      const LowerEntry e = entries[p.entry0 + k];
+      const LowerEntry e = entries[ch.entry0 + k];
       int              qx, qy, qz;
       entryPos( e, N, i, j, qx, qy, qz );
       o[k] = i64( e.cell ) * stride + cidx( w, qx, qy, qz );
       Ax += part[i64( 2 * f + k ) * NP * NP + facePartIndex( entrySlot( e ), N, qx, qy, qz )];
    }
    const T v = x[o[0]] + a * primInv[ch.prim] * ( b[o[0]] - Ax );
-   for ( int k = 0; k < p.nCells; ++k )
+   for ( int k = 0; k < ch.nCells; ++k )
       x[o[k]] = v;
 }
 
@@ -155,19 +153,21 @@ __device__ __forceinline__ void bLowCombine( int bid, const LowerChunk* __restri
    const int ci = bid * ( kBlock / 64 ) + int( threadIdx.x >> 6 );
    if ( ci >= nChunks )
       return;
-   const LowerChunk ch   = chunks[ci];
-   const LowerPrim  p    = prims[ch.prim];
-   const int        lane = int( threadIdx.x & 63 );
-   if ( !( p.bc & flag ) || lane >= ch.n )
+   const LowerChunk ch = chunks[ci];
+   if ( !( ch.bc & flag ) )
       return;
-   const int N = 1 << L, w = N + 1, NP = N + 1;
-   const int i = ch.i0 + lane;
-   T         Ax = T( 0 );
-   for ( int k = 0; k < p.nCells; ++k )
-      Ax += lowPart[i64( p.entry0 + k ) * NP + i];
+   const ChunkLanes cl = chunkLanes( ch.n );
+   const int        N = 1 << L, w = N + 1, NP = N + 1;
+   const int        i  = ch.i0 + min( cl.pt, ch.n - 1 );
+   T                Ax = T( 0 );
+   for ( int k = cl.sub; k < ch.nCells; k += cl.step )
+      Ax += lowPart[i64( ch.entry0 + k ) * NP + i];
+   Ax = chunkSum( Ax, cl );
+   if ( cl.pt >= ch.n )
+      return;
    int qx, qy, qz;
-   entryPos( entries[p.entry0], N, i, 0, qx, qy, qz );
-   const i64 o0 = i64( entries[p.entry0].cell ) * stride + cidx( w, qx, qy, qz );
+   entryPos( entries[ch.entry0], N, i, 0, qx, qy, qz );
+   const i64 o0 = i64( entries[ch.entry0].cell ) * stride + cidx( w, qx, qy, qz );
    T         xc = T( 0 ), i1 = T( 0 ), r0, r1;
    if constexpr ( MODE == MODE_JACOBI || MODE == MODE_CHEB0 )
       xc = x[o0];
@@ -176,9 +176,9 @@ __device__ __forceinline__ void bLowCombine( int bid, const LowerChunk* __restri
    if constexpr ( MODE == MODE_APPLY_ADD )
       i1 = out0[o0];
    epilogue< T, MODE >( Ax, xc, i1, i1, dinv ? dinv[o0] : T( 1 ), a, r0, r1 );
-   for ( int k = 0; k < p.nCells; ++k )
+   for ( int k = cl.sub; k < ch.nCells; k += cl.step )
    {
-      const LowerEntry e = entries[p.entry0 + k];
+      const LowerEntry e = entries[ch.entry0 + k];
       entryPos( e, N, i, 0, qx, qy, qz );
       const i64 o = i64( e.cell ) * stride + cidx( w, qx, qy, qz );
       out0[o]     = r0;

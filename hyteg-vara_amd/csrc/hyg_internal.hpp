@@ -110,7 +110,14 @@ struct ZSeg
    int z0;
    int z1;
 };
-constexpr int kZSegChunk = 24; // planes per z-marching segment (short segments balance the tail of the launch)
+// Planes per z-marching segment: at most kZSegChunk (short segments balance the tail of the launch), fewer on small levels
+// and few cells, where the march itself (one memory latency per plane) is the time of the launch and the chip has room
+// for more wavefronts, at least kZSegLeast (a segment of c planes reads c + 2). Measured with fixed lengths 4 / 6 / 8 / 12 /
+// 24: apply of 6 cells at level 5 8.3 / 8.9 / 9.5 / 10.6 / 14.0 us, cycle from level 7 on 24 cells 3.38 / 3.22 / 3.09 /
+// 3.06 / 3.12 ms; 3 and 2 planes are slower again than 4 (4.7 and 4.8 against 4.5 us with the face points in the launch).
+constexpr int kZSegChunk = 24;
+constexpr int kZSegLeast = 4;
+constexpr int kZSegWaves = 8192;
 // P2 constant operator, z-marching row pairs: a wavefront computes rows y0 (even) and y0+1 of a segment of
 // kP2ZSeg x values (x0 = kP2ZSeg k - 2 + 2 lane, lanes 0 and 63 halo) over planes [z0, z1), z0 even; the
 // table stores (y0, k, z0, z1) in a ZSeg.
@@ -145,14 +152,23 @@ struct LowerEntry
    int l0, l1, l2;
 };
 
-// A run of up to 64 points of one lower-dimensional primitive: face row j (i from i0), edge (i from i0), vertex.
+// A run of points of one lower-dimensional primitive: face row j (i from i0, up to 64 points), edge (i from i0, up to
+// kEdgeChunk points), vertex; with the primitive's incident cells and DoF type, so that a wave reaches its entries
+// without another dependent load.
 struct LowerChunk
 {
    int prim;
    int j;
    int i0;
    int n;
+   int entry0; // LowerPrim::entry0
+   int nCells; // LowerPrim::nCells
+   int bc;     // LowerPrim::bc
+   int pad;
 };
+// Points per edge chunk. A wave gives each point of a chunk 64 / n lanes that share its incident cells (4 to 10 cells
+// per edge on these meshes): with 8 points the cells of an edge point are done in one or two rounds.
+constexpr int kEdgeChunk = 8;
 
 // One face of one macro-cell, for the stencil kernels that compute one-sided face sums. Local face slots
 // in the cell's layout: 0 z = 0, 1 y = 0, 2 x = 0, 3 x+y+z = N.

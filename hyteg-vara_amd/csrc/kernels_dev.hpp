@@ -355,36 +355,44 @@ __device__ __forceinline__ void bRestrictLower( int bid, const LowerChunk* __res
    const int ci = bid * ( kBlock / 64 ) + int( threadIdx.x >> 6 );
    if ( ci >= nChunks )
       return;
-   const int        lane = int( threadIdx.x & 63 );
-   const LowerChunk ch   = chunks[ci];
-   if ( lane >= ch.n )
+   const LowerChunk ch = chunks[ci];
+   if ( !( ch.bc & flag ) )
       return;
-   const LowerPrim p = prims[ch.prim];
-   if ( !( p.bc & flag ) )
-      return;
-   const int Nc = 1 << Lc, wc = Nc + 1, Nf = 2 * Nc, wf = Nf + 1;
-   const int i = ch.i0 + lane, j = ch.j;
-   T         v = T( 0 );
-   for ( int k = 0; k < p.nCells; ++k )
+   const ChunkLanes cl = chunkLanes( ch.n );
+   const int        Nc = 1 << Lc, wc = Nc + 1, Nf = 2 * Nc, wf = Nf + 1;
+   const int        i = ch.i0 + min( cl.pt, ch.n - 1 ), j = ch.j;
+   T                v = T( 0 );
+   for ( int k0 = 0; k0 < ch.nCells; k0 += cl.step )
    {
-      const LowerEntry e = entries[p.entry0 + k];
+      const int        k = min( k0 + cl.sub, ch.nCells - 1 );
+      const LowerEntry e = entries[ch.entry0 + k];
       int              qx, qy, qz;
       entryPos( e, Nc, i, j, qx, qy, qz );
       const T*        fs = fine + i64( e.cell ) * strideF;
       const CellInfo& cf = cinfo[e.cell];
+      const int       q  = cidx( wf, 2 * qx, 2 * qy, 2 * qz );
+      // neighbours outside the cell read the point itself with weight 0: all loads of a lane are independent
+      T f[NDIR], g[NDIR];
 #pragma unroll
       for ( int d = 0; d < NDIR; ++d )
       {
-         const int ax = 2 * qx + dirX( d ), ay = 2 * qy + dirY( d ), az = 2 * qz + dirZ( d );
-         if ( !inCell( Nf, ax, ay, az ) )
-            continue;
-         const T wgt = ( d == 0 ? T( 1 ) : T( 0.5 ) ) * T( cf.invNC[classifySlot( Nf, ax, ay, az )] );
-         v += wgt * fs[cidx( wf, ax, ay, az )];
+         const int  ax = 2 * qx + dirX( d ), ay = 2 * qy + dirY( d ), az = 2 * qz + dirZ( d );
+         const bool in = inCell( Nf, ax, ay, az );
+         f[d]          = fs[in ? cidx( wf, ax, ay, az ) : q];
+         g[d]          = in ? T( cf.invNC[classifySlot( Nf, ax, ay, az )] ) : T( 0 );
       }
+      T s = g[0] * f[0];
+#pragma unroll
+      for ( int d = 1; d < NDIR; ++d )
+         s += T( 0.5 ) * g[d] * f[d];
+      v += k0 + cl.sub < ch.nCells ? s : T( 0 );
    }
-   for ( int k = 0; k < p.nCells; ++k )
+   v = chunkSum( v, cl );
+   if ( cl.pt >= ch.n )
+      return;
+   for ( int k = cl.sub; k < ch.nCells; k += cl.step )
    {
-      const LowerEntry e = entries[p.entry0 + k];
+      const LowerEntry e = entries[ch.entry0 + k];
       int              qx, qy, qz;
       entryPos( e, Nc, i, j, qx, qy, qz );
       coarse[i64( e.cell ) * strideC + cidx( wc, qx, qy, qz )] = v;

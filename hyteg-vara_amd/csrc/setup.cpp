@@ -322,14 +322,20 @@ LevelGeom& MeshCtx::geom( int L )
    // defaults for experiments.
    const char* ec    = std::getenv( "HYG_ZCHUNK" );
    const char* eo    = std::getenv( "HYG_SEG_ORDER" );
-   const int   chunk = ec ? std::max( 4, std::min( 1024, std::atoi( ec ) ) ) : kZSegChunk;
    const bool  xFast = eo && std::atoi( eo ) == 1;
    for ( int k = 0; k < kNumCellCfgs; ++k )
    {
       const int R = kCellRows[k], WO = 64 * kCellPoints[k] - 2;
       auto&     v = g.zSegsHost[k];
       v.clear();
-      auto add = [&]( int y, int x0, int z0 ) {
+      // planes per segment: as many as leave kZSegWaves wavefronts on the mesh, at most kZSegChunk
+      i64 steps = 0;
+      for ( int y = 1; y <= N - 2; y += R )
+         for ( int x0 = 1; x0 <= N - 2; x0 += WO )
+            steps += std::max( 0, N - y - x0 );
+      const int most  = int( std::max< i64 >( kZSegLeast, std::min< i64 >( kZSegChunk, steps * mesh->nC() / kZSegWaves ) ) );
+      const int chunk = ec ? std::max( 2, std::min( 1024, std::atoi( ec ) ) ) : most;
+      auto      add = [&]( int y, int x0, int z0 ) {
          const int zEnd = N - y - x0 + 1;
          if ( z0 < zEnd )
             v.push_back( { y, x0, z0, std::min( z0 + chunk, zEnd ) } );
@@ -382,19 +388,20 @@ LevelGeom& MeshCtx::geom( int L )
    g.chunksHost.clear();
    for ( int p = 0; p < (int) primsHost.size(); ++p )
    {
-      const int kind = primsHost[p].kind;
-      if ( kind == 0 )
-         g.chunksHost.push_back( { p, 0, 0, 1 } );
-      else if ( kind == 1 )
+      const LowerPrim& pr  = primsHost[p];
+      auto             add = [&]( int j, int i0, int n ) { g.chunksHost.push_back( { p, j, i0, n, pr.entry0, pr.nCells, pr.bc, 0 } ); };
+      if ( pr.kind == 0 )
+         add( 0, 0, 1 );
+      else if ( pr.kind == 1 )
       {
-         for ( int i0 = 1; i0 <= N - 1; i0 += 64 )
-            g.chunksHost.push_back( { p, 0, i0, std::min( 64, N - i0 ) } );
+         for ( int i0 = 1; i0 <= N - 1; i0 += kEdgeChunk )
+            add( 0, i0, std::min( kEdgeChunk, N - i0 ) );
       }
       else
       {
          for ( int j = 1; j <= N - 2; ++j )
             for ( int i0 = 1; i0 <= N - 1 - j; i0 += 64 )
-               g.chunksHost.push_back( { p, j, i0, std::min( 64, N - j - i0 ) } );
+               add( j, i0, std::min( 64, N - j - i0 ) );
       }
    }
    g.nChunks        = (int) g.chunksHost.size();

@@ -20,8 +20,8 @@
 // faces are whole planes/rows and are computed by faceFlat with coalesced loads. kFaceCombine adds
 // the partial sums of the two sides, applies the epilogue and writes every replica.
 //
-// Macro-edges and -vertices (lower): one lane per point gathers the one-sided stencils of all
-// incident cells.
+// Macro-edges and -vertices, and the face points of levels up to kDirectFaceLevel (lower): the lanes of a
+// point share its incident cells and gather their one-sided stencils.
 
 #include "sweep.hpp"
 
@@ -46,9 +46,6 @@ template < typename T, int MODE >
 static void stencilT( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol, int L, const StencilCall& c, hipStream_t s )
 {
    constexpr bool dbl  = std::is_same< T, double >::value;
-   const int      nC   = m.mesh->nC();
-   const T*       cst  = dbl ? (const T*) ol.cellSt : (const T*) ol.cellStF;
-   const T*       ew   = dbl ? (const T*) ol.entryW : (const T*) ol.entryWF;
    const T*       pi   = dbl ? (const T*) ol.primInv : (const T*) ol.primInvF;
    T*             part = dbl ? (T*) ol.facePart : (T*) ol.facePartF;
    const int      cfg  = cellConfig( g, dbl ? 8 : 4, MODE );
@@ -58,32 +55,9 @@ static void stencilT( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol,
    T*             out1 = (T*) c.out1;
    // 1. cell interiors with the one-sided sums of the x = 0 and diagonal faces, the one-sided sums
    // of the z = 0 and y = 0 faces, and macro-edges and -vertices: one launch
-   const int nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
-   SweepArgs< T > p;
-   p.segs    = g.zSegs[cfg];
-   p.nSegs   = g.nZSegs[cfg];
-   p.nC      = nC;
-   p.L       = L;
-   p.flag    = c.flag;
-   p.stride  = g.stride;
-   p.cellSt  = cst;
-   p.cfs     = m.cellFaces;
-   p.entryW  = ew;
-   p.primInv = pi;
-   p.part    = part;
-   p.x       = x;
-   p.in1     = in1;
-   p.out0    = out0;
-   p.out1    = out1;
-   p.a       = T( c.a );
-   p.items   = g.flatItems;
-   p.nItems  = nFace > 0 ? g.nFlatItems : 0;
-   p.chunks  = g.chunks;
-   p.nChunks = nLow;
-   p.prims   = m.prims;
-   p.entries = m.entries;
-   p.gC      = p.nSegs > 0 ? xcdGrid( ( ( p.nSegs + 3 ) / 4 ) * nC ) : 0;
-   p.gF      = p.nItems > 0 ? xcdGrid( ceilDiv( p.nItems, 4 ) ) : 0;
+   const int nFace = directFaces( g ) ? 0 : g.nChunks - g.firstFaceChunk;
+   SweepArgs< T > p = sweepArgs< T >( m, g, ol, L, c, cfg );
+   const int      nLow = p.nChunks;
    const int gL = nLow > 0 ? xcdGrid( ceilDiv( nLow, kBlock / 64 ) ) : 0;
    if ( p.gC + p.gF + gL > 0 )
    {

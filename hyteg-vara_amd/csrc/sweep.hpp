@@ -93,7 +93,7 @@ __device__ __forceinline__ void cellZ( int bid, const ZSeg* __restrict__ segs, i
                                                     const T* __restrict__ entryW, T* __restrict__ part, int flag,
                                                     const T* __restrict__ x, const T* __restrict__ in1, T* __restrict__ out0,
                                                     T* __restrict__ out1, T a, const CellInfo* __restrict__ cinfo, int sorK,
-                                                    int sorM )
+                                                    int sorM, int faces )
 {
    constexpr bool kIn1 = MODE == MODE_RESIDUAL || MODE == MODE_JACOBI || MODE == MODE_CHEB0 || MODE == MODE_CHEBK || MODE == MODE_SOR;
    constexpr bool kE   = kIn1 || MODE == MODE_APPLY_ADD;
@@ -141,7 +141,7 @@ __device__ __forceinline__ void cellZ( int bid, const ZSeg* __restrict__ segs, i
    // face's one-sided weights. Its E-group terms are formed on lane 1 (P = 1, then shifted) or on
    // lane 0 itself (P = 2), which therefore holds that face's E-group weights.
    const CellFaceSlot fx   = cfs[4 * c + 2];
-   const bool         onX0 = x0 == 1 && ( fx.bc & flag ) != 0;
+   const bool         onX0 = faces && x0 == 1 && ( fx.bc & flag ) != 0;
    T                  wu[7], we[4];
    {
       const T* wf = entryW + 16 * i64( onX0 ? fx.entry : 0 );
@@ -155,7 +155,7 @@ __device__ __forceinline__ void cellZ( int bid, const ZSeg* __restrict__ segs, i
    // diagonal face (slot 3): the row ends x = N-y-z of rows y0..y0+R-1 inside the output window
    const CellFaceSlot fd     = cfs[4 * c + 3];
    const int          xeHi   = N - y0 - z0, xeLo = N - ( y0 + R - 1 ) - ( z1 - 1 );
-   const bool         onDiag = ( fd.bc & flag ) != 0 && xeHi >= x0 && xeLo <= x0 + WO - 1;
+   const bool         onDiag = faces && ( fd.bc & flag ) != 0 && xeHi >= x0 && xeLo <= x0 + WO - 1;
    T                  wd[15], wdu[7], wde[4];
    {
       const T* wf = entryW + 16 * i64( onDiag ? fd.entry : 0 );
@@ -396,26 +396,26 @@ __device__ __forceinline__ void lower( int bid, const LowerChunk* __restrict__ c
    const int ci = remapXcd( bid, nb ) * ( kBlock / 64 ) + __builtin_amdgcn_readfirstlane( int( threadIdx.x >> 6 ) );
    if ( ci >= nChunks )
       return;
-   const int        lane = int( threadIdx.x & 63 );
-   const LowerChunk ch   = chunks[ci];
-   const LowerPrim  p    = prims[ch.prim];
-   if ( !( p.bc & flag ) )
+   const LowerChunk ch = chunks[ci];
+   if ( !( ch.bc & flag ) )
       return;
-   bool      on = lane < ch.n;
-   const int N = 1 << L, w = N + 1;
-   const int i = ch.i0 + ( on ? lane : 0 ), j = ch.j;
+   const ChunkLanes cl = chunkLanes( ch.n );
+   bool             on = cl.pt < ch.n;
+   const int        N = 1 << L, w = N + 1;
+   const int        i = ch.i0 + ( on ? cl.pt : 0 ), j = ch.j;
    if constexpr ( MODE == MODE_SOR )
-      on = on && sorColour( cinfo, entries[p.entry0], N, i, j, sorM ) == sorK;
-   T          Ax = T( 0 );
-   for ( int k = 0; k < p.nCells; ++k )
+      on = on && sorColour( cinfo, entries[ch.entry0], N, i, j, sorM ) == sorK;
+   T Ax = T( 0 );
+   for ( int k0 = 0; k0 < ch.nCells; k0 += cl.step )
    {
-      const LowerEntry e = entries[p.entry0 + k];
+      const int        k = min( k0 + cl.sub, ch.nCells - 1 );
+      const LowerEntry e = entries[ch.entry0 + k];
       int              qx, qy, qz;
       entryPos( e, N, i, j, qx, qy, qz );
       const T*  xs = x + i64( e.cell ) * stride;
-      const T*  wv = entryW + i64( p.entry0 + k ) * 16;
+      const T*  wv = entryW + i64( ch.entry0 + k ) * 16;
       const int q  = cidx( w, qx, qy, qz );
-      T         v[NDIR];
+      T         v[NDIR], s = T( 0 );
 #pragma unroll
       for ( int d = 0; d < NDIR; ++d )
       {
@@ -424,12 +424,14 @@ __device__ __forceinline__ void lower( int bid, const LowerChunk* __restrict__ c
       }
 #pragma unroll
       for ( int d = 0; d < NDIR; ++d )
-         Ax += wv[d] * v[d];
+         s += wv[d] * v[d];
+      Ax += k0 + cl.sub < ch.nCells ? s : T( 0 );
    }
+   Ax = chunkSum( Ax, cl );
    if ( !on )
       return;
    // pointwise terms from the first replica (all replicas hold the same value)
-   const LowerEntry e0 = entries[p.entry0];
+   const LowerEntry e0 = entries[ch.entry0];
    int              qx, qy, qz;
    entryPos( e0, N, i, j, qx, qy, qz );
    const i64 o0i = i64( e0.cell ) * stride + cidx( w, qx, qy, qz );
@@ -441,9 +443,9 @@ __device__ __forceinline__ void lower( int bid, const LowerChunk* __restrict__ c
    if constexpr ( MODE == MODE_APPLY_ADD )
       ov = out0[o0i];
    epilogue< T, MODE >( Ax, xc, i1, ov, primInv[ch.prim], a, r0, r1 );
-   for ( int k = 0; k < p.nCells; ++k )
+   for ( int k = cl.sub; k < ch.nCells; k += cl.step )
    {
-      const LowerEntry e = entries[p.entry0 + k];
+      const LowerEntry e = entries[ch.entry0 + k];
       entryPos( e, N, i, j, qx, qy, qz );
       const i64 o = i64( e.cell ) * stride + cidx( w, qx, qy, qz );
       out0[o]     = r0;
@@ -482,14 +484,60 @@ struct SweepArgs
    int                 gC, gF;
    const CellInfo*     cinfo = nullptr; // multi-colour SOR: cell colours, the colour of this pass and their number
    int                 sorK = 0, sorM = 1;
+   // 1: the cells leave one-sided sums of their face points in `part` (kFaceCombine adds them); 0: the face points are
+   // done in this launch like the edge points (chunks hold them, gF = 0)
+   int                 faces = 1;
 };
+
+// Up to level 6 the face points are gathered from both cells in the sweep launch itself, like the edge points: two stencils
+// of scattered loads per point against a second launch (kFaceCombine, 4 us where it has next to nothing to do). One sweep
+// of 6 cells at level 5: 8.4 us with the second launch, 4.5 us without. A Chebyshev V-cycle from level 7 on 24 cells:
+// 2.89 ms with the line at level 4, 2.80 at 5, 2.73 at 6, 2.84 at 7; an apply at level 8 takes 0.40 ms with one-sided
+// sums and 0.50 ms with gathers, whose lines on the x = 0 and diagonal faces are fetched for one value each.
+constexpr int kDirectFaceLevel = 6;
+inline bool   directFaces( const LevelGeom& g ) { return g.L <= kDirectFaceLevel; }
+
+// arguments of the sweep of one level of the constant operator
+template < typename T >
+SweepArgs< T > sweepArgs( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::Level& ol, int L, const StencilCall& c, int cfg )
+{
+   constexpr bool dbl    = std::is_same< T, double >::value;
+   const bool     direct = directFaces( g );
+   SweepArgs< T > p;
+   p.segs    = g.zSegs[cfg];
+   p.nSegs   = g.nZSegs[cfg];
+   p.nC      = m.mesh->nC();
+   p.L       = L;
+   p.flag    = c.flag;
+   p.stride  = g.stride;
+   p.cellSt  = dbl ? (const T*) ol.cellSt : (const T*) ol.cellStF;
+   p.cfs     = m.cellFaces;
+   p.entryW  = dbl ? (const T*) ol.entryW : (const T*) ol.entryWF;
+   p.primInv = dbl ? (const T*) ol.primInv : (const T*) ol.primInvF;
+   p.part    = dbl ? (T*) ol.facePart : (T*) ol.facePartF;
+   p.x       = (const T*) c.x;
+   p.in1     = (const T*) c.in1;
+   p.out0    = (T*) c.out0;
+   p.out1    = (T*) c.out1;
+   p.a       = T( c.a );
+   p.items   = g.flatItems;
+   p.nItems  = direct ? 0 : g.nFlatItems;
+   p.chunks  = g.chunks;
+   p.nChunks = direct ? g.nChunks : g.firstFaceChunk;
+   p.prims   = m.prims;
+   p.entries = m.entries;
+   p.gC      = p.nSegs > 0 ? xcdGrid( ( ( p.nSegs + 3 ) / 4 ) * p.nC ) : 0;
+   p.gF      = p.nItems > 0 ? xcdGrid( ceilDiv( p.nItems, 4 ) ) : 0;
+   p.faces   = direct ? 0 : 1;
+   return p;
+}
 
 template < typename T, int MODE, int R, int P, int D >
 __device__ __forceinline__ void bSweep( int b, const SweepArgs< T >& p )
 {
    if ( b < p.gC )
       cellZ< T, MODE, R, P, D >( b, p.segs, p.nSegs, p.nC, p.L, p.stride, p.cellSt, p.cfs, p.entryW, p.part, p.flag, p.x, p.in1,
-                              p.out0, p.out1, p.a, p.cinfo, p.sorK, p.sorM );
+                              p.out0, p.out1, p.a, p.cinfo, p.sorK, p.sorM, p.faces );
    else if ( b < p.gC + p.gF )
       faceFlat< T >( b - p.gC, p.items, p.nItems, p.L, p.stride, p.cfs, p.entryW, p.part, p.flag, p.x );
    else

@@ -20,28 +20,6 @@ namespace hyg {
 constexpr int kBatchGrid = 2048; // blocks of a persistent batched launch (8 per CU)
 
 // --------------------------------------------------------------------------------------------- task tables
-template < typename T >
-struct ElemArgs
-{
-   int                 L, tilesPerCell;
-   i64                 stride;
-   const ElemCell*     cells;
-   const T*            kb;
-   const CellInfo*     cinfo;
-   const CellFaceSlot* cfs;
-   const LowerPrim*    prims;
-   const LowerEntry*   entries;
-   T*                  part;
-   T*                  lowPart;
-   const T*            dinv;
-   int                 flag;
-   const T*            x;
-   const T*            in1;
-   T*                  out0;
-   T*                  out1;
-   T                   a;
-};
-
 // constant-coefficient sweep (cell interiors, flat faces, edges and vertices) of one problem
 template < typename T >
 struct SweepTask
@@ -166,9 +144,7 @@ __global__ __launch_bounds__( kBlock ) void kBatchElem( const ElemTask< T >* __r
    if ( vb >= total )
       return;
    const ElemTask< T >& t = tasks[findTask( tasks, nTasks, vb )];
-   const ElemArgs< T >& e = t.el;
-   bElemApply< T, MODE, false >( vb - t.first, e.L, e.tilesPerCell, e.stride, e.cells, e.kb, e.cinfo, e.cfs, e.prims, e.entries, e.part,
-                                 e.lowPart, e.dinv, e.flag, e.x, e.in1, e.out0, e.out1, e.a );
+   elemSweep< T, MODE, kElemRows >( vb - t.first, (ElemArgsAt< T >) &t.el );
 }
 
 template < typename T, int MODE >
@@ -283,7 +259,6 @@ void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item 
       const hyg_op_s&         op = *it.op;
       const hyg_op_s::Level&  ol = op.levels[it.L];
       const StencilCall&      c  = it.c;
-      const int               nC = m.mesh->nC(), N = 1 << it.L, w = N + 1;
       const int               nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
       SweepTask< T >          t{};
       ElemTask< T >           u{};
@@ -315,27 +290,10 @@ void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item 
       }
       else
       {
-         ElemArgs< T >& e = u.el;
-         u.kind           = 1;
-         e.L              = it.L;
-         e.tilesPerCell   = ceilDiv( S3i( w ), kBlock );
-         e.stride         = g.stride;
-         e.cells          = ol.elem;
-         e.kb             = dbl ? (const T*) ol.kb : (const T*) ol.kbF;
-         e.cinfo          = m.cellInfo;
-         e.cfs            = m.cellFaces;
-         e.prims          = m.prims;
-         e.entries        = m.entries;
-         e.part           = dbl ? (T*) ol.facePart : (T*) ol.facePartF;
-         e.lowPart        = dbl ? (T*) ol.lowPart : (T*) ol.lowPartF;
-         e.dinv           = dbl ? (const T*) ol.dinv : (const T*) ol.dinvF;
-         e.flag           = c.flag;
-         e.x              = (const T*) c.x;
-         e.in1            = (const T*) c.in1;
-         e.out0           = (T*) c.out0;
-         e.out1           = (T*) c.out1;
-         e.a              = T( c.a );
-         appendTask( el, u, nC * e.tilesPerCell );
+         const ElemArgs< T >& e = u.el;
+         u.kind                 = 1;
+         u.el                   = elemArgs< T >( m, g, ol, it.L, c );
+         appendTask( el, u, elemBlocks( e ) );
          f.kind    = 0;
          f.part    = e.part;
          f.primInv = nullptr;

@@ -12,9 +12,9 @@
 //      k are formed once and the 30 quadrature points of the six cell types are reached by angle
 //      addition with per-cell tables of cos/sin of the quadrature offsets (kKBarTables, once per level at
 //      operator creation; read with scalar loads);
-//   2. assembles at every point of every macro-cell the 15 weights of its stencil from the (up to) 24
-//      incident elements of that cell and applies them (kElemApply); interior points get the epilogue,
-//      points on faces, edges and vertices store the cell's one-sided sum;
+//   2. marches over the cubes of the anchor lattice plane by plane and adds the contributions of their six elements to
+//      the corners (kElemSweep); interior points get the epilogue, points on faces, edges and vertices store the cell's
+//      one-sided sum;
 //   3. adds the one-sided sums of face, edge and vertex points over their cells and writes every
 //      replica (kFaceCombine, kLowCombine).
 // The inverse diagonal (per point, since it depends on k) is built the same way at operator setup.
@@ -135,10 +135,15 @@ static void elemT( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, co
       hipLaunchKernelGGL( ( kElemApply< T, MODE, DIAG, false, true > ), dim3( xcdGrid( nC * tA ) ), dim3( kBlock ), 0, s, L, tA, g.stride,
                           ol.elem, kb, m.cellInfo, m.cellFaces, m.prims, m.entries, part, low, dv, c.flag, x, in1, out0, out1, T( c.a ),
                           nullptr, 0, dbl ? (const T*) ol.bw : (const T*) ol.bwF, nC * tA );
-   else
+   else if constexpr ( DIAG )
       hipLaunchKernelGGL( ( kElemApply< T, MODE, DIAG > ), dim3( xcdGrid( nC * tA ) ), dim3( kBlock ), 0, s, L, tA, g.stride, ol.elem, kb,
                           m.cellInfo, m.cellFaces, m.prims, m.entries, part, low, dv, c.flag, x, in1, out0, out1, T( c.a ), nullptr, 0,
                           nullptr, nC * tA );
+   else
+   {
+      const ElemArgs< T > e = elemArgs< T >( m, g, ol, L, c );
+      hipLaunchKernelGGL( ( kElemSweep< T, MODE, kElemRows > ), dim3( elemBlocks( e ) ), dim3( kBlock ), 0, s, e );
+   }
    // 3. face, edge and vertex values
    const int nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
    if ( nFace > 0 )

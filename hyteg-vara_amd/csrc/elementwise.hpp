@@ -22,6 +22,11 @@ __device__ __forceinline__ void sincosT( float a, float& s, float& c ) { sincosf
 __device__ __forceinline__ double expT( double a ) { return exp( a ); }
 __device__ __forceinline__ float  expT( float a ) { return expf( a ); }
 
+// Layout of the coefficient integrals of a cell: the rows of the anchor lattice (N points per edge) one after the other, each
+// with the six types in turn, so that a row of a wave is one run of memory. Position of type 0, x = 0 of row (y, z); the
+// types follow each other N - y - z values apart.
+__device__ __forceinline__ int kbRow( int N, int y, int z ) { return 6 * ( S3i( N ) - S3i( N - z ) + rowStart( N - z, y ) ); }
+
 // ------------------------------------------------------------------ 1. coefficient integrals
 // One thread per anchor (x, y, z), x+y+z <= N-1, of one macro-cell; kb[c][t][anchor] for the six types. The tables
 // of the block's cell are wave-uniform: they are read with scalar loads and feed the multiply-adds directly.
@@ -58,7 +63,8 @@ __global__ __launch_bounds__( kBlock ) void kKBar( int L, int tilesPerCell, cons
       for ( int k = 0; k < 30; ++k )
          g[k] += ac * tb[2 * k] - as * tb[2 * k + 1];
    }
-   T* out = kb + i64( c ) * 6 * S;
+   T*        out = kb + i64( c ) * 6 * S + kbRow( N, y, z ) + x;
+   const int nx  = N - y - z;
 #pragma unroll
    for ( int t = 0; t < 6; ++t )
    {
@@ -66,8 +72,7 @@ __global__ __launch_bounds__( kBlock ) void kKBar( int L, int tilesPerCell, cons
 #pragma unroll
       for ( int q = 0; q < 5; ++q )
          v += T( kQW6[q] ) * expT( g[5 * t + q] );
-      if ( x + y + z + kMCMax[t] <= N )
-         out[t * S + s] = T( k0 ) * v;
+      out[t * nx] = x + y + z + kMCMax[t] <= N ? T( k0 ) * v : T( 0 ); // 0: the element is not in the cell
    }
 }
 
@@ -88,11 +93,15 @@ __global__ __launch_bounds__( kBlock ) void kKBarPoly( int L, int tilesPerCell, 
    int x, y, z;
    tetXYZ( N, s, x, y, z );
    const ElemCell& ec  = cells[c];
-   T*              out = kb + i64( c ) * 6 * S;
+   T*              out = kb + i64( c ) * 6 * S + kbRow( N, y, z ) + x;
+   const int       nx  = N - y - z;
    for ( int t = 0; t < 6; ++t )
    {
-      if ( x + y + z + kMCMax[t] > N )
+      if ( x + y + z + kMCMax[t] > N ) // the element is not in the cell
+      {
+         out[t * nx] = T( 0 );
          continue;
+      }
       double v = 0.0;
       for ( int q = 0; q < 5; ++q )
       {
@@ -123,7 +132,7 @@ __global__ __launch_bounds__( kBlock ) void kKBarPoly( int L, int tilesPerCell, 
                }
          v += kQW6[q] * kq;
       }
-      out[t * S + s] = T( v );
+      out[t * nx] = T( v );
    }
 }
 
@@ -133,16 +142,16 @@ __global__ __launch_bounds__( kBlock ) void kKBarPoly( int L, int tilesPerCell, 
 template < typename T, bool DIAG >
 __device__ __forceinline__ void elemWeights( const ElemCell& ec, const T* __restrict__ kc, int N, int px, int py, int pz, T W[NDIR] )
 {
-   const int SN = S3i( N );
    // anchors p - o for the eight offsets o in {0,1}^3 (encoded x + 2y + 4z)
-   int  aIdx[8];
+   int  aIdx[8], aLen[8];
    bool aOk[8];
 #pragma unroll
    for ( int o = 0; o < 8; ++o )
    {
       const int ax = px - ( o & 1 ), ay = py - ( ( o >> 1 ) & 1 ), az = pz - ( ( o >> 2 ) & 1 );
       aOk[o]       = ax >= 0 && ay >= 0 && az >= 0;
-      aIdx[o]      = aOk[o] ? cidx( N, ax, ay, az ) : 0;
+      aLen[o]      = aOk[o] ? N - ay - az : 0;
+      aIdx[o]      = aOk[o] ? kbRow( N, ay, az ) + ax : 0;
    }
 #pragma unroll
    for ( int d = 0; d < NDIR; ++d )
@@ -155,7 +164,7 @@ __device__ __forceinline__ void elemWeights( const ElemCell& ec, const T* __rest
          const int o   = kMCOff[t][k];
          const int as  = px + py + pz - ( ( o & 1 ) + ( ( o >> 1 ) & 1 ) + ( ( o >> 2 ) & 1 ) );
          const bool ok = aOk[o] && as + kMCMax[t] <= N;
-         const T    kv = ok ? kc[t * SN + aIdx[o]] : T( 0 );
+         const T    kv = ok ? kc[t * aLen[o] + aIdx[o]] : T( 0 );
          if constexpr ( DIAG )
             W[0] += kv * T( ec.mt[t][5 * k] );
          else
@@ -165,9 +174,441 @@ __device__ __forceinline__ void elemWeights( const ElemCell& ec, const T* __rest
       }
 }
 
-// One thread per point of the closed macro-cell. DIAG: the diagonal entry instead of the product. BND: the points
-// on the cell's faces, edges and vertices only, listed in bnd[0 .. nBnd) by their index in the cell array (the
-// surrogate operator does the interior points itself). STW: the point's stencil weights are read from wst
+// ------------------------------------------------------------------ 3. the operator, z-marching wavefronts
+__device__ __forceinline__ double elemK( const ElemCell& ec, int t, int i, double* ) { return ec.mt[t][i]; }
+__device__ __forceinline__ float  elemK( const ElemCell& ec, int t, int i, float* ) { return ec.mtF[t][i]; }
+
+// A "down" micro-cell is the point reflection of the "up" cell of its colour (p -> (1,1,1) - p up to a lattice step), so its
+// element matrix holds the same entries: the vertex of type 0, 1 or 2 that vertex v of type 3, 4 or 5 is mapped to.
+constexpr int kMCMirror[3][4] = { { 3, 0, 1, 2 }, { 2, 0, 1, 3 }, { 2, 3, 1, 0 } };
+constexpr bool mirrorFits()
+{
+   for ( int t = 0; t < 3; ++t )
+      for ( int a = 0; a < 4; ++a )
+         for ( int b = 0; b < 4; ++b )
+            for ( int k = 0; k < 3; ++k )
+               if ( kMC[3 + t][a][k] - kMC[3 + t][b][k] != kMC[t][kMCMirror[t][b]][k] - kMC[t][kMCMirror[t][a]][k] )
+                  return false;
+   return true;
+}
+static_assert( mirrorFits(), "down micro-cells are point reflections of up micro-cells" );
+constexpr int kMCEdge[4][4] = { { -1, 0, 1, 2 }, { 0, -1, 3, 4 }, { 1, 3, -1, 5 }, { 2, 4, 5, -1 } }; // vertex pair -> edge
+
+// Contributions of the six micro-cells of the cube anchored at one lattice point to its eight corners (x + 2y + 4z):
+// y_i += sum_t kb_t K_t[i,j] (u_j - u_i) over the element edges (the rows of K_t sum to zero). Elements that share an edge
+// of the cube share its difference: 19 edges, 36 products with kb, against 96 for the element matrices. K: the edge entries
+// of the three up types. Only the corners in WANT are formed.
+template < typename T, int WANT >
+__device__ __forceinline__ void cubeContributions( const T ( &K )[3][6], const T ( &k )[6], const T ( &u )[8], T ( &acc )[8] )
+{
+   constexpr int EA[6] = { 0, 0, 0, 1, 1, 2 }, EB[6] = { 1, 2, 3, 2, 3, 3 }; // vertex pairs of an element
+#pragma unroll
+   for ( int i = 0; i < 8; ++i )
+#pragma unroll
+      for ( int j = i + 1; j < 8; ++j )
+      {
+         if ( !( ( WANT >> i ) & 1 ) && !( ( WANT >> j ) & 1 ) )
+            continue;
+         T    c    = T( 0 );
+         bool edge = false;
+#pragma unroll
+         for ( int t = 0; t < 6; ++t )
+#pragma unroll
+            for ( int e = 0; e < 6; ++e )
+            {
+               const int a = kMCOff[t][EA[e]], b = kMCOff[t][EB[e]];
+               if ( ( a == i && b == j ) || ( a == j && b == i ) )
+               {
+                  const T w = K[t % 3][t < 3 ? e : kMCEdge[kMCMirror[t % 3][EA[e]]][kMCMirror[t % 3][EB[e]]]];
+                  c         = edge ? fma( k[t], w, c ) : k[t] * w;
+                  edge      = true;
+               }
+            }
+         if ( !edge )
+            continue;
+         const T d = u[j] - u[i];
+         if ( ( WANT >> i ) & 1 )
+            acc[i] = fma( c, d, acc[i] );
+         if ( ( WANT >> j ) & 1 )
+            acc[j] = fma( -c, d, acc[j] );
+      }
+}
+
+// one-sided sum of a point on a cell's face (slot 1..4), edge or vertex, for kFaceCombine / kLowCombine
+template < typename T >
+__device__ __forceinline__ void elemStoreBoundary( int c, int N, int slot, int px, int py, int pz, T val, int flag,
+                                                   const CellInfo* __restrict__ cinfo, const CellFaceSlot* __restrict__ cfs,
+                                                   const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
+                                                   T* __restrict__ part, T* __restrict__ lowPart )
+{
+   const int NP = N + 1;
+   if ( slot <= 4 )
+   {
+      const CellFaceSlot fs = cfs[4 * c + slot - 1];
+      if ( fs.bc & flag )
+         part[i64( fs.block ) * NP * NP + facePartIndex( slot - 1, N, px, py, pz )] = val;
+      return;
+   }
+   const CellInfo& ci = cinfo[c];
+   if ( !( prims[ci.prim[slot]].bc & flag ) )
+      return;
+   const int e = ci.entry[slot];
+   int       i = 0;
+   if ( slot <= 10 )
+   {
+      const int b[4] = { N - px - py - pz, px, py, pz };
+      i              = b[entries[e].l1];
+   }
+   lowPart[i64( e ) * NP + i] = val;
+}
+
+template < typename T >
+struct ElemArgs
+{
+   const ZSeg*         segs;
+   int                 nSegs, nC, L;
+   i64                 stride;
+   const ElemCell*     cells;
+   const T*            kb;
+   const CellInfo*     cinfo;
+   const CellFaceSlot* cfs;
+   const LowerPrim*    prims;
+   const LowerEntry*   entries;
+   T*                  part;
+   T*                  lowPart;
+   const T*            dinv;
+   int                 flag;
+   const T*            x;
+   const T*            in1;
+   T*                  out0;
+   T*                  out1;
+   T                   a;
+};
+
+// the arguments of a sweep in constant memory (the kernel's argument segment, or a batch's task table)
+template < typename T >
+using ElemArgsAt = const __attribute__( ( address_space( 4 ) ) ) ElemArgs< T >*;
+
+// What a wave loads for one cube layer z: kb of the six types of anchor rows y0-1 .. y0+R-1, and point rows y0-1 .. y0+R
+// of plane z+1.
+template < typename T, int R >
+struct ElemLayer
+{
+   T k[R + 1][6];
+   T u[R + 2];
+};
+
+// All points of the closed cells. A wave owns R rows (y0 ..) and 62 points (x0 .., lanes 1..62) and marches z: layer z (the
+// cubes between planes z and z+1) gives its contributions to plane z, which completes it, and to plane z+1, which are
+// carried; corners at x+1 are moved by one lane shift per row. It reads the six kb of an anchor and each value about once
+// (64 B per point in FP64) where a thread per point gathered 39 values: level 7 on 24 cells (8.4 million points) 314 -> 242
+// us in FP64, FP32 Jacobi sweep 244 -> 140 us. Bound by the vector instructions of a step (180 FP32, of which 105 are the
+// edge products) at 55% of the lanes: rows of a tetrahedron end inside the 62-point windows.
+// Lanes outside a row, rows outside a plane and anchors outside the cell load 0 (the descriptor's range check), so they
+// add nothing; elements that stick out of the cell have kb = 0.
+// The arguments are read where they are used (ap, made opaque for the rare boundary rows): held in scalar registers through
+// the march they spilled, 66 of 250 vector instructions per plane.
+template < typename T, int MODE, int R >
+__device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
+{
+   const auto&    p    = *ap;
+   constexpr bool kIn1 = MODE == MODE_RESIDUAL || MODE == MODE_JACOBI || MODE == MODE_CHEB0 || MODE == MODE_CHEBK;
+   constexpr bool kE   = kIn1 || MODE == MODE_APPLY_ADD;
+   constexpr bool kD   = MODE == MODE_JACOBI || MODE == MODE_CHEB0 || MODE == MODE_CHEBK;
+   constexpr bool kTwo = MODE == MODE_CHEB0 || MODE == MODE_CHEBK;
+   constexpr int  B    = int( sizeof( T ) );
+   const int      nbx  = ( p.nSegs + 3 ) / 4, nb = nbx * p.nC; // blocks per cell
+   const int      lb   = remapXcd( bid, nb );
+   if ( lb >= nb )
+      return;
+   const int c  = lb / nbx;
+   const int si = ( lb - c * nbx ) * 4 + __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 6 );
+   if ( si >= p.nSegs )
+      return;
+   const ZSeg     sg = p.segs[si];
+   const int      N = 1 << p.L, w = N + 1, NP = N + 1, y0 = sg.y, x0 = sg.x0, z0 = sg.z0, z1 = sg.z1;
+   const int      lane = int( threadIdx.x & 63u );
+   const int      px   = x0 - 1 + lane;
+   const int      SN = S3i( N ), SW = S3i( w );
+   const i64      cb    = i64( c ) * p.stride;
+   const unsigned bytes = unsigned( ( p.stride + kTailSlack ) * B );
+   const auto     rx = makeRsrc( p.x + cb, bytes ), r0 = makeRsrc( p.out0 + cb, bytes );
+   const auto     re = makeRsrc( kIn1 ? p.in1 + cb : p.out0 + cb, bytes ), r1 = makeRsrc( kTwo ? p.out1 + cb : p.out0 + cb, bytes );
+   const auto     rd = makeRsrc( kD ? p.dinv + cb : p.x + cb, bytes );
+   const T*       kc = p.kb + i64( c ) * 6 * SN;
+   // the x = 0 and diagonal faces (slots 2 and 3)
+   const CellFaceSlot f2 = p.cfs[4 * c + 2], f3 = p.cfs[4 * c + 3];
+   const auto         rp2 = makeRsrc( p.part + i64( f2.block ) * NP * NP, unsigned( NP * NP * B ) );
+   const auto         rp3 = makeRsrc( p.part + i64( f3.block ) * NP * NP, unsigned( NP * NP * B ) );
+   const ElemCell&    ec  = p.cells[c];
+   T                  K[3][6];
+   constexpr int      EA[6] = { 0, 0, 0, 1, 1, 2 }, EB[6] = { 1, 2, 3, 2, 3, 3 };
+#pragma unroll
+   for ( int t = 0; t < 3; ++t )
+#pragma unroll
+      for ( int e = 0; e < 6; ++e )
+         K[t][e] = elemK( ec, t, 4 * EA[e] + EB[e], static_cast< T* >( nullptr ) );
+
+   // point row y of plane z: byte offset of x = 0, and the number of its points (0 outside the cell)
+   auto rowU = [&]( int y, int z, int& n ) {
+      n = y >= 0 && z >= 0 ? max( 0, N - y - z + 1 ) : 0;
+      return n > 0 ? ( SW - S3i( w - z ) + rowStart( w - z, y ) ) * B : 0;
+   };
+   auto loadU = [&]( int y, int z ) {
+      int       n;
+      const int o = rowU( y, z, n );
+      return bufLoad< T >( rx, unsigned( px ) < unsigned( n ) ? unsigned( px * B ) : kDropOffset, o );
+   };
+   // layer z: kb of the anchor rows and the point rows of plane z+1
+   auto loadLayer = [&]( ElemLayer< T, R >& Q, int z ) {
+      const int  W  = N - z; // anchors of row 0
+      const auto rk = makeRsrc( kc + 6 * ( SN - S3i( W ) ), W > 0 ? unsigned( 6 * T2i( W ) * B ) : 0u );
+#pragma unroll
+      for ( int r = 0; r <= R; ++r )
+      {
+         const int      y = y0 - 1 + r, n = y >= 0 ? max( 0, W - y ) : 0;
+         const int      o  = n > 0 ? 6 * rowStart( W, y ) * B : 0;
+         const unsigned vo = unsigned( px ) < unsigned( n ) ? unsigned( px * B ) : kDropOffset;
+#pragma unroll
+         for ( int t = 0; t < 6; ++t )
+            Q.k[r][t] = bufLoad< T >( rk, vo, o + t * n * B );
+      }
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+         Q.u[r] = loadU( y0 - 1 + r, z + 1 );
+   };
+   T lo[R + 2], loX[R + 2]; // plane z: the rows and their values at x+1
+   T cn[R], cs[R];          // contributions of layer z-1 to plane z: at the anchor's x, and at x+1 (to be shifted)
+#pragma unroll
+   for ( int r = 0; r < R; ++r )
+      cn[r] = cs[r] = T( 0 );
+   // contributions of layer z: `first` forms only those to plane z+1
+   auto layer = [&]( const ElemLayer< T, R >& Q, const T ( &hiX )[R + 2], bool first, T ( &n )[R], T ( &s )[R] ) {
+#pragma unroll
+      for ( int r = 0; r < R; ++r )
+      {
+         n[r]  = cn[r];
+         s[r]  = cs[r];
+         cn[r] = cs[r] = T( 0 );
+      }
+#pragma unroll
+      for ( int r = 0; r <= R; ++r )
+      {
+         const T u[8] = { lo[r], loX[r], lo[r + 1], loX[r + 1], Q.u[r], hiX[r], Q.u[r + 1], hiX[r + 1] };
+         T       q[8];
+#pragma unroll
+         for ( int k = 0; k < 8; ++k )
+            q[k] = T( 0 );
+         // anchor row y0-1+r: its y corners are point rows r-1 (if r > 0) and r (if r < R)
+         if ( first )
+         {
+            if ( r == 0 )
+               cubeContributions< T, 0xc0 >( K, Q.k[r], u, q );
+            else if ( r == R )
+               cubeContributions< T, 0x30 >( K, Q.k[r], u, q );
+            else
+               cubeContributions< T, 0xf0 >( K, Q.k[r], u, q );
+         }
+         else if ( r == 0 )
+            cubeContributions< T, 0xcc >( K, Q.k[r], u, q );
+         else if ( r == R )
+            cubeContributions< T, 0x33 >( K, Q.k[r], u, q );
+         else
+            cubeContributions< T, 0xff >( K, Q.k[r], u, q );
+         if ( r > 0 )
+         {
+            n[r - 1] += q[0];
+            s[r - 1] += q[1];
+            cn[r - 1] += q[4];
+            cs[r - 1] += q[5];
+         }
+         if ( r < R )
+         {
+            n[r] += q[2];
+            s[r] += q[3];
+            cn[r] += q[6];
+            cs[r] += q[7];
+         }
+      }
+   };
+   const bool     on2 = x0 == 0 && ( f2.bc & p.flag ) != 0, on3 = ( f3.bc & p.flag ) != 0;
+   const bool     mine = lane >= 1 && lane <= 62;
+   const int      pIn  = mine && px > 0 && ( p.flag & 1 ) ? px : ( 1 << 28 ); // interior when it lies before the row end
+   const unsigned vx   = unsigned( px * B ), v2 = mine && px == 0 ? 0u : kDropOffset;
+   const T        a    = p.a;
+   int            z    = z0;
+   // points of the planes z = 0 and y = 0 and the edge x = 0 on the diagonal face
+   auto boundary = [&]( int y, T val ) {
+      ElemArgsAt< T > q = ap;
+      asm volatile( "" : "+s"( q ) );
+      elemStoreBoundary( c, N, classifySlot( N, px, y, z ), px, y, z, val, q->flag, q->cinfo, q->cfs, q->prims, q->entries, q->part,
+                         q->lowPart );
+   };
+   T vEdge[R] = {}; // values of the rows' points on the edge between local vertices 2 and 3 (x = 0 on the diagonal face)
+   // one plane: `cur` holds layer z, `nxt` receives layer z+1; EDGE: the plane or a row of it lies on a face of the cell
+   auto step = [&]( auto EDGE, ElemLayer< T, R >& cur, ElemLayer< T, R >& nxt ) {
+      T ein[R], edi[R];
+#pragma unroll
+      for ( int r = 0; r < R; ++r )
+      {
+         int            n;
+         const int      o  = rowU( y0 + r, z, n );
+         // lanes past the row end read what follows in the array (or 0 past its slack); their results are dropped
+         if constexpr ( kE )
+            ein[r] = bufLoad< T >( re, vx, o );
+         if constexpr ( kD )
+            edi[r] = bufLoad< T >( rd, vx, o );
+      }
+      if ( z + 1 < z1 )
+         loadLayer( nxt, z + 1 );
+      T hiX[R + 2], n[R], s[R];
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+         hiX[r] = laneMove< kDppWaveShl1 >( cur.u[r] );
+      layer( cur, hiX, false, n, s );
+#pragma unroll
+      for ( int r = 0; r < R; ++r )
+      {
+         const T   Ax = n[r] + laneMove< kDppWaveShr1 >( s[r] );
+         const int y = y0 + r, xe = N - y - z; // row end
+         if ( xe < x0 )
+            continue; // (wave-uniform) nothing of this row in the window
+         if constexpr ( EDGE.value )
+            if ( y == 0 || z == 0 )
+            {
+               if ( mine && px <= xe )
+                  boundary( y, Ax );
+               continue;
+            }
+         int       cnt;
+         const int o  = rowU( y, z, cnt );
+         T         q0 = T( 0 ), q1 = T( 0 );
+         epilogue< T, MODE >( Ax, lo[r + 1], kE ? ein[r] : T( 0 ), kE ? ein[r] : T( 0 ), kD ? edi[r] : T( 0 ), a, q0, q1 );
+         const unsigned so = pIn < xe ? vx : kDropOffset;
+         bufStore( q0, r0, so, o );
+         if constexpr ( kTwo )
+            bufStore( q1, r1, so, o );
+         if ( xe > 0 )
+         {
+            // face points: x = 0 and the row end
+            if ( on2 )
+               bufStore( Ax, rp2, v2, facePartIndex( 2, N, 0, y, z ) * B );
+            if ( on3 && xe <= x0 + 61 )
+               bufStore( Ax, rp3, mine && px == xe ? 0u : kDropOffset, facePartIndex( 3, N, xe, y, z ) * B );
+         }
+         else
+            vEdge[r] = Ax;
+      }
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+      {
+         lo[r]  = cur.u[r];
+         loX[r] = hiX[r];
+      }
+      ++z;
+   };
+   ElemLayer< T, R > A, Bq;
+   if ( z0 > 0 )
+   {
+      T hiX[R + 2], n[R], s[R];
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+         lo[r] = loadU( y0 - 1 + r, z0 - 1 );
+      loadLayer( Bq, z0 - 1 );
+      loadLayer( A, z0 );
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+      {
+         loX[r] = laneMove< kDppWaveShl1 >( lo[r] );
+         hiX[r] = laneMove< kDppWaveShl1 >( Bq.u[r] );
+      }
+      layer( Bq, hiX, true, n, s );
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+      {
+         lo[r]  = Bq.u[r];
+         loX[r] = hiX[r];
+      }
+   }
+   else
+   {
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+         lo[r] = loadU( y0 - 1 + r, 0 );
+      loadLayer( A, 0 );
+#pragma unroll
+      for ( int r = 0; r < R + 2; ++r )
+         loX[r] = laneMove< kDppWaveShl1 >( lo[r] );
+   }
+   // The general stores of the rows y = 0 and the plane z = 0 stay out of the main loop, whose scalar registers they would
+   // spill.
+   if ( y0 == 0 || z0 == 0 )
+      do
+      {
+         step( std::true_type(), A, Bq );
+         A = Bq;
+      } while ( y0 == 0 && z < z1 );
+   while ( z < z1 )
+   {
+      step( std::false_type(), A, Bq );
+      if ( z >= z1 )
+         break;
+      step( std::false_type(), Bq, A );
+   }
+   if ( x0 == 0 && lane == 1 )
+#pragma unroll
+      for ( int r = 0; r < R; ++r )
+      {
+         z = N - y0 - r;
+         if ( y0 + r > 0 && z > 0 && z >= z0 && z < z1 )
+            boundary( y0 + r, vEdge[r] );
+      }
+}
+
+template < typename T, int MODE, int R >
+__global__ __launch_bounds__( kBlock ) void kElemSweep( ElemArgs< T > p )
+{
+   // p is the whole argument segment
+   elemSweep< T, MODE, R >( int( blockIdx.x ), (ElemArgsAt< T >) __builtin_amdgcn_kernarg_segment_ptr() );
+}
+
+// arguments of the sweep of one level, and its blocks
+template < typename T >
+ElemArgs< T > elemArgs( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::Level& ol, int L, const StencilCall& c )
+{
+   constexpr bool dbl = std::is_same< T, double >::value;
+   ElemArgs< T >  e;
+   e.segs    = g.eSegs;
+   e.nSegs   = g.nESegs;
+   e.nC      = m.mesh->nC();
+   e.L       = L;
+   e.stride  = g.stride;
+   e.cells   = ol.elem;
+   e.kb      = dbl ? (const T*) ol.kb : (const T*) ol.kbF;
+   e.cinfo   = m.cellInfo;
+   e.cfs     = m.cellFaces;
+   e.prims   = m.prims;
+   e.entries = m.entries;
+   e.part    = dbl ? (T*) ol.facePart : (T*) ol.facePartF;
+   e.lowPart = dbl ? (T*) ol.lowPart : (T*) ol.lowPartF;
+   e.dinv    = dbl ? (const T*) ol.dinv : (const T*) ol.dinvF;
+   e.flag    = c.flag;
+   e.x       = (const T*) c.x;
+   e.in1     = (const T*) c.in1;
+   e.out0    = (T*) c.out0;
+   e.out1    = (T*) c.out1;
+   e.a       = T( c.a );
+   return e;
+}
+template < typename T >
+int elemBlocks( const ElemArgs< T >& e )
+{
+   return xcdGrid( ( ( e.nSegs + 3 ) / 4 ) * e.nC );
+}
+
+// One thread per point of the closed macro-cell, for what is not done by the march above. DIAG: the diagonal entry instead of
+// the product. BND: the points on the cell's faces, edges and vertices only, listed in bnd[0 .. nBnd) by their index in the
+// cell array (the surrogate operator does the interior points itself). STW: the point's stencil weights are read from wst
 // ([cell][direction][point], the blended operator) instead of assembled from the coefficient integrals.
 template < typename T, int MODE, bool DIAG, bool BND = false, bool STW = false >
 __device__ __forceinline__ void bElemApply( int bid, int L, int tilesPerCell, i64 stride, const ElemCell* __restrict__ cells,
@@ -182,7 +623,7 @@ __device__ __forceinline__ void bElemApply( int bid, int L, int tilesPerCell, i6
 {
    const int c    = bid / tilesPerCell;
    const int tile = bid - c * tilesPerCell;
-   const int N = 1 << L, w = N + 1, NP = N + 1;
+   const int N = 1 << L, w = N + 1;
    int       s = tile * kBlock + int( threadIdx.x );
    if constexpr ( BND )
    {
@@ -238,27 +679,8 @@ __device__ __forceinline__ void bElemApply( int bid, int L, int tilesPerCell, i6
             out1[q] = r1;
       }
    }
-   else if ( slot <= 4 )
-   {
-      const CellFaceSlot fs = cfs[4 * c + slot - 1];
-      if ( fs.bc & flag )
-         part[i64( fs.block ) * NP * NP + facePartIndex( slot - 1, N, px, py, pz )] = val;
-   }
    else
-   {
-      const CellInfo& ci = cinfo[c];
-      if ( prims[ci.prim[slot]].bc & flag )
-      {
-         const int e = ci.entry[slot];
-         int       i = 0;
-         if ( slot <= 10 )
-         {
-            const int b[4] = { N - px - py - pz, px, py, pz };
-            i              = b[entries[e].l1];
-         }
-         lowPart[i64( e ) * NP + i] = val;
-      }
-   }
+      elemStoreBoundary( c, N, slot, px, py, pz, val, flag, cinfo, cfs, prims, entries, part, lowPart );
 }
 
 template < typename T, int MODE, bool DIAG, bool BND = false, bool STW = false >

@@ -118,6 +118,12 @@ struct ZSeg
 constexpr int kZSegChunk = 24;
 constexpr int kZSegLeast = 4;
 constexpr int kZSegWaves = 8192;
+// The variable-coefficient sweep: one row per wavefront (two rows share more loads and edge differences but halve the waves
+// in flight: 208 against 196 us for an FP32 sweep at level 7), and segments for four times the waves (6 planes at level 7
+// on 24 cells: with 4 / 6 / 8 / 12 / 16 / 24 planes that sweep takes 188 / 181 / 180 / 182 / 186 / 196 us, a batched cycle
+// of 12 problems of levels 4 to 6 4.42 / 4.43 / 4.51 / 4.82 / 5.00 / 5.42 ms).
+constexpr int kElemRows  = 1;
+constexpr int kElemWaves = 32768;
 // P2 constant operator, z-marching row pairs: a wavefront computes rows y0 (even) and y0+1 of a segment of
 // kP2ZSeg x values (x0 = kP2ZSeg k - 2 + 2 lane, lanes 0 and 63 halo) over planes [z0, z1), z0 even; the
 // table stores (y0, k, z0, z1) in a ZSeg.
@@ -205,6 +211,7 @@ struct ElemCell
    double v0[3];       // position of local vertex 0
    double a[3][3];     // a[r][k]: component r of (v_{k+1} - v0) / N, the lattice step along local axis k
    double mt[6][16];   // element matrix of each micro-cell type for k = 1 (vertex order of the type)
+   float  mtF[6][16];  // the same rounded to FP32
 };
 
 // P2 (quadratic Lagrange) on the refined vertex lattice: a P2 function of level L keeps its vertex DoFs at
@@ -563,6 +570,10 @@ struct LevelGeom
          for ( int& v : t )
             v = -1;
    }
+   // variable-coefficient operator: z-marching segments over all points of a cell, rows and planes from 0 (elemSweep)
+   std::vector< ZSeg >                      eSegsHost;
+   ZSeg*                                    eSegs  = nullptr;
+   int                                      nESegs = 0;
    std::vector< int4 >                      flatItemsHost; // z = 0 / y = 0 face rows: (cell, slot, line, x0)
    int4*                                    flatItems  = nullptr;
    int                                      nFlatItems = 0;

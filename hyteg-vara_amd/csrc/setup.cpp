@@ -356,6 +356,23 @@ LevelGeom& MeshCtx::geom( int L )
       g.nZSegs[k] = (int) v.size();
       g.zSegs[k]  = upload( v );
    }
+   {
+      // variable-coefficient sweep: rows y .. y+kElemRows-1, points x0 .. x0+61, planes z0 .. z1-1 of the closed cell
+      auto& v = g.eSegsHost;
+      v.clear();
+      i64 steps = 0;
+      for ( int y = 0; y <= N; y += kElemRows )
+         for ( int x0 = 0; x0 <= N - y; x0 += 62 )
+            steps += N - y - x0 + 1;
+      const int most  = int( std::max< i64 >( kZSegLeast, std::min< i64 >( kZSegChunk, steps * mesh->nC() / kElemWaves ) ) );
+      const int chunk = ec ? std::max( 2, std::min( 1024, std::atoi( ec ) ) ) : most;
+      for ( int z0 = 0; z0 <= N; z0 += chunk )
+         for ( int x0 = 0; x0 <= N - z0; x0 += 62 )
+            for ( int y = 0; y + x0 + z0 <= N; y += kElemRows )
+               v.push_back( { y, x0, z0, std::min( z0 + chunk, N - y - x0 + 1 ) } );
+      g.nESegs = (int) v.size();
+      g.eSegs  = upload( v );
+   }
    // P2 row pairs (y0, y0+1), y0 even: segment k holds the x values 124k .. 124k+123 (k = 0 from x = 1); the
    // pair has interior outputs while z <= N - 1 - x_first - max(y0, 1). Planes are chunked from z = 0 so every
    // segment starts on an even plane (plane 0 itself has no interior output).
@@ -425,6 +442,7 @@ MeshCtx::~MeshCtx()
       (void) hipFree( g.tiles );
       for ( auto* zs : g.zSegs )
          (void) hipFree( zs );
+      (void) hipFree( g.eSegs );
       (void) hipFree( g.flatItems );
       for ( auto* zs : g.p2ZSegs )
          (void) hipFree( zs );
@@ -565,7 +583,10 @@ void assembleP1DivKGrad( hyg_op_s& op )
          for ( int t = 0; t < 6; ++t )
             for ( int i = 0; i < 4; ++i )
                for ( int j = 0; j < 4; ++j )
-                  ec[c].mt[t][4 * i + j] = K[t][i][j];
+               {
+                  ec[c].mt[t][4 * i + j]  = K[t][i][j];
+                  ec[c].mtF[t][4 * i + j] = float( K[t][i][j] );
+               }
       }
       ol.elem                = upload( ec );
       const size_t nKb       = size_t( m.nC() ) * 6 * size_t( S3( N ) );

@@ -57,3 +57,65 @@ def test_face_points_in_the_sweep_and_from_one_sided_sums(hyg, name, L, dtype):
             else:
                 op.smooth_jac(d, b, x, 0.7, L, flag)
             assert rel_inf(d.download(L), np.where(on, ref, d0)) <= TOL[dt], (what, flag)
+
+
+# 8 modes of wavenumber <= 3: FP32 phases up to 2 pi 3 sqrt(3) |x| ~ 60 are off by 60 * 2^-24, which moves a cosine of total
+# amplitude 0.5 sqrt(2 * 8) and so log k by 8e-6 at most; with the 34 roundings of the sum this stays below 2e-5
+@pytest.mark.parametrize("dtype", ["F64", "F32"])
+@pytest.mark.parametrize("name,L", [("three_tets_with_two_joint_faces.msh", 0), ("three_tets_with_two_joint_faces.msh", 1),
+                                    ("pyramid_tilted_4el.msh", 6), ("three_tets_with_two_joint_faces.msh", 7)])
+def test_variable_coefficient_sweep(hyg, name, L, dtype):
+    """The z-marching sweep: rows of one and of several 62-point windows, segments of 4 to 24 planes, every kind of point."""
+    dt = getattr(hyg, dtype)
+    modes = ol.random_field(33, modes=8, kmax=3)
+    gm, om = hyg.Mesh(name), ol.Mesh(name)
+    n = gm.ndofs(L)
+    x0, b0, d0 = (rnd(n, 30 + k, dt == hyg.F32) for k in range(3))
+    op = hyg.P1DivKGradOperator(gm, L, L, 1.3, modes)
+    op.store_local_matrices()
+    oop = ol.DivKGradOperator(om, L, L, ("fourier", 1.3, modes))
+    ox, od = ol.Function(om, L, L), ol.Function(om, L, L)
+    ox.set(L, x0)
+    oop.apply(ox, od, L, ol.ALL, False)
+    Ax = od.get(L)
+    inv = hyg.Function(gm, L, L)
+    op.inverse_diagonal(inv, L)
+    dinv = inv.download(L)
+    bnd = gm.boundary(L)
+    for flag in (hyg.INNER, hyg.ALL):
+        on = ~bnd if flag == hyg.INNER else np.ones(n, dtype=bool)
+        x, b, d = (hyg.Function(gm, L, L, dt) for _ in range(3))
+        x.upload(L, x0)
+        b.upload(L, b0)
+        for what, ref in (("apply", Ax), ("add", d0 + Ax), ("residual", b0 - Ax), ("jacobi", x0 + 0.7 * dinv * (b0 - Ax))):
+            print(name, L, dtype, flag, what, flush=True)
+            d.upload(L, d0)
+            if what in ("apply", "add"):
+                op.apply(x, d, L, flag, hyg.ADD if what == "add" else hyg.REPLACE)
+            elif what == "residual":
+                op.residual(d, b, x, L, flag)
+            else:
+                op.smooth_jac(d, b, x, 0.7, L, flag)
+            assert rel_inf(d.download(L), np.where(on, ref, d0)) <= (1e-13 if dt == hyg.F64 else 2e-5), (what, flag)
+
+
+def test_points_do_not_see_values_that_are_not_their_neighbours(hyg):
+    """An infinite value reaches the points whose stencil holds it and no other (the lanes past a row end of the sweep)."""
+    L, name = 6, "tet_1el.msh"
+    gm, om = hyg.Mesh(name), ol.Mesh(name)
+    n = gm.ndofs(L)
+    modes = ol.random_field(33, modes=8, kmax=3)
+    op = hyg.P1DivKGradOperator(gm, L, L, 1.3, modes)
+    op.store_local_matrices()
+    xyz, _ = gm.coords(L)
+    rng = np.random.default_rng(8)
+    x, y = hyg.Function(gm, L, L), hyg.Function(gm, L, L)
+    for k in rng.choice(n, 12, replace=False):
+        v = rng.uniform(-1.0, 1.0, n)
+        v[k] = np.inf
+        x.upload(L, v)
+        op.apply(x, y, L, hyg.ALL)
+        bad = ~np.isfinite(y.download(L))
+        assert bad[k]
+        # neighbours lie within one lattice step in every local coordinate
+        assert np.abs(xyz[bad] - xyz[k]).max() <= 2.0 * np.abs(xyz).max() / (1 << L) + 1e-12

@@ -8,10 +8,9 @@
 // ElemCell::mt) and kb_e = 6 sum_q w_q k(x_q) is the 5-point degree-3 quadrature of k over the
 // element divided by its volume (w = -2/15 at the centroid, 3/40 at the four points with barycentric
 // coordinates (1/2, 1/6, 1/6, 1/6)). Each apply
-//   1. evaluates kb_e for every micro-cell (kKBar): per lattice point the phases of the Fourier modes of
-//      k are formed once and the 30 quadrature points of the six cell types are reached by angle
-//      addition with per-cell tables of cos/sin of the quadrature offsets (kKBarTables, once per level at
-//      operator creation; read with scalar loads);
+//   1. evaluates kb_e for every micro-cell (kKBar): the log-coefficient at the 30 quadrature points of the six cell
+//      types of a lattice point is a matrix product of the modes' phase factors there with a constant matrix of
+//      their amplitudes and offsets (kKBarTables, once per level at operator creation), on the matrix cores;
 //   2. marches over the cubes of the anchor lattice plane by plane and adds the contributions of their six elements to
 //      the corners (kElemSweep); interior points get the epilogue, points on faces, edges and vertices store the cell's
 //      one-sided sum;
@@ -24,44 +23,64 @@
 namespace hyg {
 
 // ------------------------------------------------------------------ coefficient tables
-// Tables of one level, built once (one block per cell): per mode the phase at the cell's vertex 0, its steps
-// along the three lattice axes and the amplitude (phase[(c nModes + m) 5 + ..]), and cos/sin of the phase offsets of
-// the 30 quadrature points of the six types from their anchor (tab[(c nModes + m) 60 + 2 (5 t + q) + {0, 1}]).
+// Tables of one level, built once. axis[((c 3 + axis) N + n) MP + m]: e^(i phase) of mode m at n lattice steps along an axis
+// (axis 0: with the phase at the cell's vertex 0), MP modes with zeros behind the nModes given; mat: the matrix of kKBar in
+// the order in which its lanes hold it (step, tile, lane). Phases are reduced in turns before the sine is taken.
+template < typename T >
+__device__ void kbMatrix( const ElemCell& ec, const double* __restrict__ modes, int nModes, int i, T* __restrict__ mat )
+{
+   const int s = i >> 7, tile = ( i >> 6 ) & 1, lane = i & 63, k = 4 * s + ( lane >> 4 ), m = k >> 1;
+   int       g, r;
+   mmaRow( lane & 15, g, r, static_cast< T* >( nullptr ) );
+   const int j = 4 * tile + r; // slot of the group
+   const int t = j < 5 ? g : 4 + ( g >> 1 ), q = j < 5 ? j : ( ( g & 1 ) ? j - 2 : j - 5 );
+   double    v = 0.0;
+   if ( m < nModes && q < 5 )
+   {
+      double d[3] = { 0.0, 0.0, 0.0 }; // lattice offset of quadrature point q of type t from the anchor
+      for ( int u = 0; u < 4; ++u )
+      {
+         const double lam = q == 0 ? 0.25 : ( u == q - 1 ? 0.5 : 1.0 / 6.0 );
+         for ( int b = 0; b < 3; ++b )
+            d[b] += lam * kMC[t][u][b];
+      }
+      double turns = 0.0;
+      for ( int b = 0; b < 3; ++b )
+         turns += d[b] * ( modes[5 * m] * ec.a[0][b] + modes[5 * m + 1] * ec.a[1][b] + modes[5 * m + 2] * ec.a[2][b] );
+      double sn, cs;
+      sincos( 2.0 * M_PI * turns, &sn, &cs );
+      v = modes[5 * m + 4] * ( ( k & 1 ) ? -sn : cs );
+   }
+   mat[i] = T( v );
+}
 __global__ __launch_bounds__( kBlock ) void kKBarTables( const ElemCell* __restrict__ cells, const double* __restrict__ modes, int nModes,
-                                                         double* __restrict__ phase, double* __restrict__ tab, float* __restrict__ tabF )
+                                                         int MP, int N, KbPair< double >* __restrict__ axis,
+                                                         KbPair< float >* __restrict__ axisF, double* __restrict__ mat,
+                                                         float* __restrict__ matF )
 {
    const int       c  = int( blockIdx.x );
    const ElemCell& ec = cells[c];
-   double*         mp = phase + i64( c ) * nModes * 5;
-   for ( int m = int( threadIdx.x ); m < nModes; m += kBlock )
+   const int       i0 = int( blockIdx.y ) * kBlock + int( threadIdx.x ), step = int( gridDim.y ) * kBlock;
+   for ( int i = i0; i < 3 * N * MP; i += step )
    {
-      const double kx = modes[5 * m], ky = modes[5 * m + 1], kz = modes[5 * m + 2];
-      const double tp = 2.0 * M_PI;
-      mp[5 * m]       = tp * ( kx * ec.v0[0] + ky * ec.v0[1] + kz * ec.v0[2] ) + modes[5 * m + 3];
-      for ( int k = 0; k < 3; ++k )
-         mp[5 * m + 1 + k] = tp * ( kx * ec.a[0][k] + ky * ec.a[1][k] + kz * ec.a[2][k] );
-      mp[5 * m + 4] = modes[5 * m + 4];
-   }
-   __syncthreads();
-   for ( int i = int( threadIdx.x ); i < 30 * nModes; i += kBlock )
-   {
-      const int m = i / 30, tq = i - 30 * m, t = tq / 5, q = tq - 5 * t;
-      // lattice offset of quadrature point q of type t from the anchor
-      double d[3] = { 0.0, 0.0, 0.0 };
-      for ( int v = 0; v < 4; ++v )
+      const int m = i % MP, n = ( i / MP ) % N, b = i / ( MP * N );
+      double    cs = 0.0, sn = 0.0;
+      if ( m < nModes )
       {
-         const double lam = q == 0 ? 0.25 : ( v == q - 1 ? 0.5 : 1.0 / 6.0 );
-         for ( int k = 0; k < 3; ++k )
-            d[k] += lam * kMC[t][v][k];
+         const double kx = modes[5 * m], ky = modes[5 * m + 1], kz = modes[5 * m + 2];
+         double       t  = n * ( kx * ec.a[0][b] + ky * ec.a[1][b] + kz * ec.a[2][b] );
+         if ( b == 0 )
+            t += kx * ec.v0[0] + ky * ec.v0[1] + kz * ec.v0[2];
+         sincos( 2.0 * M_PI * ( t - rint( t ) ) + ( b == 0 ? modes[5 * m + 3] : 0.0 ), &sn, &cs );
       }
-      const double ang = mp[5 * m + 1] * d[0] + mp[5 * m + 2] * d[1] + mp[5 * m + 3] * d[2];
-      double       sn, cs;
-      sincos( ang, &sn, &cs );
-      const i64 o  = ( i64( c ) * nModes ) * 60 + 2 * i;
-      tab[o]       = cs;
-      tab[o + 1]   = sn;
-      tabF[o]      = float( cs );
-      tabF[o + 1]  = float( sn );
+      const i64 o = i64( c ) * 3 * N * MP + i;
+      axis[o]     = { cs, sn };
+      axisF[o]    = { float( cs ), float( sn ) };
+   }
+   for ( int i = i0; i < MP * 64; i += step )
+   {
+      kbMatrix( ec, modes, nModes, i, mat + i64( c ) * MP * 64 );
+      kbMatrix( ec, modes, nModes, i, matF + i64( c ) * MP * 64 );
    }
 }
 
@@ -69,26 +88,39 @@ __global__ __launch_bounds__( kBlock ) void kKBarTables( const ElemCell* __restr
 template < typename T >
 static void launchKBar( const hyg_op_s& op, int L, int nC, T* kb, hipStream_t s )
 {
-   const int N  = 1 << L;
-   const int tK = ceilDiv( S3i( N ), kBlock );
-   if ( tK > 0 && S3i( N ) > 0 && op.kPolyDeg >= 0 )
-      hipLaunchKernelGGL( ( kKBarPoly< T > ), dim3( nC * tK ), dim3( kBlock ), 0, s, L, tK, op.levels[L].elem, op.kPoly, op.kPolyDeg, kb );
-   else if ( tK > 0 && S3i( N ) > 0 )
+   constexpr bool         dbl = std::is_same< T, double >::value;
+   const hyg_op_s::Level& ol  = op.levels[L];
+   const int              N   = 1 << L;
+   if ( op.kPolyDeg >= 0 )
    {
-      const hyg_op_s::Level& ol = op.levels[L];
-      const T*               tb = std::is_same< T, double >::value ? (const T*) ol.kbTab : (const T*) ol.kbTabF;
-      hipLaunchKernelGGL( ( kKBar< T > ), dim3( nC * tK ), dim3( kBlock ), 0, s, L, tK, (const double*) ol.kbPhase, tb, op.nModes, op.k0,
-                          kb );
+      const int tK = ceilDiv( S3i( N ), kBlock );
+      hipLaunchKernelGGL( ( kKBarPoly< T > ), dim3( nC * tK ), dim3( kBlock ), 0, s, L, tK, ol.elem, op.kPoly, op.kPolyDeg, kb );
+      return;
    }
+   const int   rows   = nC * N * ceilDiv( N, kKBarRows ) >= 2048 ? kKBarRows : 16; // 2048: four blocks per CU and half of them empty
+   const int   chunks = ceilDiv( N, rows );
+   const auto* axis   = static_cast< const KbPair< T >* >( dbl ? ol.kbAxis : ol.kbAxisF );
+   const T*    mat    = dbl ? (const T*) ol.kbMat : (const T*) ol.kbMatF;
+   auto        kf     = kKBar< T, 32 >;
+   switch ( kbModes( op.nModes ) )
+   {
+   case 8: kf = kKBar< T, 4 >; break;
+   case 32: kf = kKBar< T, 16 >; break;
+   default: break;
+   }
+   hipLaunchKernelGGL( kf, dim3( nC * N * chunks ), dim3( kBlock ), 0, s, N, nC, rows, axis, mat, T( op.k0 ), kb );
 }
 
-// per-level tables of the Fourier coefficient (phases and quadrature-offset cos/sin), once at operator setup
+// per-level tables of the Fourier coefficient, once at operator setup
 void launchKBarTables( const MeshCtx& m, const hyg_op_s& op, int L, hipStream_t s )
 {
    const hyg_op_s::Level& ol = op.levels[L];
-   if ( op.nModes > 0 )
-      hipLaunchKernelGGL( kKBarTables, dim3( m.mesh->nC() ), dim3( kBlock ), 0, s, ol.elem, op.modes, op.nModes, ol.kbPhase, ol.kbTab,
-                          ol.kbTabF );
+   if ( op.kPolyDeg >= 0 || !ol.kbAxis )
+      return;
+   const int N = 1 << L, MP = kbModes( op.nModes );
+   hipLaunchKernelGGL( kKBarTables, dim3( m.mesh->nC(), std::min( 16, ceilDiv( 3 * N * MP, kBlock ) ) ), dim3( kBlock ), 0, s, ol.elem,
+                       op.modes, op.nModes, MP, N, static_cast< KbPair< double >* >( ol.kbAxis ),
+                       static_cast< KbPair< float >* >( ol.kbAxisF ), ol.kbMat, ol.kbMatF );
 }
 
 // coefficient integrals of every level in both value types, kept for the applies that follow

@@ -17,8 +17,6 @@ constexpr int kMCOff[6][4] = { { 0, 1, 2, 4 }, { 1, 3, 2, 5 }, { 1, 2, 5, 4 }, {
 // 6 x the quadrature weights (centroid first), so that kb = 1 for k = 1
 constexpr double kQW6[5] = { -0.8, 0.45, 0.45, 0.45, 0.45 };
 
-__device__ __forceinline__ void sincosT( double a, double& s, double& c ) { sincos( a, &s, &c ); }
-__device__ __forceinline__ void sincosT( float a, float& s, float& c ) { sincosf( a, &s, &c ); }
 __device__ __forceinline__ double expT( double a ) { return exp( a ); }
 __device__ __forceinline__ float  expT( float a ) { return expf( a ); }
 
@@ -28,53 +26,107 @@ __device__ __forceinline__ float  expT( float a ) { return expf( a ); }
 __device__ __forceinline__ int kbRow( int N, int y, int z ) { return 6 * ( S3i( N ) - S3i( N - z ) + rowStart( N - z, y ) ); }
 
 // ------------------------------------------------------------------ 1. coefficient integrals
-// One thread per anchor (x, y, z), x+y+z <= N-1, of one macro-cell; kb[c][t][anchor] for the six types. The tables
-// of the block's cell are wave-uniform: they are read with scalar loads and feed the multiply-adds directly.
+// k(x_q) = k0 exp( g ), g = sum_m a_m cos( theta_m + delta_mq ) with the phase theta_m of the anchor and delta_mq of the
+// quadrature point's offset from it: for all anchors of a cell a product of the 30 x 2M matrix (a cos delta, -a sin delta)
+// with the 2M x anchors matrix (cos theta, sin theta), done on the matrix cores (16 x 16 x 4 tiles of the same precision).
+// e^(i theta) = X_m[x] Y_m[y] Z_m[z] from tables of the three lattice axes, so no sine is taken here.
+//
+// Rows of the product: 32 slots, 8 for each of the four 16-lane groups of a wave (that is where a lane finds its results):
+// slots 0..4 of group g are the points of type g; types 4 and 5 are shared by groups 0, 1 and 2, 3 (points 0..2 and 3, 4 in
+// slots 5..7), the last slot of groups 1 and 3 is empty. Columns: 16 anchors of a row.
+// A block takes rowsPer (32, or 16 where that leaves too few blocks) rows of a plane, each wave every fourth of them; per tile
+// of 16 anchors a wave holds X Z (2 values per step in registers) and walks its rows, whose Y is staged in LDS with the
+// constant matrix. (Waves on tiles of their own, whose rows are fewer at large x: 1570 us.)
+// 32 modes, level 7, 24 cells (8.6 million anchors): FP64 2180 -> 1130 us, FP32 814 -> 600 us against a thread per anchor with
+// a sincos per mode and the matrix read through the scalar cache. The FP64 time is that of 2 S matrix instructions (30 ns
+// each per SIMD, 600 us in all; 30 of 32 rows used) and of the 8 exponentials per lane, which use the same FP64 units.
+constexpr int kKBarRows = 32;
+
+typedef double f64x4 __attribute__( ( ext_vector_type( 4 ) ) );
+typedef float  f32x4 __attribute__( ( ext_vector_type( 4 ) ) );
+__device__ __forceinline__ f64x4 mma16( double a, double b, f64x4 c ) { return __builtin_amdgcn_mfma_f64_16x16x4f64( a, b, c, 0, 0, 0 ); }
+__device__ __forceinline__ f32x4 mma16( float a, float b, f32x4 c ) { return __builtin_amdgcn_mfma_f32_16x16x4f32( a, b, c, 0, 0, 0 ); }
+// lane group and slot within its tile of row i of a 16 x 16 result: FP64 results lie 4 rows apart, FP32 ones in sequence
+__device__ __forceinline__ void mmaRow( int i, int& g, int& r, double* ) { g = i & 3, r = i >> 2; }
+__device__ __forceinline__ void mmaRow( int i, int& g, int& r, float* ) { g = i >> 2, r = i & 3; }
+
 template < typename T >
-__global__ __launch_bounds__( kBlock ) void kKBar( int L, int tilesPerCell, const double* __restrict__ phase, const T* __restrict__ tab,
-                                                   int nModes, double k0, T* __restrict__ kb )
+struct KbPair
 {
-   typedef const double __attribute__( ( address_space( 4 ) ) ) CD;
-   typedef const T __attribute__( ( address_space( 4 ) ) ) CT;
-   const int c    = int( blockIdx.x ) / tilesPerCell;
-   const int tile = int( blockIdx.x ) - c * tilesPerCell;
-   const int N    = 1 << L;
-   const CD* mp   = (const CD*) ( phase + i64( c ) * nModes * 5 );
-   const CT* tc   = (const CT*) ( tab + i64( c ) * nModes * 60 );
-   const int S    = S3i( N );
-   const int s    = tile * kBlock + int( threadIdx.x );
-   if ( s >= S )
+   T re, im;
+};
+
+template < typename T, int S >
+__global__ __launch_bounds__( kBlock, S > 16 ? 1 : ( sizeof( T ) == 8 ? 2 : 3 ) ) void kKBar( int N, int nC, int rowsPer, const KbPair< T >* __restrict__ axis, const T* __restrict__ mat, T k0,
+                                                   T* __restrict__ kb )
+{
+   typedef typename std::conditional< std::is_same< T, double >::value, f64x4, f32x4 >::type V4;
+   constexpr int          MP = 2 * S;
+   __shared__ T           At[S * 128];
+   __shared__ KbPair< T > Yt[kKBarRows * MP];
+   // cell fastest, then plane, then row chunk: all cells' blocks of a kind have the same work, so the 8 XCDs, which get blocks
+   // in turn, are loaded alike, and the large blocks come first (row chunk fastest: one XCD had all the long rows, 2750 us)
+   const int              c  = int( blockIdx.x ) % nC;
+   const int              b  = int( blockIdx.x ) / nC;
+   const int              z = b % N, y0 = b / N * rowsPer;
+   if ( y0 + z >= N ) // (the whole block) no anchors
       return;
-   int x, y, z;
-   tetXYZ( N, s, x, y, z );
-   T g[30];
-#pragma unroll
-   for ( int k = 0; k < 30; ++k )
-      g[k] = T( 0 );
-   for ( int m = 0; m < nModes; ++m )
+   const int          rows = min( rowsPer, N - z - y0 );
+   const KbPair< T >* ax   = axis + i64( c ) * 3 * N * MP;
+   for ( int i = int( threadIdx.x ); i < S * 128; i += kBlock )
+      At[i] = mat[i64( c ) * S * 128 + i];
+   for ( int i = int( threadIdx.x ); i < rows * MP; i += kBlock )
+      Yt[i] = ax[( N + y0 ) * MP + i];
+   __syncthreads();
+   const int lane = int( threadIdx.x & 63u ), g = lane >> 4, h = g >> 1;
+   const int tMax = g == 0 ? kMCMax[0] : ( g == 3 ? kMCMax[3] : kMCMax[1] ); // of type g (types 1 and 2 alike)
+   T*        out  = kb + i64( c ) * 6 * S3i( N );
+   const int wave = int( threadIdx.x >> 6 );
+   for ( int xt = 0; 16 * xt < N - z - y0 - wave; ++xt )
    {
-      const T th = T( mp[5 * m] + mp[5 * m + 1] * x + mp[5 * m + 2] * y + mp[5 * m + 3] * z );
-      T       sn, cs;
-      sincosT( th, sn, cs );
-      const T   am = T( mp[5 * m + 4] );
-      const T   ac = am * cs, as = am * sn;
-      const CT* tb = tc + 60 * m;
+      const int x = 16 * xt + ( lane & 15 );
+      T         a[S], d[S];
 #pragma unroll
-      for ( int k = 0; k < 30; ++k )
-         g[k] += ac * tb[2 * k] - as * tb[2 * k + 1];
-   }
-   T*        out = kb + i64( c ) * 6 * S + kbRow( N, y, z ) + x;
-   const int nx  = N - y - z;
+      for ( int s = 0; s < S; ++s )
+      {
+         const KbPair< T > X = ax[min( x, N - 1 ) * MP + 2 * s + h], Z = ax[( 2 * N + z ) * MP + 2 * s + h];
+         const T           re = X.re * Z.re - X.im * Z.im, im = X.re * Z.im + X.im * Z.re;
+         a[s] = ( g & 1 ) ? im : re; // (X Z Y)'s real or imaginary part = a Y.re + d Y.im
+         d[s] = ( g & 1 ) ? re : -im;
+      }
+      for ( int y = y0 + wave; y < y0 + rows && 16 * xt < N - z - y; y += kBlock / 64 )
+      {
+         V4                 c0 = { 0, 0, 0, 0 }, c1 = { 0, 0, 0, 0 };
+         const KbPair< T >* Yr = Yt + ( y - y0 ) * MP + h;
 #pragma unroll
-   for ( int t = 0; t < 6; ++t )
-   {
-      T v = T( 0 );
+         for ( int s = 0; s < S; ++s )
+         {
+            const KbPair< T > Y = Yr[2 * s];
+            const T           v = a[s] * Y.re + d[s] * Y.im;
+            c0                  = mma16( At[128 * s + lane], v, c0 );
+            c1                  = mma16( At[128 * s + 64 + lane], v, c1 );
+         }
+         T v = T( kQW6[0] ) * expT( T( c0[0] ) );
 #pragma unroll
-      for ( int q = 0; q < 5; ++q )
-         v += T( kQW6[q] ) * expT( g[5 * t + q] );
-      out[t * nx] = x + y + z + kMCMax[t] <= N ? T( k0 ) * v : T( 0 ); // 0: the element is not in the cell
+         for ( int q = 1; q < 4; ++q )
+            v += T( kQW6[q] ) * expT( T( c0[q] ) );
+         v += T( kQW6[4] ) * expT( T( c1[0] ) );
+         T e = T( ( g & 1 ) ? kQW6[3] : kQW6[0] ) * expT( T( c1[1] ) ) + T( kQW6[1] ) * expT( T( c1[2] ) );
+         e += T( ( g & 1 ) ? 0.0 : kQW6[2] ) * expT( T( c1[3] ) );
+         e += __shfl_xor( e, 16, 64 );
+         const int nx = N - y - z;
+         if ( x < nx )
+         {
+            // 0: the element is not in the cell
+            T* o      = out + kbRow( N, y, z ) + x;
+            o[g * nx] = x + tMax <= nx ? k0 * v : T( 0 );
+            if ( !( g & 1 ) )
+               o[( 4 + h ) * nx] = x + kMCMax[4] <= nx ? k0 * e : T( 0 );
+         }
+      }
    }
 }
+static_assert( kMCMax[1] == kMCMax[2] && kMCMax[4] == kMCMax[5], "types handled alike by kKBar" );
 
 // The same integrals for a polynomial coefficient k(x) = sum_i poly[i] x^a y^b z^c over the monomials of degree <= deg
 // in the order of the reference's MonomialBasis3D (by total degree; within a degree by decreasing a, then b). One

@@ -479,6 +479,9 @@ constexpr double kXG4Weight[11] = { 0.006541848487473325,  0.0092122281926561474
                                     0.0099888641910932524, 0.011578327656272558,  0.012693785874259723, 0.013237780011337548,
                                     0.017744672359248346,  0.018372372071416277,  0.025829352669374347 };
 
+// modes of a Fourier coefficient (at most 64) padded to what a variant of kKBar holds
+inline int kbModes( int n ) { return n <= 8 ? 8 : ( n <= 32 ? 32 : 64 ); }
+
 // ------------------------------------------------------------------ host objects
 struct Mesh
 {
@@ -729,11 +732,12 @@ struct hyg_op_s
       hyg::ElemCell*        elem    = nullptr;
       double*               kb      = nullptr;
       float*                kbF     = nullptr;
-      // Fourier coefficient: per cell and mode the phase terms (theta0, gx, gy, gz, amplitude) and the cos/sin of the
-      // 30 quadrature offsets of the six micro-cell types (built once at operator setup, read by kKBar)
-      double*               kbPhase = nullptr;
-      double*               kbTab   = nullptr;
-      float*                kbTabF  = nullptr;
+      // Fourier coefficient: per cell the phase factors of the modes along the three lattice axes (pairs of cos, sin) and
+      // the matrix of their amplitudes at the 30 quadrature offsets (built once at operator setup, read by kKBar)
+      void*                 kbAxis  = nullptr;
+      void*                 kbAxisF = nullptr;
+      double*               kbMat   = nullptr;
+      float*                kbMatF  = nullptr;
       double*               lowPart = nullptr;
       float*                lowPartF = nullptr;
       double*               dinv    = nullptr;

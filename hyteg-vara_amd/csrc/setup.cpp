@@ -601,12 +601,13 @@ void assembleP1DivKGrad( hyg_op_s& op )
       ol.facePartF = static_cast< float* >( alloc( nFace * sizeof( float ) ) );
       ol.dinv      = static_cast< double* >( alloc( nFunc * sizeof( double ) ) );
       ol.dinvF     = static_cast< float* >( alloc( nFunc * sizeof( float ) ) );
-      if ( op.nModes > 0 )
+      if ( op.kPolyDeg < 0 && !op.blend )
       {
-         const size_t nm = size_t( m.nC() ) * size_t( op.nModes );
-         ol.kbPhase      = static_cast< double* >( alloc( nm * 5 * sizeof( double ) ) );
-         ol.kbTab        = static_cast< double* >( alloc( nm * 60 * sizeof( double ) ) );
-         ol.kbTabF       = static_cast< float* >( alloc( nm * 60 * sizeof( float ) ) );
+         const size_t nm = size_t( m.nC() ) * size_t( kbModes( op.nModes ) );
+         ol.kbAxis       = alloc( nm * 6 * N * sizeof( double ) );
+         ol.kbAxisF      = alloc( nm * 6 * N * sizeof( float ) );
+         ol.kbMat        = static_cast< double* >( alloc( nm * 64 * sizeof( double ) ) );
+         ol.kbMatF       = static_cast< float* >( alloc( nm * 64 * sizeof( float ) ) );
       }
    }
 }
@@ -962,9 +963,10 @@ hyg_op_s::~hyg_op_s()
       (void) hipFree( l.elem );
       (void) hipFree( l.kb );
       (void) hipFree( l.kbF );
-      (void) hipFree( l.kbPhase );
-      (void) hipFree( l.kbTab );
-      (void) hipFree( l.kbTabF );
+      (void) hipFree( l.kbAxis );
+      (void) hipFree( l.kbAxisF );
+      (void) hipFree( l.kbMat );
+      (void) hipFree( l.kbMatF );
       (void) hipFree( l.lowPart );
       (void) hipFree( l.lowPartF );
       (void) hipFree( l.dinv );

@@ -119,3 +119,27 @@ def test_points_do_not_see_values_that_are_not_their_neighbours(hyg):
         assert bad[k]
         # neighbours lie within one lattice step in every local coordinate
         assert np.abs(xyz[bad] - xyz[k]).max() <= 2.0 * np.abs(xyz).max() / (1 << L) + 1e-12
+
+
+@pytest.mark.parametrize("dtype", ["F64", "F32"])
+@pytest.mark.parametrize("nmodes,L", [(0, 1), (1, 3), (8, 5), (9, 2), (32, 6), (33, 4), (64, 5)])
+def test_coefficient_integrals_of_every_variant(hyg, nmodes, L, dtype):
+    """The matrix product behind k, by the number of modes (padded to 8, 32 or 64) and the length of rows (16-anchor tiles
+    and their remainders, blocks of 16 and 32 rows)."""
+    dt = getattr(hyg, dtype)
+    name = "pyramid_tilted_4el.msh"
+    modes = ol.random_field(5, modes=nmodes, kmax=3) if nmodes else []
+    gm, om = hyg.Mesh(name), ol.Mesh(name)
+    n = gm.ndofs(L)
+    x0 = rnd(n, 40, dt == hyg.F32)
+    op = hyg.P1DivKGradOperator(gm, L, L, 1.3, modes)
+    oop = ol.DivKGradOperator(om, L, L, ("fourier", 1.3, modes if nmodes else np.zeros((0, 5))))
+    x, y = hyg.Function(gm, L, L, dt), hyg.Function(gm, L, L, dt)
+    ox, od = ol.Function(om, L, L), ol.Function(om, L, L)
+    x.upload(L, x0)
+    ox.set(L, x0)
+    print(nmodes, L, dtype, flush=True)
+    op.apply(x, y, L, hyg.ALL)
+    oop.apply(ox, od, L, ol.ALL, False)
+    # FP32: rounding of up to 2 * 64 terms of total size sqrt(2 * 64) * 0.5 in log k, 6e-6, and 34 roundings of the sum
+    assert rel_inf(y.download(L), od.get(L)) <= (1e-13 if dt == hyg.F64 else 2e-5)

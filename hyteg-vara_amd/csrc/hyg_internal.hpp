@@ -743,8 +743,8 @@ struct hyg_op_s
       double*               dinv    = nullptr;
       float*                dinvF   = nullptr;
       // P2: element matrices (6 types x 10 x 10 per cell) of the micro-cells of level lattice-1;
-      // variable coefficient: per cell and type the 11 quadrature-point matrices w_q |det J| grad phi grad phi^T
-      // (11 x 10 x 10) and per micro-cell the coefficient at its 11 quadrature points
+      // variable coefficient: per cell and type the ten products |det J| grad lambda_a . grad lambda_b and per micro-cell
+      // the ten moments of k against lambda_a lambda_b (p2_common.hpp)
       double*               p2el    = nullptr;
       float*                p2elF   = nullptr;
       double*               p2kq    = nullptr;

@@ -48,8 +48,9 @@ __device__ __forceinline__ double p2CoefAt( const P2Coef& k, double x, double y,
 }
 
 // One thread per anchor of the micro-cell lattice (level L-1) of a macro-cell; the valid types of that anchor.
-// Element id (6 c + t) S3(Nc + 1) + index(Nc + 1, anchor); kq[q kqStride + id], kqStride = 6 nC S3(Nc + 1), so that
-// threads of consecutive anchors read consecutive values of one quadrature point.
+// Element id (6 c + t) S3(Nc + 1) + index(Nc + 1, anchor); the moments of k (p2Mom), formed in FP64 from its values at the 11
+// quadrature points, are kq[q kqStride + id], kqStride = 6 nC S3(Nc + 1), so that threads of consecutive anchors read
+// consecutive values of one moment.
 template < typename T >
 __global__ __launch_bounds__( kBlock ) void kP2KQ( int L, int tilesPerCell, const ElemCell* __restrict__ cells, P2Coef coef,
                                                    T* __restrict__ kq, i64 kqStride )
@@ -77,19 +78,29 @@ __global__ __launch_bounds__( kBlock ) void kP2KQ( int L, int tilesPerCell, cons
             X[v][r] = ec.v0[r] + ec.a[r][0] * i + ec.a[r][1] * j + ec.a[r][2] * k;
       }
       const uint64_t eid = uint64_t( c * 6 + t ) * uint64_t( SA ) + uint64_t( s );
+      double         m[kP2Moments] = {};
+#pragma unroll
       for ( int q = 0; q < 11; ++q )
       {
          double x[3];
 #pragma unroll
          for ( int r = 0; r < 3; ++r )
             x[r] = kXG4Lambda[q][0] * X[0][r] + kXG4Lambda[q][1] * X[1][r] + kXG4Lambda[q][2] * X[2][r] + kXG4Lambda[q][3] * X[3][r];
-         kq[i64( q ) * kqStride + i64( eid )] = T( p2CoefAt( coef, x[0], x[1], x[2], eid ) );
+         const double k = kXG4Weight[q] * p2CoefAt( coef, x[0], x[1], x[2], eid );
+#pragma unroll
+         for ( int a = 0; a < 4; ++a )
+#pragma unroll
+            for ( int b = a; b < 4; ++b )
+               m[p2Mom( a, b )] += k * ( kXG4Lambda[q][a] * kXG4Lambda[q][b] );
       }
+#pragma unroll
+      for ( int q = 0; q < kP2Moments; ++q )
+         kq[i64( q ) * kqStride + i64( eid )] = T( m[q] );
    }
 }
 
 // ------------------------------------------------------------------ operator application
-// KQ: variable coefficient (el = 11 quadrature-point matrices per cell and type, kq per micro-cell)
+// KQ: variable coefficient (el = the ten G_ab of p2Row per cell and type, kq = the moments per micro-cell), diagonal only
 // points on the cell edges and vertices of a cell lattice with N intervals per edge: the four vertices, then
 // N - 1 points of each edge e0 = (v0, v1) ... e5 = (v2, v3)
 constexpr int kP2EvLanes = 4; // lanes per point of the edge/vertex kernel
@@ -156,7 +167,8 @@ __global__ __launch_bounds__( kBlock ) void kP2Apply( int L, int tilesPerCell, i
    if ( slot == 0 && ( SKIPIN || !( flag & 1 ) ) )
       return;
    const int cls = ( px & 1 ) | ( ( py & 1 ) << 1 ) | ( ( pz & 1 ) << 2 );
-   const T*  ec  = el + i64( c ) * ( KQ ? 6600 : 600 );
+   static_assert( !KQ || DIAG, "the variable coefficient is applied by kP2KQInt and kP2KEdge" );
+   const T*  ec  = el + i64( c ) * ( KQ ? 6 * kP2Moments : 600 );
    const int SA  = S3i( Nc + 1 );
    const T*  xc  = x + i64( c ) * stride;
    T         val = T( 0 );
@@ -171,30 +183,15 @@ __global__ __launch_bounds__( kBlock ) void kP2Apply( int L, int tilesPerCell, i
          continue;
       if constexpr ( KQ )
       {
-         const T* M  = ec + 1100 * t + 10 * l; // M[100 q + j]: row l of quadrature-point matrix q
          const T* kv = kq + i64( c * 6 + t ) * SA + cidx( Nc + 1, ax, ay, az );
-         T        kk[11];
+         T        m[kP2Moments], r[10];
 #pragma unroll
-         for ( int q = 0; q < 11; ++q )
-            kk[q] = kv[i64( q ) * kqStride];
-         if constexpr ( DIAG )
-         {
+         for ( int q = 0; q < kP2Moments; ++q )
+            m[q] = kv[i64( q ) * kqStride];
+         p2RowOf( l, m, ec + kP2Moments * t, r );
 #pragma unroll
-            for ( int q = 0; q < 11; ++q )
-               val += kk[q] * M[100 * q + l];
-         }
-         else
-         {
-#pragma unroll
-            for ( int j = 0; j < 10; ++j )
-            {
-               T r = T( 0 );
-#pragma unroll
-               for ( int q = 0; q < 11; ++q )
-                  r += kk[q] * M[100 * q + j];
-               val += r * xc[cidx( w, 2 * ax + tb->nd[t][j][0], 2 * ay + tb->nd[t][j][1], 2 * az + tb->nd[t][j][2] )];
-            }
-         }
+         for ( int j = 0; j < 10; ++j )
+            val += j == l ? r[j] : T( 0 );
       }
       else
       {
@@ -258,6 +255,109 @@ __global__ __launch_bounds__( kBlock ) void kP2Apply( int L, int tilesPerCell, i
    }
 }
 
+// Variable coefficient, points on the cell edges and vertices, up to three components at once: kP2EvLanes lanes per point
+// share its micro-cells, of any type and node, so the row product is written with run-time indices. With T_w[d] =
+// |det J| grad lambda_d . grad u at vertex w, vertex node a takes sum_w (4 kappa_aw - R_w) T_w[a] (R_w the row sums of kappa) and
+// edge node (a, b) takes 4 sum_w (kappa_aw T_w[b] + kappa_bw T_w[a]).
+template < typename T >
+__global__ __launch_bounds__( kBlock ) void kP2KEdge( int L, int tilesPerCell, i64 stride, const T* __restrict__ el, const T* __restrict__ kq,
+                                                      i64 kqStride, const P2Tables* __restrict__ tb, const CellInfo* __restrict__ cinfo,
+                                                      const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
+                                                      T* __restrict__ lowPart, i64 lowStride, int flag, P2Comps< T > cp, int nc )
+{
+   const int c    = int( blockIdx.x ) / tilesPerCell;
+   const int tile = int( blockIdx.x ) - c * tilesPerCell;
+   const int N = 1 << L, w = N + 1, NP = N + 1, Nc = N >> 1, SA = S3i( Nc + 1 );
+   const int s   = ( tile * kBlock + int( threadIdx.x ) ) / kP2EvLanes;
+   const int sub = int( threadIdx.x ) % kP2EvLanes;
+   int       px, py, pz;
+   // the lanes of one point leave together
+   if ( s >= p2EdgeVertexCount( N ) || !edgeVertexXYZ( N, s, px, py, pz ) )
+      return;
+   const int       slot = classifySlot( N, px, py, pz );
+   const CellInfo& ci   = cinfo[c];
+   if ( slot <= 4 || !( prims[ci.prim[slot]].bc & flag ) )
+      return;
+   const int cls    = ( px & 1 ) | ( ( py & 1 ) << 1 ) | ( ( pz & 1 ) << 2 );
+   const i64 cb     = i64( c ) * stride;
+   T         val[3] = { T( 0 ), T( 0 ), T( 0 ) };
+   const int ne     = tb->nEnt[cls];
+   for ( int k = sub; k < ne; k += kP2EvLanes )
+   {
+      const int tl = tb->ent[cls][k];
+      const int t = tl >> 4, l = tl & 15;
+      // anchor of the micro-cell of type t that has this point as node l
+      const int ax = ( px - tb->nd[t][l][0] ) >> 1, ay = ( py - tb->nd[t][l][1] ) >> 1, az = ( pz - tb->nd[t][l][2] ) >> 1;
+      if ( ax < 0 || ay < 0 || az < 0 || ax + ay + az + kMCMax[t] > Nc )
+         continue;
+      const T*  kv = kq + i64( c * 6 + t ) * SA + cidx( Nc + 1, ax, ay, az );
+      const T*  g  = el + ( c * 6 + t ) * kP2Moments;
+      const int na = l < 4 ? l : kP2EdgeNodes[l - 4][0], nb = l < 4 ? l : kP2EdgeNodes[l - 4][1];
+      T         m[kP2Moments], A[4], Bv[4], ga[4], gb[4];
+#pragma unroll
+      for ( int q = 0; q < kP2Moments; ++q )
+         m[q] = kv[i64( q ) * kqStride];
+#pragma unroll
+      for ( int v = 0; v < 4; ++v )
+      {
+         const T R  = ( m[p2Mom( v, 0 )] + m[p2Mom( v, 1 )] ) + ( m[p2Mom( v, 2 )] + m[p2Mom( v, 3 )] );
+         const T ka = kv[i64( p2Mom( na, v ) ) * kqStride], kb = kv[i64( p2Mom( nb, v ) ) * kqStride];
+         A[v]       = T( 4 ) * ka - ( l < 4 ? R : T( 0 ) );
+         Bv[v]      = l < 4 ? T( 0 ) : T( 4 ) * kb;
+         ga[v]      = g[p2Mom( na, v )];
+         gb[v]      = g[p2Mom( nb, v )];
+      }
+      int o[10];
+#pragma unroll
+      for ( int j = 0; j < 10; ++j )
+         o[j] = cidx( w, 2 * ax + tb->nd[t][j][0], 2 * ay + tb->nd[t][j][1], 2 * az + tb->nd[t][j][2] );
+#pragma unroll
+      for ( int q = 0; q < 3; ++q )
+      {
+         if ( q >= nc )
+            break;
+         const T* xc = cp.x[q] + cb;
+         T        u[10];
+#pragma unroll
+         for ( int j = 0; j < 10; ++j )
+            u[j] = xc[o[j]];
+#pragma unroll
+         for ( int v = 0; v < 4; ++v )
+         {
+            // grad u at vertex v = sum_b gam_b grad lambda_b
+            T ta = T( 0 ), tbv = T( 0 );
+#pragma unroll
+            for ( int b = 0; b < 4; ++b )
+            {
+               const T gam = b == v ? T( 3 ) * u[v] : fma( T( 4 ), u[p2EdgeNode( b, v )], -u[b] );
+               ta          = fma( ga[b], gam, ta );
+               tbv         = fma( gb[b], gam, tbv );
+            }
+            // a vertex node has ga = gb and Bv = 0; an edge node (a, b) takes kappa_a with T[b] and kappa_b with T[a]
+            val[q] = fma( A[v], tbv, fma( Bv[v], ta, val[q] ) );
+         }
+      }
+   }
+   const int e = ci.entry[slot];
+   int       i = 0;
+   if ( slot <= 10 )
+   {
+      const int b[4] = { N - px - py - pz, px, py, pz };
+      i              = b[entries[e].l1];
+   }
+#pragma unroll
+   for ( int q = 0; q < 3; ++q )
+   {
+      if ( q >= nc )
+         break;
+#pragma unroll
+      for ( int m = 1; m < kP2EvLanes; m <<= 1 )
+         val[q] += __shfl_xor( val[q], m, kP2EvLanes );
+      if ( sub == 0 )
+         lowPart[i64( q ) * lowStride + i64( e ) * NP + i] = val[q];
+   }
+}
+
 // ------------------------------------------------------------------ constant operator: cell-face points
 // Points inside a cell face (not on a cell edge) take the one-sided merged stencil of their face and parity
 // class; the sum goes to the face's partial-sum block like the element kernel's. On each face the points split
@@ -266,10 +366,10 @@ __global__ __launch_bounds__( kBlock ) void kP2Apply( int L, int tilesPerCell, i
 // point of (u, v) is (u, v, 0), (u, 0, v), (0, u, v) and (u, N - u - v, v) on faces 0..3: consecutive threads (u)
 // stay in one z-plane, on the diagonal face too.
 
-// Stored stencils of the variable-coefficient operator: per cell, the merged stencils of the cell-interior
-// points class by class ([e][point of the class sub-lattice], the class-kappa points p = 2 q + kappa of the cell
-// form a tetrahedral lattice of width (N - |kappa|) / 2 + 1), then the one-sided stencils of the cell-face points
-// face by face and sub-lattice by sub-lattice ([e][face sub-lattice index]).
+// Stored stencils of the variable-coefficient operator: per cell, class by class, the stencils of all points of the class
+// sub-lattice ([e][point], the class-kappa points p = 2 q + kappa of the cell form a tetrahedral lattice of width
+// (N - |kappa|) / 2 + 1); those of cell-face points are one-sided (0 for nodes outside the cell), cell edges and vertices
+// have none.
 __host__ __device__ constexpr int p2SubWidth( int N, int cls )
 {
    return ( N - ( cls & 1 ) - ( ( cls >> 1 ) & 1 ) - ( ( cls >> 2 ) & 1 ) ) / 2 + 1;
@@ -283,27 +383,12 @@ __host__ __device__ inline i64 p2StoredIntBase( int N, int cls )
       b += i64( n[k] ) * S3i( p2SubWidth( N, k ) );
    return b;
 }
-__host__ __device__ inline i64 p2StoredFaceBase( int N, int F, int sub )
-{
-   constexpr int nf[4][4] = { { p2StencilOffsets( p2FaceClass( 0, 0, 0 ), 0 ).n, p2StencilOffsets( p2FaceClass( 0, 1, 0 ), 0 ).n,
-                                p2StencilOffsets( p2FaceClass( 0, 0, 1 ), 0 ).n, p2StencilOffsets( p2FaceClass( 0, 1, 1 ), 0 ).n },
-                              { p2StencilOffsets( p2FaceClass( 1, 0, 0 ), 1 ).n, p2StencilOffsets( p2FaceClass( 1, 1, 0 ), 1 ).n,
-                                p2StencilOffsets( p2FaceClass( 1, 0, 1 ), 1 ).n, p2StencilOffsets( p2FaceClass( 1, 1, 1 ), 1 ).n },
-                              { p2StencilOffsets( p2FaceClass( 2, 0, 0 ), 2 ).n, p2StencilOffsets( p2FaceClass( 2, 1, 0 ), 2 ).n,
-                                p2StencilOffsets( p2FaceClass( 2, 0, 1 ), 2 ).n, p2StencilOffsets( p2FaceClass( 2, 1, 1 ), 2 ).n },
-                              { p2StencilOffsets( p2FaceClass( 3, 0, 0 ), 3 ).n, p2StencilOffsets( p2FaceClass( 3, 1, 0 ), 3 ).n,
-                                p2StencilOffsets( p2FaceClass( 3, 0, 1 ), 3 ).n, p2StencilOffsets( p2FaceClass( 3, 1, 1 ), 3 ).n } };
-   i64 b = p2StoredIntBase( N, 8 );
-   for ( int k = 0; k < 4 * F + sub; ++k )
-      b += i64( nf[k >> 2][k & 3] ) * p2FaceSubCount( N, k & 1, ( k >> 1 ) & 1 );
-   return b;
-}
 __host__ __device__ inline i64 p2StoredCellSize( int N )
 {
-   return ( p2StoredFaceBase( N, 4, 0 ) + 63 ) / 64 * 64;
+   return ( p2StoredIntBase( N, 8 ) + 63 ) / 64 * 64;
 }
 
-template < typename T, int F, int KU, int KV, bool STORED >
+template < typename T, int F, int KU, int KV >
 __device__ __forceinline__ void p2FacePoint( int c, int s, int N, i64 stride, const T* __restrict__ fst, const CellFaceSlot& fs,
                                              T* __restrict__ part, const T* __restrict__ x )
 {
@@ -319,10 +404,7 @@ __device__ __forceinline__ void p2FacePoint( int c, int s, int N, i64 stride, co
    const int px = F == 2 ? 0 : u, py = F == 0 ? v : ( F == 2 ? u : ( F == 3 ? N - u - v : 0 ) ), pz = F == 0 ? 0 : v;
    const int w = N + 1;
    typedef const T __attribute__( ( address_space( 4 ) ) ) CT;
-   // uniform weights of the cell (constant coefficient), or this point's stored stencil
-   const CT* wc = (const CT*) ( fst + ( i64( c * 4 + F ) * 8 + CLS ) * kP2StencilMax );
-   const T*  ws = fst + i64( c ) * p2StoredCellSize( N ) + p2StoredFaceBase( N, F, KU | ( KV << 1 ) ) + s;
-   const int cnt = triCount( M + 1 );
+   const CT* wc = (const CT*) ( fst + ( i64( c * 4 + F ) * 8 + CLS ) * kP2StencilMax ); // uniform weights of the cell
    const T*  xc  = x + i64( c ) * stride;
    int       rb[5][5];
 #pragma unroll
@@ -337,21 +419,17 @@ __device__ __forceinline__ void p2FacePoint( int c, int s, int N, i64 stride, co
    T val = T( 0 );
 #pragma unroll
    for ( int e = 0; e < off.n; ++e )
-      val += ( STORED ? ws[i64( e ) * cnt] : wc[e] ) * xc[rb[off.d[e][2] + 2][off.d[e][1] + 2] + px + off.d[e][0]];
+      val += wc[e] * xc[rb[off.d[e][2] + 2][off.d[e][1] + 2] + px + off.d[e][0]];
    part[i64( fs.block ) * w * w + facePartIndex( F, N, px, py, pz )] = val;
 }
 
-template < typename T, bool STORED >
+template < typename T >
 __global__ __launch_bounds__( kBlock ) void kP2Face( int L, i64 stride, P2FaceTiles ft, const T* __restrict__ fst,
                                                      const CellFaceSlot* __restrict__ cfs, int flag, T* __restrict__ part,
-                                                     const T* __restrict__ x, int nC )
+                                                     const T* __restrict__ x )
 {
    const int per = ft.start[4];
-   // nC > 0: each XCD takes a contiguous range of cells (grid padded to a multiple of 8), keeping a cell's data in one
-   // L2 (pays off for the stored stencils of many cells; the constant operator's launch keeps the plain order)
-   const int b = nC > 0 ? remapXcd( int( blockIdx.x ), nC * 4 * per ) : int( blockIdx.x );
-   if ( nC > 0 && b >= nC * 4 * per )
-      return;
+   const int b   = int( blockIdx.x );
    const int c = b / ( 4 * per );
    int       r = b - c * 4 * per;
    const int f   = r / per;
@@ -365,7 +443,7 @@ __global__ __launch_bounds__( kBlock ) void kP2Face( int L, i64 stride, P2FaceTi
       return;
    const int N = 1 << L;
 #define HYG_P2_FACE( F, SUB )                                                                                         \
-   case 4 * F + SUB: p2FacePoint< T, F, ( SUB & 1 ), ( SUB >> 1 ), STORED >( c, s, N, stride, fst, fs, part, x ); break;
+   case 4 * F + SUB: p2FacePoint< T, F, ( SUB & 1 ), ( SUB >> 1 ) >( c, s, N, stride, fst, fs, part, x ); break;
    switch ( 4 * f + sub )
    {
       HYG_P2_FACE( 0, 0 )
@@ -383,7 +461,7 @@ __global__ __launch_bounds__( kBlock ) void kP2Face( int L, i64 stride, P2FaceTi
       HYG_P2_FACE( 3, 0 )
       HYG_P2_FACE( 3, 1 )
       HYG_P2_FACE( 3, 2 )
-   default: p2FacePoint< T, 3, 1, 1, STORED >( c, s, N, stride, fst, fs, part, x ); break;
+   default: p2FacePoint< T, 3, 1, 1 >( c, s, N, stride, fst, fs, part, x ); break;
    }
 #undef HYG_P2_FACE
 }
@@ -747,49 +825,54 @@ __global__ __launch_bounds__( kBlock ) void kP2RestrictInt( int Lc, i64 strideC,
    p2RestrictDispatch< T, 0 >( cls, c, ( t - ct.start[cls] ) * kBlock + int( threadIdx.x ), 1 << Lc, strideC, strideF, coarse, fine );
 }
 
-// Stored stencils, cell-interior points one class per wave (the class sub-lattice, p2InteriorExtent): each
-// thread gathers its point's neighbours and reads its own weights ([e][sub-lattice point], consecutive threads
-// read consecutive weights), then the mode's epilogue; the inverse diagonal is the inverse centre weight.
-
+// Stored stencils, the points of a cell that are not on its edges, one class per block (the class sub-lattice): each thread
+// gathers its point's neighbours and reads its own weights (consecutive threads consecutive weights), each weight once for
+// all components; then the mode's epilogue (the inverse diagonal is the inverse centre weight), or the one-sided sum of
+// a face point. Face points in kernels of their own, one component at a time, took longer than all interior points (FP32,
+// three components, shell at P2 level 4: 339 against 282 us; together now 538 us).
 template < typename T, int MODE, int CLS, int NC >
-__device__ __forceinline__ void p2StoredIntPt( int c, int s, int N, i64 stride, const T* __restrict__ sw, const P2Comps< T >& cp, T a )
+__device__ __forceinline__ void p2StoredIntPt( int c, int s, int N, i64 stride, const T* __restrict__ sw, const P2Comps< T >& cp, T a,
+                                               const CellFaceSlot* __restrict__ cfs, int flag, T* __restrict__ part, i64 partStride )
 {
    constexpr int              kx = CLS & 1, ky = ( CLS >> 1 ) & 1, kz = ( CLS >> 2 ) & 1;
    constexpr P2StencilOffsets off = p2StencilOffsets( CLS );
-   const int                  M   = p2InteriorExtent( N, CLS );
-   if ( M < 0 || s >= S3i( M + 1 ) )
+   const int                  M   = p2ClassExtent( N, CLS ), nS = S3i( M + 1 );
+   if ( s >= nS )
       return;
    int qx, qy, qz;
    tetXYZ( M + 1, s, qx, qy, qz );
-   const int px = 2 * ( qx + 1 - kx ) + kx, py = 2 * ( qy + 1 - ky ) + ky, pz = 2 * ( qz + 1 - kz ) + kz;
-   const int w = N + 1, SW = p2SubWidth( N, CLS ), nS = S3i( SW );
-   const T*  ws = sw + i64( c ) * p2StoredCellSize( N ) + p2StoredIntBase( N, CLS ) + cidx( SW, px >> 1, py >> 1, pz >> 1 );
-   int       rb[5][5];
-#pragma unroll
-   for ( int dz = -2; dz <= 2; ++dz )
-   {
-      const int W  = w - ( pz + dz );
-      const int pb = S3i( w ) - S3i( W );
-#pragma unroll
-      for ( int dy = -2; dy <= 2; ++dy )
-         rb[dz + 2][dy + 2] = pb + rowStart( W, py + dy );
-   }
-   // each weight is read once and applied to every component
-   T val[NC];
+   const int px = 2 * qx + kx, py = 2 * qy + ky, pz = 2 * qz + kz;
+   int       slot;
+   i64       pi;
+   if ( !p2PointWanted( c, N, px, py, pz, cfs, flag, slot, pi ) )
+      return;
+   const T* ws = sw + i64( c ) * p2StoredCellSize( N ) + p2StoredIntBase( N, CLS ) + s;
+   int      rb[5][5];
+   p2RowStarts( N, px, py, pz, rb );
+   const P2Inside in( N, px, py, pz );
+   const i64      cb = i64( c ) * stride, q = cb + rb[2][2];
+   T              val[NC];
 #pragma unroll
    for ( int k = 0; k < NC; ++k )
       val[k] = T( 0 );
 #pragma unroll
    for ( int e = 0; e < off.n; ++e )
    {
-      const T   wt = ws[i64( e ) * nS];
-      const i64 o  = i64( c ) * stride + rb[off.d[e][2] + 2][off.d[e][1] + 2] + px + off.d[e][0];
+      const T wt = ws[i64( e ) * nS];
+      // a node outside the cell has no weight: the point reads itself instead
+      const int o = in.has( off.d[e][0], off.d[e][1], off.d[e][2] ) ? rb[off.d[e][2] + 2][off.d[e][1] + 2] + off.d[e][0] : rb[2][2];
 #pragma unroll
       for ( int k = 0; k < NC; ++k )
-         val[k] += wt * cp.x[k][o];
+         val[k] += wt * ( cp.x[k] + cb )[unsigned( o )];
    }
-   const i64 q  = i64( c ) * stride + rb[2][2] + px;
-   T         dv = T( 1 );
+   if ( slot > 0 )
+   {
+#pragma unroll
+      for ( int k = 0; k < NC; ++k )
+         part[i64( k ) * partStride + pi] = val[k];
+      return;
+   }
+   T dv = T( 1 );
    if constexpr ( MODE == MODE_JACOBI || MODE == MODE_CHEB0 || MODE == MODE_CHEBK )
       dv = T( 1 ) / ws[i64( p2CentreIndex( off ) ) * nS];
 #pragma unroll
@@ -809,16 +892,18 @@ __device__ __forceinline__ void p2StoredIntPt( int c, int s, int N, i64 stride, 
    }
 }
 template < typename T, int MODE, int CLS, int NC >
-__device__ __forceinline__ void p2StoredIntDispatch( int cls, int c, int s, int N, i64 stride, const T* sw, const P2Comps< T >& cp, T a )
+__device__ __forceinline__ void p2StoredIntDispatch( int cls, int c, int s, int N, i64 stride, const T* sw, const P2Comps< T >& cp, T a,
+                                                     const CellFaceSlot* cfs, int flag, T* part, i64 partStride )
 {
    if ( cls == CLS )
-      p2StoredIntPt< T, MODE, CLS, NC >( c, s, N, stride, sw, cp, a );
+      p2StoredIntPt< T, MODE, CLS, NC >( c, s, N, stride, sw, cp, a, cfs, flag, part, partStride );
    else if constexpr ( CLS < 7 )
-      p2StoredIntDispatch< T, MODE, CLS + 1, NC >( cls, c, s, N, stride, sw, cp, a );
+      p2StoredIntDispatch< T, MODE, CLS + 1, NC >( cls, c, s, N, stride, sw, cp, a, cfs, flag, part, partStride );
 }
 template < typename T, int MODE, int NC >
 __global__ __launch_bounds__( kBlock ) void kP2StoredInt( int L, i64 stride, P2ClassTiles ct, const T* __restrict__ sw, P2Comps< T > cp,
-                                                          T a, int nC )
+                                                          T a, const CellFaceSlot* __restrict__ cfs, int flag, T* __restrict__ part,
+                                                          i64 partStride, int nC )
 {
    const int per = ct.start[8];
    // each XCD takes a contiguous range of cells (grid padded to a multiple of 8), keeping a cell's source in one L2
@@ -830,140 +915,79 @@ __global__ __launch_bounds__( kBlock ) void kP2StoredInt( int L, i64 stride, P2C
    int       cls = 0;
    while ( cls < 7 && t >= ct.start[cls + 1] )
       ++cls;
-   p2StoredIntDispatch< T, MODE, 0, NC >( cls, c, ( t - ct.start[cls] ) * kBlock + int( threadIdx.x ), 1 << L, stride, sw, cp, a );
+   p2StoredIntDispatch< T, MODE, 0, NC >( cls, c, ( t - ct.start[cls] ) * kBlock + int( threadIdx.x ), 1 << L, stride, sw, cp, a, cfs,
+                                         flag, part, partStride );
 }
 
 // ------------------------------------------------------------------ stored stencils (variable coefficient)
-// Setup: the stencil of a point is the sum, over the micro-cells that have it as node l (on the cell's side of
-// face F for a face point), of row l of sum_q k_q M_{t,q}, keyed by the offset to the other node.
-// Stores the stencil of a point (p2StencilOffsets(CLS, F), entry e at out[e estride]): the sum, over the micro-cells
-// that have the point as node l, of row l of sum_q k_q M_{t,q} (rows staged in LDS by p2StageRows), accumulated in
-// place in the point's own output slots (one micro-cell per loop iteration, in the same order as the on-the-fly
-// assembly), so no per-point stencil array is held.
-template < int CLS, int F >
+// Setup: stores the stencil of a point (p2StencilOffsets(CLS), entry e at out[e estride]): the sum, over the micro-cells inside
+// the cell that have the point as node l, of row l of their element matrices (p2Row), accumulated in place in the point's own
+// output slots (one micro-cell per loop iteration, in the same order as the on-the-fly assembly), so no per-point stencil
+// array is held.
+template < int CLS >
 __device__ __forceinline__ void p2StorePoint( int c, int N, int px, int py, int pz, const double* __restrict__ kq, i64 kqStride,
-                                              double* __restrict__ out, i64 estride, const double* __restrict__ Ms )
+                                              double* __restrict__ out, i64 estride, const double* __restrict__ el )
 {
-   constexpr P2StencilOffsets off = p2StencilOffsets( CLS, F );
+   constexpr P2StencilOffsets off = p2StencilOffsets( CLS );
 #pragma unroll
    for ( int e = 0; e < off.n; ++e )
       out[i64( e ) * estride] = 0.0;
    const int          Nc = N >> 1, SA = S3i( Nc + 1 );
-   const P2KQEntries& E  = kP2KQTab.c[CLS][F + 1];
+   const P2KQEntries& E  = kP2KQTab.c[CLS];
 #pragma unroll 1
    for ( int k = 0; k < E.n; ++k )
    {
       const P2KQEntry& e  = E.e[k];
       const int        ax = ( px - e.nd[0] ) >> 1, ay = ( py - e.nd[1] ) >> 1, az = ( pz - e.nd[2] ) >> 1;
-      const double*    kv = kq + i64( c * 6 + e.t ) * SA + cidx( Nc + 1, ax, ay, az );
-      double           kk[11];
+      if ( ax < 0 || ay < 0 || az < 0 || ax + ay + az + e.mcmax > Nc )
+         continue;
+      const double* kv = kq + i64( c * 6 + e.t ) * SA + cidx( Nc + 1, ax, ay, az );
+      double        m[kP2Moments], r[10];
 #pragma unroll
-      for ( int q = 0; q < 11; ++q )
-         kk[q] = kv[i64( q ) * kqStride];
+      for ( int q = 0; q < kP2Moments; ++q )
+         m[q] = kv[i64( q ) * kqStride];
+      p2RowOf( e.l, m, el + ( c * 6 + e.t ) * kP2Moments, r );
 #pragma unroll
       for ( int jj = 0; jj < 10; ++jj )
-      {
-         const double* row = Ms + ( e.ord * 10 + jj ) * kP2RowPad;
-         double        r   = 0.0;
-#pragma unroll
-         for ( int q = 0; q < 11; ++q )
-            r += kk[q] * row[q];
-         out[i64( e.slot[jj] ) * estride] += r;
-      }
+         out[i64( e.slot[jj] ) * estride] += r[jj];
    }
 }
 template < int CLS >
 __device__ __forceinline__ void p2StoreIntPt( int c, int s, int N, const double* __restrict__ el, const double* __restrict__ kq,
-                                              i64 kqStride, double* __restrict__ sw, double* __restrict__ Ms )
+                                              i64 kqStride, double* __restrict__ sw )
 {
    constexpr int kx = CLS & 1, ky = ( CLS >> 1 ) & 1, kz = ( CLS >> 2 ) & 1;
-   p2StageRows< double, CLS >( el, c, Ms );
-   const int M = p2InteriorExtent( N, CLS );
-   if ( M < 0 || s >= S3i( M + 1 ) )
+   const int M = p2ClassExtent( N, CLS );
+   if ( s >= S3i( M + 1 ) )
       return;
    int qx, qy, qz;
    tetXYZ( M + 1, s, qx, qy, qz );
-   // lattice point and its position (p - CLS) / 2 in the class sub-lattice
-   const int px = 2 * ( qx + 1 - kx ) + kx, py = 2 * ( qy + 1 - ky ) + ky, pz = 2 * ( qz + 1 - kz ) + kz;
-   const int SW = p2SubWidth( N, CLS );
-   double*   o  = sw + i64( c ) * p2StoredCellSize( N ) + p2StoredIntBase( N, CLS ) + cidx( SW, px >> 1, py >> 1, pz >> 1 );
-   p2StorePoint< CLS, -1 >( c, N, px, py, pz, kq, kqStride, o, S3i( SW ), Ms );
+   const int px = 2 * qx + kx, py = 2 * qy + ky, pz = 2 * qz + kz;
+   if ( classifySlot( N, px, py, pz ) > 4 )
+      return;
+   double* o = sw + i64( c ) * p2StoredCellSize( N ) + p2StoredIntBase( N, CLS ) + s;
+   p2StorePoint< CLS >( c, N, px, py, pz, kq, kqStride, o, S3i( M + 1 ), el );
 }
 template < int CLS >
 __device__ __forceinline__ void p2StoreIntDispatch( int cls, int c, int s, int N, const double* el, const double* kq, i64 kqStride,
-                                                    double* sw, double* Ms )
+                                                    double* sw )
 {
    if ( cls == CLS )
-      p2StoreIntPt< CLS >( c, s, N, el, kq, kqStride, sw, Ms );
+      p2StoreIntPt< CLS >( c, s, N, el, kq, kqStride, sw );
    else if constexpr ( CLS < 7 )
-      p2StoreIntDispatch< CLS + 1 >( cls, c, s, N, el, kq, kqStride, sw, Ms );
+      p2StoreIntDispatch< CLS + 1 >( cls, c, s, N, el, kq, kqStride, sw );
 }
 __global__ __launch_bounds__( kBlock ) void kP2StoreInt( int L, P2ClassTiles ct, const double* __restrict__ el,
                                                          const double* __restrict__ kq, i64 kqStride, double* __restrict__ sw )
 {
-   __shared__ double Ms[kP2MaxPairs * 10 * kP2RowPad];
-   const int         per = ct.start[8];
-   const int         c   = int( blockIdx.x ) / per;
-   const int         t   = int( blockIdx.x ) - c * per;
-   int               cls = 0;
+   const int per = ct.start[8];
+   const int c   = int( blockIdx.x ) / per;
+   const int t   = int( blockIdx.x ) - c * per;
+   int       cls = 0;
    while ( cls < 7 && t >= ct.start[cls + 1] )
       ++cls;
-   p2StoreIntDispatch< 0 >( cls, c, ( t - ct.start[cls] ) * kBlock + int( threadIdx.x ), 1 << L, el, kq, kqStride, sw, Ms );
+   p2StoreIntDispatch< 0 >( cls, c, ( t - ct.start[cls] ) * kBlock + int( threadIdx.x ), 1 << L, el, kq, kqStride, sw );
 }
-template < int F, int KU, int KV >
-__device__ __forceinline__ void p2StoreFacePt( int c, int s, int N, const double* __restrict__ el, const double* __restrict__ kq,
-                                               i64 kqStride, double* __restrict__ sw, double* __restrict__ Ms )
-{
-   p2StageRows< double, p2FaceClass( F, KU, KV ) >( el, c, Ms );
-   const int M = ( N - 5 + KU + KV ) / 2;
-   if ( s >= triCount( M + 1 ) )
-      return;
-   int i, j;
-   planeXY( M + 1, s, i, j );
-   const int u = 2 * i + 2 - KU, v = 2 * j + 2 - KV;
-   const int px = F == 2 ? 0 : u, py = F == 0 ? v : ( F == 2 ? u : ( F == 3 ? N - u - v : 0 ) ), pz = F == 0 ? 0 : v;
-   double*   o  = sw + i64( c ) * p2StoredCellSize( N ) + p2StoredFaceBase( N, F, KU | ( KV << 1 ) ) + s;
-   p2StorePoint< p2FaceClass( F, KU, KV ), F >( c, N, px, py, pz, kq, kqStride, o, triCount( M + 1 ), Ms );
-}
-__global__ __launch_bounds__( kBlock ) void kP2StoreFace( int L, P2FaceTiles ft, const double* __restrict__ el,
-                                                          const double* __restrict__ kq, i64 kqStride, double* __restrict__ sw )
-{
-   const int per = ft.start[4];
-   const int c   = int( blockIdx.x ) / ( 4 * per );
-   int       r   = int( blockIdx.x ) - c * 4 * per;
-   const int f   = r / per;
-   r -= f * per;
-   int sub = 0;
-   while ( sub < 3 && r >= ft.start[sub + 1] )
-      ++sub;
-   const int s = ( r - ft.start[sub] ) * kBlock + int( threadIdx.x );
-   const int N = 1 << L;
-   __shared__ double Ms[kP2MaxPairs * 10 * kP2RowPad];
-#define HYG_P2_STORE_FACE( F, SUB ) \
-   case 4 * F + SUB: p2StoreFacePt< F, ( SUB & 1 ), ( SUB >> 1 ) >( c, s, N, el, kq, kqStride, sw, Ms ); break;
-   switch ( 4 * f + sub )
-   {
-      HYG_P2_STORE_FACE( 0, 0 )
-      HYG_P2_STORE_FACE( 0, 1 )
-      HYG_P2_STORE_FACE( 0, 2 )
-      HYG_P2_STORE_FACE( 0, 3 )
-      HYG_P2_STORE_FACE( 1, 0 )
-      HYG_P2_STORE_FACE( 1, 1 )
-      HYG_P2_STORE_FACE( 1, 2 )
-      HYG_P2_STORE_FACE( 1, 3 )
-      HYG_P2_STORE_FACE( 2, 0 )
-      HYG_P2_STORE_FACE( 2, 1 )
-      HYG_P2_STORE_FACE( 2, 2 )
-      HYG_P2_STORE_FACE( 2, 3 )
-      HYG_P2_STORE_FACE( 3, 0 )
-      HYG_P2_STORE_FACE( 3, 1 )
-      HYG_P2_STORE_FACE( 3, 2 )
-   default: p2StoreFacePt< 3, 1, 1 >( c, s, N, el, kq, kqStride, sw, Ms ); break;
-   }
-#undef HYG_P2_STORE_FACE
-}
-
-
 // ------------------------------------------------------------------ prolongation
 // Value at point p (fine lattice, N = 2^Lf) of the quadratic interpolant of the coarse function cs
 // (lattice Lf-1, w = Nf/2 + 1) on a micro-cell of level Lf-2 of the macro-cell containing p.
@@ -1101,24 +1125,53 @@ static i64 p2KqStride( const MeshCtx& m, int L ) { return i64( m.mesh->nC() ) * 
 static i64 p2PartStride( const MeshCtx& m, int L ) { return i64( m.mesh->nF() ) * 2 * i64( ( 1 << L ) + 1 ) * ( ( 1 << L ) + 1 ); }
 static i64 p2LowStride( const MeshCtx& m, int L ) { return i64( m.entriesHost.size() ) * ( ( 1 << L ) + 1 ); }
 
+// Face, edge and vertex points of up to three components (one per grid row) from their partial sums, one launch
 template < typename T, int MODE >
-static void p2Combines( const MeshCtx& m, const LevelGeom& g, int L, const StencilCall& c, T* part, T* low, const T* dv, hipStream_t s )
+__global__ __launch_bounds__( kBlock ) void kP2Combine( int gF, const LowerChunk* __restrict__ chunks, int nLow, int nFace,
+                                                        const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
+                                                        int firstFacePrim, const T* __restrict__ part, i64 partStride,
+                                                        const T* __restrict__ low, i64 lowStride, const T* __restrict__ dinv, int L, i64 stride,
+                                                        int flag, P2Comps< T > cp, T a )
+{
+   const int k = int( blockIdx.y ), b = int( blockIdx.x );
+   const T*  x    = k == 0 ? cp.x[0] : ( k == 1 ? cp.x[1] : cp.x[2] );
+   const T*  in1  = k == 0 ? cp.in1[0] : ( k == 1 ? cp.in1[1] : cp.in1[2] );
+   T*        out0 = k == 0 ? cp.out0[0] : ( k == 1 ? cp.out0[1] : cp.out0[2] );
+   T*        out1 = k == 0 ? cp.out1[0] : ( k == 1 ? cp.out1[1] : cp.out1[2] );
+   if ( b < gF )
+      bFaceCombine< T, MODE >( b, chunks + nLow, nFace, prims, entries, firstFacePrim, part + i64( k ) * partStride, (const T*) nullptr, dinv, L,
+                               stride, flag, x, in1, out0, out1, a );
+   else
+      bLowCombine< T, MODE >( b - gF, chunks, nLow, prims, entries, low + i64( k ) * lowStride, dinv, L, stride, flag, x, in1, out0, out1, a );
+}
+template < typename T >
+static P2Comps< T > p2Comps( const StencilCall* cs, int n )
+{
+   P2Comps< T > cp{};
+   for ( int k = 0; k < n; ++k )
+   {
+      cp.x[k]    = (const T*) cs[k].x;
+      cp.in1[k]  = (const T*) cs[k].in1;
+      cp.out0[k] = (T*) cs[k].out0;
+      cp.out1[k] = (T*) cs[k].out1;
+   }
+   return cp;
+}
+template < typename T, int MODE >
+static void p2Combines( const MeshCtx& m, const LevelGeom& g, int L, const StencilCall* cs, int n, const T* part, const T* low, const T* dv,
+                        hipStream_t s )
 {
    const int nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
-   if ( nFace > 0 )
-      hipLaunchKernelGGL( ( kFaceCombine< T, MODE > ), dim3( xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) ), dim3( kBlock ), 0, s,
-                          g.chunks + g.firstFaceChunk, nFace, m.prims, m.entries, m.mesh->nV() + m.mesh->nE(), part,
-                          (const T*) nullptr, dv, L, g.stride, c.flag, (const T*) c.x, (const T*) c.in1, (T*) c.out0,
-                          (T*) c.out1, T( c.a ) );
-   if ( nLow > 0 )
-      hipLaunchKernelGGL( ( kLowCombine< T, MODE > ), dim3( ceilDiv( nLow, kBlock / 64 ) ), dim3( kBlock ), 0, s, g.chunks, nLow,
-                          m.prims, m.entries, low, dv, L, g.stride, c.flag, (const T*) c.x, (const T*) c.in1, (T*) c.out0,
-                          (T*) c.out1, T( c.a ) );
+   const int gF   = nFace > 0 ? xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) : 0;
+   hipLaunchKernelGGL( ( kP2Combine< T, MODE > ), dim3( gF + ceilDiv( nLow, kBlock / 64 ), n ), dim3( kBlock ), 0, s, gF, g.chunks, nLow, nFace,
+                       m.prims, m.entries, m.mesh->nV() + m.mesh->nE(), part, p2PartStride( m, L ), low, p2LowStride( m, L ), dv, L, g.stride,
+                       cs[0].flag, p2Comps< T >( cs, n ), T( cs[0].a ) );
 }
 
-// variable coefficient assembled on the fly for n = 1 or 3 components (one assembly per point for all of them)
+// variable coefficient for n <= 3 components at once (n = 1 or 3 without stored stencils): each point's stencil is assembled, or
+// its stored weights are read, once for all of them
 template < typename T, int MODE >
-static void p2KQOnTheFly( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, const StencilCall* cs, int n, hipStream_t s )
+static void p2Variable( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, const StencilCall* cs, int n, hipStream_t s )
 {
    constexpr bool         dbl  = std::is_same< T, double >::value;
    const hyg_op_s::Level& ol   = op.levels[L];
@@ -1130,38 +1183,31 @@ static void p2KQOnTheFly( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, in
    const T*               dv   = dbl ? (const T*) ol.dinv : (const T*) ol.dinvF;
    const i64              kqs = p2KqStride( m, L ), ps = p2PartStride( m, L ), ls = p2LowStride( m, L );
    const int              flag = cs[0].flag;
-   P2Comps< T >           cp{};
-   for ( int k = 0; k < n; ++k )
+   const P2Comps< T >     cp   = p2Comps< T >( cs, n );
+   if ( ol.p2s )
    {
-      cp.x[k]    = (const T*) cs[k].x;
-      cp.in1[k]  = (const T*) cs[k].in1;
-      cp.out0[k] = (T*) cs[k].out0;
-      cp.out1[k] = (T*) cs[k].out1;
+      // stored stencils
+      const T*           sw = dbl ? (const T*) ol.p2s : (const T*) ol.p2sF;
+      const P2ClassTiles ct = p2ClassTiles( N );
+      auto               kf = n == 3 ? kP2StoredInt< T, MODE, 3 > : ( n == 2 ? kP2StoredInt< T, MODE, 2 > : kP2StoredInt< T, MODE, 1 > );
+      hipLaunchKernelGGL( kf, dim3( xcdGrid( nC * ct.start[8] ) ), dim3( kBlock ), 0, s, L, g.stride, ct, sw, cp, T( cs[0].a ), m.cellFaces, flag,
+                          part, ps, nC );
    }
-   launchP2KQPoints< T >( L, nC, g.stride, el, kq, kqs, dv, cp, n, MODE, T( cs[0].a ), m.cellFaces, flag, part, ps, s );
+   else
+      launchP2KQPoints< T >( L, nC, g.stride, el, kq, kqs, dv, cp, n, MODE, T( cs[0].a ), m.cellFaces, flag, part, ps, s );
    const int tB = ceilDiv( i64( p2EdgeVertexCount( N ) ) * kP2EvLanes, kBlock );
-   for ( int k = 0; k < n; ++k )
-   {
-      const StencilCall& c = cs[k];
-      hipLaunchKernelGGL( ( kP2Apply< T, MODE, false, true, true > ), dim3( nC * tB ), dim3( kBlock ), 0, s, L, tB, g.stride, el, kq, kqs,
-                          m.p2tab, m.cellInfo, m.cellFaces, m.prims, m.entries, part + k * ps, low + k * ls, dv, c.flag,
-                          (const T*) c.x, (const T*) c.in1, (T*) c.out0, (T*) c.out1, T( c.a ) );
-   }
-   for ( int k = 0; k < n; ++k )
-      p2Combines< T, MODE >( m, g, L, cs[k], part + k * ps, low + k * ls, dv, s );
+   hipLaunchKernelGGL( ( kP2KEdge< T > ), dim3( nC * tB ), dim3( kBlock ), 0, s, L, tB, g.stride, el, kq, kqs, m.p2tab, m.cellInfo, m.prims,
+                       m.entries, low, ls, flag, cp, n );
+   p2Combines< T, MODE >( m, g, L, cs, n, part, low, dv, s );
 }
 
 template < typename T, int MODE, bool DIAG, bool KQ >
-static void p2TK( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, const StencilCall& c, hipStream_t s,
-                  bool skipInterior = false )
+static void p2TK( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, const StencilCall& c, hipStream_t s )
 {
    if constexpr ( KQ && !DIAG )
    {
-      if ( !op.levels[L].p2s )
-      {
-         p2KQOnTheFly< T, MODE >( m, g, op, L, &c, 1, s );
-         return;
-      }
+      p2Variable< T, MODE >( m, g, op, L, &c, 1, s );
+      return;
    }
    constexpr bool         dbl  = std::is_same< T, double >::value;
    const hyg_op_s::Level& ol   = op.levels[L];
@@ -1197,41 +1243,18 @@ static void p2TK( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, con
          ft.start[k + 1] = ft.start[k] + ceilDiv( p2FaceSubCount( 1 << L, k & 1, k >> 1 ), kBlock );
       const T* fsw = dbl ? (const T*) ol.p2fst : (const T*) ol.p2fstF;
       if ( ft.start[4] > 0 )
-         hipLaunchKernelGGL( ( kP2Face< T, false > ), dim3( nC * 4 * ft.start[4] ), dim3( kBlock ), 0, s, L, g.stride, ft, fsw, m.cellFaces,
-                             c.flag, part, (const T*) c.x, 0 );
+         hipLaunchKernelGGL( ( kP2Face< T > ), dim3( nC * 4 * ft.start[4] ), dim3( kBlock ), 0, s, L, g.stride, ft, fsw, m.cellFaces, c.flag,
+                             part, (const T*) c.x );
       const int tB = ceilDiv( i64( p2EdgeVertexCount( 1 << L ) ) * kP2EvLanes, kBlock );
       hipLaunchKernelGGL( ( kP2Apply< T, MODE, DIAG, KQ, true > ), dim3( nC * tB ), dim3( kBlock ), 0, s, L, tB, g.stride, el, kq, kqs,
                           m.p2tab, m.cellInfo, m.cellFaces, m.prims, m.entries, part, low, dv, c.flag, (const T*) c.x,
                           (const T*) c.in1, (T*) c.out0, (T*) c.out1, T( c.a ) );
    }
-   else if ( KQ && !DIAG && ol.p2s )
-   {
-      // variable coefficient with stored stencils: the same row and face kernels with per-point weights
-      const T*           sw = dbl ? (const T*) ol.p2s : (const T*) ol.p2sF;
-      const P2ClassTiles ct = p2InteriorTiles( 1 << L );
-      if ( ct.start[8] > 0 && ( c.flag & 1 ) && !skipInterior )
-      {
-         const P2Comps< T > cp{ { (const T*) c.x }, { (const T*) c.in1 }, { (T*) c.out0 }, { (T*) c.out1 } };
-         hipLaunchKernelGGL( ( kP2StoredInt< T, MODE, 1 > ), dim3( xcdGrid( nC * ct.start[8] ) ), dim3( kBlock ), 0, s, L, g.stride, ct, sw,
-                             cp, T( c.a ), nC );
-      }
-      P2FaceTiles ft;
-      ft.start[0] = 0;
-      for ( int k = 0; k < 4; ++k )
-         ft.start[k + 1] = ft.start[k] + ceilDiv( p2FaceSubCount( 1 << L, k & 1, k >> 1 ), kBlock );
-      if ( ft.start[4] > 0 )
-         hipLaunchKernelGGL( ( kP2Face< T, true > ), dim3( xcdGrid( nC * 4 * ft.start[4] ) ), dim3( kBlock ), 0, s, L, g.stride, ft, sw,
-                             m.cellFaces, c.flag, part, (const T*) c.x, nC );
-      const int tB = ceilDiv( i64( p2EdgeVertexCount( 1 << L ) ) * kP2EvLanes, kBlock );
-      hipLaunchKernelGGL( ( kP2Apply< T, MODE, DIAG, KQ, true > ), dim3( nC * tB ), dim3( kBlock ), 0, s, L, tB, g.stride, el, kq, kqs,
-                          m.p2tab, m.cellInfo, m.cellFaces, m.prims, m.entries, part, low, dv, c.flag, (const T*) c.x,
-                          (const T*) c.in1, (T*) c.out0, (T*) c.out1, T( c.a ) );
-   }
-   else
-   hipLaunchKernelGGL( ( kP2Apply< T, MODE, DIAG, KQ > ), dim3( nC * tA ), dim3( kBlock ), 0, s, L, tA, g.stride, el, kq, kqs, m.p2tab,
+   else if constexpr ( DIAG )
+      hipLaunchKernelGGL( ( kP2Apply< T, MODE, DIAG, KQ > ), dim3( nC * tA ), dim3( kBlock ), 0, s, L, tA, g.stride, el, kq, kqs, m.p2tab,
                        m.cellInfo, m.cellFaces, m.prims, m.entries, part, low, dv, c.flag, (const T*) c.x, (const T*) c.in1,
                        (T*) c.out0, (T*) c.out1, T( c.a ) );
-   p2Combines< T, MODE >( m, g, L, c, part, low, dv, s );
+   p2Combines< T, MODE >( m, g, L, &c, 1, part, low, dv, s );
 }
 
 template < typename T, int MODE, bool DIAG >
@@ -1277,53 +1300,11 @@ void launchP2( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, int dt
       p2Mode< float >( m, g, op, L, c, s );
 }
 
-// Apply (replace or add) to up to three functions at once. With stored stencils the cell interiors of all
-// components go through one pass that reads every weight once; the face, edge and vertex points and the
-// combine run per component. Other operators apply component by component.
-template < typename T, int MODE >
-static void p2VectorT( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, const StencilCall* cs, int n, hipStream_t s )
-{
-   constexpr bool         dbl = std::is_same< T, double >::value;
-   const hyg_op_s::Level& ol  = op.levels[L];
-   const P2ClassTiles     ct  = p2InteriorTiles( 1 << L );
-   if ( ct.start[8] > 0 && ( cs[0].flag & 1 ) )
-   {
-      P2Comps< T > cp{};
-      for ( int k = 0; k < n; ++k )
-      {
-         cp.x[k]    = (const T*) cs[k].x;
-         cp.out0[k] = (T*) cs[k].out0;
-      }
-      const T*  sw = dbl ? (const T*) ol.p2s : (const T*) ol.p2sF;
-      const int nC = m.mesh->nC();
-      if ( n == 3 )
-         hipLaunchKernelGGL( ( kP2StoredInt< T, MODE, 3 > ), dim3( xcdGrid( nC * ct.start[8] ) ), dim3( kBlock ), 0, s, L, g.stride, ct, sw, cp,
-                             T( 0 ), nC );
-      else if ( n == 2 )
-         hipLaunchKernelGGL( ( kP2StoredInt< T, MODE, 2 > ), dim3( xcdGrid( nC * ct.start[8] ) ), dim3( kBlock ), 0, s, L, g.stride, ct, sw, cp,
-                             T( 0 ), nC );
-      else
-         hipLaunchKernelGGL( ( kP2StoredInt< T, MODE, 1 > ), dim3( xcdGrid( nC * ct.start[8] ) ), dim3( kBlock ), 0, s, L, g.stride, ct, sw, cp,
-                             T( 0 ), nC );
-   }
-   for ( int k = 0; k < n; ++k )
-      p2TK< T, MODE, false, true >( m, g, op, L, cs[k], s, true );
-}
-
+// Apply (replace or add) to up to three functions at once: the variable coefficient in one pass (without stored stencils for
+// one or three functions), other operators component by component.
 void launchP2Vector( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, int dtype, const StencilCall* cs, int n, hipStream_t s )
 {
-   if ( op.kind == 3 && !op.levels[L].p2s && n == 3 && ( cs[0].mode == MODE_APPLY || cs[0].mode == MODE_APPLY_ADD ) )
-   {
-      // one on-the-fly assembly per point for the three components
-      if ( dtype == 8 )
-         cs[0].mode == MODE_APPLY ? p2KQOnTheFly< double, MODE_APPLY >( m, g, op, L, cs, n, s )
-                                  : p2KQOnTheFly< double, MODE_APPLY_ADD >( m, g, op, L, cs, n, s );
-      else
-         cs[0].mode == MODE_APPLY ? p2KQOnTheFly< float, MODE_APPLY >( m, g, op, L, cs, n, s )
-                                  : p2KQOnTheFly< float, MODE_APPLY_ADD >( m, g, op, L, cs, n, s );
-      return;
-   }
-   const bool fused = op.kind == 3 && op.levels[L].p2s && n >= 1 && n <= 3 &&
+   const bool fused = op.kind == 3 && ( n == 3 || ( op.levels[L].p2s && n >= 1 && n < 3 ) ) &&
                       ( cs[0].mode == MODE_APPLY || cs[0].mode == MODE_APPLY_ADD );
    if ( !fused )
    {
@@ -1332,9 +1313,9 @@ void launchP2Vector( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, 
       return;
    }
    if ( dtype == 8 )
-      cs[0].mode == MODE_APPLY ? p2VectorT< double, MODE_APPLY >( m, g, op, L, cs, n, s ) : p2VectorT< double, MODE_APPLY_ADD >( m, g, op, L, cs, n, s );
+      cs[0].mode == MODE_APPLY ? p2Variable< double, MODE_APPLY >( m, g, op, L, cs, n, s ) : p2Variable< double, MODE_APPLY_ADD >( m, g, op, L, cs, n, s );
    else
-      cs[0].mode == MODE_APPLY ? p2VectorT< float, MODE_APPLY >( m, g, op, L, cs, n, s ) : p2VectorT< float, MODE_APPLY_ADD >( m, g, op, L, cs, n, s );
+      cs[0].mode == MODE_APPLY ? p2Variable< float, MODE_APPLY >( m, g, op, L, cs, n, s ) : p2Variable< float, MODE_APPLY_ADD >( m, g, op, L, cs, n, s );
 }
 
 // coefficient values of every micro-cell at its 11 quadrature points (variable-coefficient P2 operator)
@@ -1360,23 +1341,10 @@ void launchP2StoreStencils( const MeshCtx& m, hyg_op_s& op, int L, hipStream_t s
            hipMalloc( &ol.p2sF, size_t( n ) * sizeof( float ) ) != hipSuccess )
          throw std::runtime_error( "hipMalloc failed for the stored P2 stencils" );
    }
-   // positions of a class sub-lattice that are no cell-interior points keep weight 0
+   // positions of a class sub-lattice on cell edges keep weight 0
    (void) hipMemsetAsync( ol.p2s, 0, size_t( n ) * sizeof( double ), s );
-   P2ClassTiles ct;
-   ct.start[0] = 0;
-   for ( int k = 0; k < 8; ++k )
-   {
-      const int M     = p2InteriorExtent( N, k );
-      ct.start[k + 1] = ct.start[k] + ( M >= 0 ? ceilDiv( S3i( M + 1 ), kBlock ) : 0 );
-   }
-   if ( ct.start[8] > 0 )
-      hipLaunchKernelGGL( kP2StoreInt, dim3( nC * ct.start[8] ), dim3( kBlock ), 0, s, L, ct, ol.p2el, ol.p2kq, p2KqStride( m, L ), ol.p2s );
-   P2FaceTiles ft;
-   ft.start[0] = 0;
-   for ( int k = 0; k < 4; ++k )
-      ft.start[k + 1] = ft.start[k] + ceilDiv( p2FaceSubCount( N, k & 1, k >> 1 ), kBlock );
-   if ( ft.start[4] > 0 )
-      hipLaunchKernelGGL( kP2StoreFace, dim3( nC * 4 * ft.start[4] ), dim3( kBlock ), 0, s, L, ft, ol.p2el, ol.p2kq, p2KqStride( m, L ), ol.p2s );
+   const P2ClassTiles ct = p2ClassTiles( N );
+   hipLaunchKernelGGL( kP2StoreInt, dim3( nC * ct.start[8] ), dim3( kBlock ), 0, s, L, ct, ol.p2el, ol.p2kq, p2KqStride( m, L ), ol.p2s );
    launchConvert( n, 4, ol.p2sF, 8, ol.p2s, s );
 }
 

@@ -7,61 +7,43 @@
 namespace hyg {
 
 // ------------------------------------------------------------------ variable coefficient, assembled on the fly
-// Each point sums, over the micro-cells that have it as node l (known at compile time per parity class; for a
-// cell-face point only those on the cell's side), row l of sum_q k_q M_{t,q} (the rows staged in LDS by p2StageRows,
-// read with wave-uniform loads) times the ten node values, for up to three components at once, so a vector
-// function's components share the assembly. No per-point stencil array is kept, which keeps the register footprint
-// small. Cell-interior points go by class sub-lattice as the stored stencils do, cell-face points per face and
-// sub-lattice (one-sided sums into each component's partial-sum block), the points on cell edges and vertices
-// element by element (kP2Apply).
-// Each point sums, over the micro-cells that have it as node l (on the cell's side of face F for a face point), row
-// l of sum_q k_q M_{t,q} times the ten node values, for up to three components (val[k] += ...). One micro-cell per
-// iteration of a loop that is not unrolled: the micro-cell's data are wave-uniform (scalar loads), and no loads of
-// one micro-cell can be hoisted above another's, so the register footprint is that of one micro-cell. rb: starts of
-// the rows py + dy of the planes pz + dz (|dy|, |dz| <= 2) relative to the cell, base = cell offset + px.
-template < typename T, int CLS, int F >
-__device__ __forceinline__ void p2KQDirect( int c, int N, int px, int py, int pz, const T* __restrict__ kq, i64 kqStride,
-                                            const T* __restrict__ Ms, const int ( &rb )[5][5], i64 base, const P2Comps< T >& cp, int nc,
-                                            T ( &val )[3], bool onFace = false )
+// The stencil of a point is assembled in registers from the rows of its micro-cells (p2Row; the slots of the ten nodes are
+// known at compile time) and then applied to up to three components, so a vector function's components share it. A
+// micro-cell's moments are 10 loads of consecutive values by consecutive threads, each value of the 65 (vertex class), 27 or
+// 19 points of the stencil is loaded once. A micro-cell at a time: the branch around it (a face point takes those inside the
+// cell) keeps the loads of one from being hoisted above another's (branch-free, with zero moments outside the cell, the
+// compiler kept the loads of all 24 micro-cells of a vertex point in flight and spilled 400 registers).
+// Three components on the shell (960 cells, P2 level 4, 3 x 5.2 million points, FP64): the two launches 960 us, against 1868
+// us with rows of 11-point sums read from LDS (110 multiply-adds and 55 LDS reads per row, a load per node and micro-cell).
+// Per point 75 loads of moments and 29 per component of values remain; the vertex class (1/8 of the points, 24 micro-cells each)
+// takes 420 us of it at two waves per SIMD.
+template < typename T, int CLS, int K >
+__device__ __forceinline__ void p2AddRow( int c, int Nc, int SA, int px, int py, int pz, const T* __restrict__ kq, i64 kqStride,
+                                          const T* __restrict__ g, T ( &W )[p2StencilOffsets( CLS ).n] )
 {
-   const int          Nc = N >> 1, SA = S3i( Nc + 1 );
-   const P2KQEntries& E  = kP2KQTab.c[CLS][F + 1];
-   int                rf[25];
-#pragma unroll
-   for ( int a = 0; a < 25; ++a )
-      rf[a] = rb[a / 5][a % 5];
-#pragma unroll 1
-   for ( int k = 0; k < E.n; ++k )
+   typedef const T __attribute__( ( address_space( 4 ) ) ) CT;
+   constexpr P2KQEntry e  = kP2Entries.c[CLS].e[K];
+   const int           ax = ( px - e.nd[0] ) >> 1, ay = ( py - e.nd[1] ) >> 1, az = ( pz - e.nd[2] ) >> 1;
+   if ( ax >= 0 && ay >= 0 && az >= 0 && ax + ay + az + e.mcmax <= Nc )
    {
-      const P2KQEntry& e  = E.e[k];
-      const int        ax = ( px - e.nd[0] ) >> 1, ay = ( py - e.nd[1] ) >> 1, az = ( pz - e.nd[2] ) >> 1;
-      // a point on a cell face takes the micro-cells inside the cell (its one-sided sum)
-      if ( onFace && ( ax < 0 || ay < 0 || az < 0 || ax + ay + az + e.mcmax > Nc ) )
-         continue;
-      const T* kv = kq + i64( c * 6 + e.t ) * SA + cidx( Nc + 1, ax, ay, az );
-      T        kk[11];
+      const T*       kv = kq + i64( c * 6 + e.t ) * SA;
+      const unsigned o  = unsigned( cidx( Nc + 1, ax, ay, az ) );
+      T              m[kP2Moments], r[10];
 #pragma unroll
-      for ( int q = 0; q < 11; ++q )
-         kk[q] = kv[i64( q ) * kqStride];
+      for ( int q = 0; q < kP2Moments; ++q )
+         m[q] = ( kv + i64( q ) * kqStride )[o];
+      p2Row< e.l >( m, (CT*) ( g + ( c * 6 + e.t ) * kP2Moments ), r );
 #pragma unroll
-      for ( int jj = 0; jj < 10; ++jj )
-      {
-         const T* row = Ms + ( e.ord * 10 + jj ) * kP2RowPad;
-         T        r   = T( 0 );
-#pragma unroll
-         for ( int q = 0; q < 11; ++q )
-            r += kk[q] * row[q];
-         const int nk = e.node[jj];
-         const i64 o  = base + rf[nk & 255] + ( ( nk >> 8 ) - 2 );
-         // explicit fused multiply-adds: every component (and the single-component pass) rounds alike
-         val[0] = fma( r, cp.x[0][o], val[0] );
-         if ( nc > 1 )
-         {
-            val[1] = fma( r, cp.x[1][o], val[1] );
-            val[2] = fma( r, cp.x[2][o], val[2] );
-         }
-      }
+      for ( int j = 0; j < 10; ++j )
+         W[e.slot[j]] += r[j];
    }
+}
+template < typename T, int CLS, int... K >
+__device__ __forceinline__ void p2Assemble( int c, int Nc, int px, int py, int pz, const T* __restrict__ kq, i64 kqStride,
+                                            const T* __restrict__ g, T ( &W )[p2StencilOffsets( CLS ).n], std::integer_sequence< int, K... > )
+{
+   const int SA = S3i( Nc + 1 );
+   ( p2AddRow< T, CLS, K >( c, Nc, SA, px, py, pz, kq, kqStride, g, W ), ... );
 }
 template < typename T >
 __device__ __forceinline__ void p2EmitInterior( int mode, int nc, const T ( &val )[3], i64 q, const P2Comps< T >& cp,
@@ -118,43 +100,46 @@ __device__ __forceinline__ void p2EmitInterior( int mode, int nc, const T ( &val
 template < typename T, int CLS >
 __device__ __forceinline__ void p2KQIntPt( int c, int s, int N, i64 stride, const T* __restrict__ el, const T* __restrict__ kq,
                                            i64 kqStride, const T* __restrict__ dinv, const P2Comps< T >& cp, int nc, int mode, T a,
-                                           T* __restrict__ Ms, const CellFaceSlot* __restrict__ cfs, int flag, T* __restrict__ part,
-                                           i64 partStride )
+                                           const CellFaceSlot* __restrict__ cfs, int flag, T* __restrict__ part, i64 partStride )
 {
-   constexpr int kx = CLS & 1, ky = ( CLS >> 1 ) & 1, kz = ( CLS >> 2 ) & 1;
-   p2StageRows< T, CLS >( el, c, Ms );
-   const int M = p2ClassExtent( N, CLS );
+   constexpr int              kx = CLS & 1, ky = ( CLS >> 1 ) & 1, kz = ( CLS >> 2 ) & 1;
+   constexpr P2StencilOffsets off = p2StencilOffsets( CLS );
+   const int                  M   = p2ClassExtent( N, CLS );
    if ( s >= S3i( M + 1 ) )
       return;
    int qx, qy, qz;
    tetXYZ( M + 1, s, qx, qy, qz );
    const int px = 2 * qx + kx, py = 2 * qy + ky, pz = 2 * qz + kz;
-   const int slot = classifySlot( N, px, py, pz );
-   if ( slot > 4 || ( slot == 0 && !( flag & 1 ) ) ) // cell edges and vertices: kP2Apply
+   int       slot;
+   i64       pi;
+   if ( !p2PointWanted( c, N, px, py, pz, cfs, flag, slot, pi ) )
       return;
-   i64 pi = 0;
-   if ( slot > 0 )
-   {
-      const CellFaceSlot fs = cfs[4 * c + slot - 1];
-      if ( !( fs.bc & flag ) )
-         return;
-      pi = i64( fs.block ) * ( N + 1 ) * ( N + 1 ) + facePartIndex( slot - 1, N, px, py, pz );
-   }
-   const int w = N + 1;
-   int       rb[5][5];
+   T W[off.n];
 #pragma unroll
-   for ( int dz = -2; dz <= 2; ++dz )
-   {
-      const int Wz = w - ( pz + dz );
-      const int pb = S3i( w ) - S3i( Wz );
+   for ( int e = 0; e < off.n; ++e )
+      W[e] = T( 0 );
+   p2Assemble< T, CLS >( c, N >> 1, px, py, pz, kq, kqStride, el, W, std::make_integer_sequence< int, kP2Entries.c[CLS].n >() );
+   int rb[5][5];
+   p2RowStarts( N, px, py, pz, rb );
+   const i64 cb     = i64( c ) * stride;
+   const int q      = rb[2][2];
+   const P2Inside in( N, px, py, pz );
+   T          val[3] = { T( 0 ), T( 0 ), T( 0 ) };
 #pragma unroll
-      for ( int dy = -2; dy <= 2; ++dy )
-         rb[dz + 2][dy + 2] = pb + rowStart( Wz, py + dy );
+   for ( int e = 0; e < off.n; ++e )
+   {
+      // a node outside the cell has no weight: the point reads itself instead
+      const int o = in.has( off.d[e][0], off.d[e][1], off.d[e][2] ) ? rb[off.d[e][2] + 2][off.d[e][1] + 2] + off.d[e][0] : q;
+      // explicit fused multiply-adds: every component (and the single-component pass) rounds alike
+      val[0] = fma( W[e], ( cp.x[0] + cb )[unsigned( o )], val[0] );
+      if ( nc > 1 )
+      {
+         val[1] = fma( W[e], ( cp.x[1] + cb )[unsigned( o )], val[1] );
+         val[2] = fma( W[e], ( cp.x[2] + cb )[unsigned( o )], val[2] );
+      }
    }
-   T val[3] = { T( 0 ), T( 0 ), T( 0 ) };
-   p2KQDirect< T, CLS, -1 >( c, N, px, py, pz, kq, kqStride, Ms, rb, i64( c ) * stride + px, cp, nc, val, slot > 0 );
    if ( slot == 0 )
-      p2EmitInterior< T >( mode, nc, val, i64( c ) * stride + rb[2][2] + px, cp, dinv, a );
+      p2EmitInterior< T >( mode, nc, val, cb + q, cp, dinv, a );
    else
    {
 #pragma unroll
@@ -168,46 +153,52 @@ __device__ __forceinline__ void p2KQIntPt( int c, int s, int N, i64 stride, cons
 }
 template < typename T, int CLS >
 __device__ __forceinline__ void p2KQIntDispatch( int cls, int c, int s, int N, i64 stride, const T* el, const T* kq, i64 kqStride,
-                                                 const T* dinv, const P2Comps< T >& cp, int nc, int mode, T a, T* Ms,
-                                                 const CellFaceSlot* cfs, int flag, T* part, i64 partStride )
+                                                 const T* dinv, const P2Comps< T >& cp, int nc, int mode, T a, const CellFaceSlot* cfs,
+                                                 int flag, T* part, i64 partStride )
 {
    if ( cls == CLS )
-      p2KQIntPt< T, CLS >( c, s, N, stride, el, kq, kqStride, dinv, cp, nc, mode, a, Ms, cfs, flag, part, partStride );
+      p2KQIntPt< T, CLS >( c, s, N, stride, el, kq, kqStride, dinv, cp, nc, mode, a, cfs, flag, part, partStride );
    else if constexpr ( CLS < 7 )
-      p2KQIntDispatch< T, CLS + 1 >( cls, c, s, N, stride, el, kq, kqStride, dinv, cp, nc, mode, a, Ms, cfs, flag, part, partStride );
+      p2KQIntDispatch< T, CLS + 1 >( cls, c, s, N, stride, el, kq, kqStride, dinv, cp, nc, mode, a, cfs, flag, part, partStride );
 }
-template < typename T >
-__global__ __launch_bounds__( kBlock ) void kP2KQInt( int L, i64 stride, P2ClassTiles ct, const T* __restrict__ el,
+// VERTEX: the points of class 0, whose 65-point stencil needs twice the registers of the other classes; else classes 1..7
+template < typename T, bool VERTEX >
+__global__ __launch_bounds__( kBlock, VERTEX ? 2 : 4 ) void kP2KQInt( int L, i64 stride, P2ClassTiles ct, const T* __restrict__ el,
                                                       const T* __restrict__ kq, i64 kqStride, const T* __restrict__ dinv,
                                                       P2Comps< T > cp, int nc, int mode, T a, const CellFaceSlot* __restrict__ cfs,
                                                       int flag, T* __restrict__ part, i64 partStride, int nC )
 {
-   __shared__ T Ms[kP2MaxPairs * 10 * kP2RowPad];
-   const int    per = ct.start[8];
+   const int t0 = VERTEX ? 0 : ct.start[1], per = ( VERTEX ? ct.start[1] : ct.start[8] ) - t0;
    // each XCD takes a contiguous range of cells (the hardware deals workgroups out round-robin over the 8 XCDs), so
    // a cell's coefficient values and source stay in one XCD's L2 while its class blocks run
    const int b = remapXcd( int( blockIdx.x ), nC * per );
    if ( b >= nC * per ) // the whole block (grid padded to a multiple of 8)
       return;
    const int c = b / per;
-   const int t = b - c * per;
-   int          cls = 0;
-   while ( cls < 7 && t >= ct.start[cls + 1] )
-      ++cls;
-   p2KQIntDispatch< T, 0 >( cls, c, ( t - ct.start[cls] ) * kBlock + int( threadIdx.x ), 1 << L, stride, el, kq, kqStride, dinv, cp,
-                            nc, mode, a, Ms, cfs, flag, part, partStride );
+   const int t = t0 + b - c * per;
+   if constexpr ( VERTEX )
+      p2KQIntPt< T, 0 >( c, t * kBlock + int( threadIdx.x ), 1 << L, stride, el, kq, kqStride, dinv, cp, nc, mode, a, cfs, flag, part,
+                         partStride );
+   else
+   {
+      int cls = 1;
+      while ( cls < 7 && t >= ct.start[cls + 1] )
+         ++cls;
+      p2KQIntDispatch< T, 1 >( cls, c, ( t - ct.start[cls] ) * kBlock + int( threadIdx.x ), 1 << L, stride, el, kq, kqStride, dinv, cp, nc,
+                               mode, a, cfs, flag, part, partStride );
+   }
 }
 template < typename T >
 void launchP2KQPoints( int L, int nC, i64 stride, const T* el, const T* kq, i64 kqStride, const T* dinv, const P2Comps< T >& cp, int nc,
                        int mode, T a, const CellFaceSlot* cfs, int flag, T* part, i64 partStride, hipStream_t s )
 {
-   const int    N = 1 << L;
-   P2ClassTiles ct;
-   ct.start[0] = 0;
-   for ( int k = 0; k < 8; ++k )
-      ct.start[k + 1] = ct.start[k] + ceilDiv( S3i( p2ClassExtent( N, k ) + 1 ), kBlock );
-   hipLaunchKernelGGL( ( kP2KQInt< T > ), dim3( xcdGrid( nC * ct.start[8] ) ), dim3( kBlock ), 0, s, L, stride, ct, el, kq, kqStride, dinv,
-                       cp, nc, mode, a, cfs, flag, part, partStride, nC );
+   const P2ClassTiles ct = p2ClassTiles( 1 << L );
+   if ( ct.start[1] > 0 )
+      hipLaunchKernelGGL( ( kP2KQInt< T, true > ), dim3( xcdGrid( nC * ct.start[1] ) ), dim3( kBlock ), 0, s, L, stride, ct, el, kq, kqStride,
+                          dinv, cp, nc, mode, a, cfs, flag, part, partStride, nC );
+   if ( ct.start[8] > ct.start[1] )
+      hipLaunchKernelGGL( ( kP2KQInt< T, false > ), dim3( xcdGrid( nC * ( ct.start[8] - ct.start[1] ) ) ), dim3( kBlock ), 0, s, L, stride, ct,
+                          el, kq, kqStride, dinv, cp, nc, mode, a, cfs, flag, part, partStride, nC );
 }
 
 } // namespace hyg

@@ -877,7 +877,7 @@ void assembleP2DivKGrad( hyg_op_s& op )
       hyg_op_s::Level& ol = op.levels[L];
       const int        N  = 1 << L;
       const int        Ne = N / 2;
-      std::vector< double >   el( size_t( m.nC() ) * 6600 );
+      std::vector< double >   el( size_t( m.nC() ) * 60 );
       std::vector< ElemCell > ec( m.nC() );
       for ( int c = 0; c < m.nC(); ++c )
       {
@@ -907,30 +907,18 @@ void assembleP2DivKGrad( hyg_op_s& op )
                for ( int r = 0; r < 3; ++r )
                   g[i][r] = nrm[r] / sc;
             }
-            for ( int q = 0; q < 11; ++q )
-            {
-               const double* lam = kXG4Lambda[q];
-               V3            d[10];
-               for ( int v = 0; v < 4; ++v )
-                  for ( int r = 0; r < 3; ++r )
-                     d[v][r] = ( 4.0 * lam[v] - 1.0 ) * g[v][r];
-               for ( int e = 0; e < 6; ++e )
-               {
-                  const int pa = kP2Edge[e][0], pb = kP2Edge[e][1];
-                  for ( int r = 0; r < 3; ++r )
-                     d[4 + e][r] = 4.0 * ( lam[pa] * g[pb][r] + lam[pb] * g[pa][r] );
-               }
-               for ( int i = 0; i < 10; ++i )
-                  for ( int j = 0; j < 10; ++j )
-                     el[size_t( c ) * 6600 + 1100 * t + 100 * q + 10 * i + j] = kXG4Weight[q] * adet * dot3( d[i], d[j] );
-            }
+            // G_ab = |det J| grad lambda_a . grad lambda_b, a <= b
+            double* gt = &el[size_t( c ) * 60 + 10 * t];
+            for ( int i = 0; i < 4; ++i )
+               for ( int j = i; j < 4; ++j )
+                  *gt++ = adet * dot3( g[i], g[j] );
          }
       }
       std::vector< float > elF( el.begin(), el.end() );
       ol.p2el              = upload( el );
       ol.p2elF             = upload( elF );
       ol.elem              = upload( ec );
-      const size_t nKq     = size_t( m.nC() ) * 6 * size_t( S3( Ne + 1 ) ) * 11;
+      const size_t nKq     = size_t( m.nC() ) * 6 * size_t( S3( Ne + 1 ) ) * 10;
       const size_t nLow    = mc.entriesHost.size() * size_t( N + 1 );
       const size_t nFace   = size_t( m.nF() ) * 2 * size_t( N + 1 ) * size_t( N + 1 );
       const size_t nFunc   = size_t( m.nC() ) * size_t( cellStride( L ) ) + size_t( kTailSlack );

@@ -143,3 +143,35 @@ def test_coefficient_integrals_of_every_variant(hyg, nmodes, L, dtype):
     oop.apply(ox, od, L, ol.ALL, False)
     # FP32: rounding of up to 2 * 64 terms of total size sqrt(2 * 64) * 0.5 in log k, 6e-6, and 34 roundings of the sum
     assert rel_inf(y.download(L), od.get(L)) <= (1e-13 if dt == hyg.F64 else 2e-5)
+
+
+@pytest.mark.parametrize("stored", [False, True])
+@pytest.mark.parametrize("name,L", [("tet_1el.msh", 0), ("tet_1el.msh", 1), ("three_tets_with_two_joint_faces.msh", 2),
+                                    ("pyramid_tilted_4el.msh", 4)])
+def test_variable_p2_every_kind_of_point(hyg, name, L, stored):
+    """Vertex, edge-midpoint, face and cell-edge points by the moments of k, one and several components, both value types."""
+    gm, om = hyg.Mesh(name), ol.Mesh(name)
+    n = gm.ndofs(L + 1)
+    op = hyg.P2DivKGradOperator(gm, L, L, kind=0, k0=1.2, alpha=0.7, beta=0.3, seed=11)
+    if stored:
+        op.store_local_matrices()
+    oop = ol.P2DivKGradOperator(om, L, L, kind=0, k0=1.2, alpha=0.7, beta=0.3, seed=11)
+    # FP32: at most 24 micro-cells of 10 products, 240 + 24 roundings of terms of at most a few times the largest result
+    for dt, tol in ((hyg.F64, 1e-13), (hyg.F32, 264 * 4 * 2.0 ** -24)):
+        xs = [hyg.Function(gm, L, L, dt, space="p2") for _ in range(3)]
+        ys = [hyg.Function(gm, L, L, dt, space="p2") for _ in range(3)]
+        ref = []
+        for k in range(3):
+            v = rnd(n, 50 + k, dt == hyg.F32)
+            xs[k].upload(L, v)
+            ox, oy = ol.Function(om, L + 1, L + 1), ol.Function(om, L + 1, L + 1)
+            ox.set(L + 1, v)
+            oop.apply(ox, oy, L + 1, ol.ALL, False)
+            ref.append(oy.get(L + 1))
+        for comps in (1, 2, 3):
+            print(name, L, stored, dt, comps, flush=True)
+            for y in ys:
+                y.interpolate(0.0, L)
+            hyg.apply_vector(op, xs[:comps], ys[:comps], L, hyg.ALL)
+            for k in range(comps):
+                assert rel_inf(ys[k].download(L), ref[k]) <= tol, (comps, k)

@@ -173,7 +173,7 @@ __global__ __launch_bounds__( kBlock ) void kBatchTransfer( const TransferTask< 
       if ( t.kind == 0 )
          bRestrictCell< T >( b, t.tiles, t.tile0, t.nTiles, t.nC, t.L, t.strideC, t.strideF, t.dst, t.src );
       else if ( t.kind == 1 )
-         bRestrictLower< T >( b, t.chunks, t.nChunks, t.prims, t.entries, t.cinfo, t.L, t.strideC, t.strideF, t.flag, t.dst, t.src );
+         bRestrictLower< T >( b, t.chunks, t.nChunks, t.entries, t.cinfo, t.L, t.strideC, t.strideF, t.flag, t.dst, t.src );
       else
          bProlongate< T >( b, t.tiles, t.nTiles, t.nC, t.L, t.strideF, t.strideC, t.cinfo, t.flag, t.dst, t.src, t.add );
    }

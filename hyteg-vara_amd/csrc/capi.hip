@@ -305,18 +305,6 @@ int smoothImpl( hyg_gmg_s* g, hyg_func_s* x, hyg_func_s* b, int L, hipStream_t s
 {
    StencilCall c;
    c.flag = kGmgFlag;
-   if ( g->smoother == 0 )
-   {
-      // WeightedJacobiSmoother::solve: tmp := x (All); smooth_jac(x, b, tmp)
-      launchCopy( levelValues( x, L ), g->dtype, g->jt->data[L], x->data[L], st );
-      HYG_TRY( launched( "copy" ) );
-      c.mode = MODE_JACOBI;
-      c.x    = g->jt->data[L];
-      c.in1  = b->data[L];
-      c.out0 = x->data[L];
-      c.a    = g->relax;
-      return stencilImpl( g->op, L, g->dtype, c, st );
-   }
    if ( g->smoother >= 4 )
    {
       // the same in the reference's own order (smooth_sor_ordered)
@@ -363,6 +351,35 @@ int smoothImpl( hyg_gmg_s* g, hyg_func_s* x, hyg_func_s* b, int L, hipStream_t s
       const double one = 1.0;
       hyg_func_s*  src = g->cy;
       return lincombImpl( x, 1, &one, &src, false, 0.0, L, kGmgFlag, st );
+   }
+   return HYG_OK;
+}
+
+// n smoothing steps. WeightedJacobiSmoother::solve (tmp := x (All); smooth_jac(x, b, tmp)) n times: x and tmp change places
+// between the steps, so only the first needs the copy (points outside the flag then hold the same values in both).
+int smoothSteps( hyg_gmg_s* g, hyg_func_s* x, hyg_func_s* b, int L, int n, hipStream_t st )
+{
+   if ( g->smoother != 0 )
+   {
+      for ( int i = 0; i < n; ++i )
+         HYG_TRY( smoothImpl( g, x, b, L, st ) );
+      return HYG_OK;
+   }
+   if ( n <= 0 )
+      return HYG_OK;
+   launchCopy( levelValues( x, L ), g->dtype, g->jt->data[L], x->data[L], st );
+   HYG_TRY( launched( "copy" ) );
+   for ( int i = n; i > 0; --i )
+   {
+      // the last step ends in x: step i of the remaining ones goes from tmp to x when i is odd
+      StencilCall c;
+      c.flag = kGmgFlag;
+      c.mode = MODE_JACOBI;
+      c.x    = ( i & 1 ) ? g->jt->data[L] : x->data[L];
+      c.in1  = b->data[L];
+      c.out0 = ( i & 1 ) ? x->data[L] : g->jt->data[L];
+      c.a    = g->relax;
+      HYG_TRY( stencilImpl( g->op, L, g->dtype, c, st ) );
    }
    return HYG_OK;
 }
@@ -457,8 +474,7 @@ int vcycleImpl( hyg_gmg_s* g, hyg_func_s* x, hyg_func_s* b, int L, int invoked, 
       return deviceCg ? cgDeviceImpl( g, x, b, L, st ) : cgImpl( g, x, b, L, st );
    MeshCtx&  mc   = g->op->mesh->ctx;
    const int preS = g->pre + g->inc * ( invoked - L );
-   for ( int i = 0; i < preS; ++i )
-      HYG_TRY( smoothImpl( g, x, b, L, st ) );
+   HYG_TRY( smoothSteps( g, x, b, L, preS, st ) );
    StencilCall c;
    c.flag = kGmgFlag;
    c.mode = MODE_RESIDUAL;
@@ -466,15 +482,18 @@ int vcycleImpl( hyg_gmg_s* g, hyg_func_s* x, hyg_func_s* b, int L, int invoked, 
    c.in1  = b->data[L];
    c.out0 = g->tmp->data[L];
    HYG_TRY( stencilImpl( g->op, L, g->dtype, c, st ) );
+   // the restricted residual is the right-hand side of the coarse level, whose iterate starts from 0
    if ( g->op->lat )
-      launchP2Restrict( mc, mc.geom( L - 1 ), mc.p2Tables(), L - 1, g->dtype, g->tmp->data[L - 1], g->tmp->data[L], kGmgFlag, st );
+   {
+      launchP2Restrict( mc, mc.geom( L - 1 ), mc.p2Tables(), L - 1, g->dtype, b->data[L - 1], g->tmp->data[L], kGmgFlag, st );
+      HYG_TRY( launched( "restrict" ) );
+      HYG_TRY( lincombImpl( x, 0, nullptr, nullptr, false, 0.0, L - 1, HYG_ALL, st ) );
+   }
    else
-      launchRestrict( mc, mc.geom( L - 1 ), L - 1, g->dtype, g->tmp->data[L - 1], g->tmp->data[L], kGmgFlag, st );
-   HYG_TRY( launched( "restrict" ) );
-   const double one = 1.0;
-   hyg_func_s*  t   = g->tmp;
-   HYG_TRY( lincombImpl( b, 1, &one, &t, false, 0.0, L - 1, kGmgFlag, st ) );
-   HYG_TRY( lincombImpl( x, 0, nullptr, nullptr, false, 0.0, L - 1, HYG_ALL, st ) );
+   {
+      launchRestrict( mc, mc.geom( L - 1 ), L - 1, g->dtype, b->data[L - 1], g->tmp->data[L], kGmgFlag, st, x->data[L - 1] );
+      HYG_TRY( launched( "restrict" ) );
+   }
    HYG_TRY( vcycleImpl( g, x, b, L - 1, invoked, st, deviceCg ) );
    if ( g->op->lat )
       launchP2Prolongate( mc, mc.geom( L ), mc.p2Tables(), L, g->dtype, x->data[L], x->data[L - 1], kGmgFlag, true, st );
@@ -482,8 +501,7 @@ int vcycleImpl( hyg_gmg_s* g, hyg_func_s* x, hyg_func_s* b, int L, int invoked, 
       launchProlongate( mc, mc.geom( L ), L, g->dtype, x->data[L], x->data[L - 1], kGmgFlag, true, st );
    HYG_TRY( launched( "prolongate" ) );
    const int postS = g->post + g->inc * ( invoked - L );
-   for ( int i = 0; i < postS; ++i )
-      HYG_TRY( smoothImpl( g, x, b, L, st ) );
+   HYG_TRY( smoothSteps( g, x, b, L, postS, st ) );
    return HYG_OK;
 }
 

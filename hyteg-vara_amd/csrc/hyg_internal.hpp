@@ -573,7 +573,8 @@ struct LevelGeom
          for ( int& v : t )
             v = -1;
    }
-   // variable-coefficient operator: z-marching segments over all points of a cell, rows and planes from 0 (elemSweep)
+   // variable-coefficient operator: z-marching segments over all points of a cell, rows and planes from 0 (elemSweep), built
+   // when such an operator is created
    std::vector< ZSeg >                      eSegsHost;
    ZSeg*                                    eSegs  = nullptr;
    int                                      nESegs = 0;
@@ -636,6 +637,7 @@ struct MeshCtx
    void                        setShellMap(); // throws when a cell is not a shell cell
    void                        buildTopology(); // prims, entries, cell info (host + device)
    LevelGeom&                  geom( int L );
+   void                        buildElemSegs( int L );
    const P2Tables*             p2Tables();
    ~MeshCtx();
 };

@@ -221,31 +221,25 @@ void launchInvDiag( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::Level&
 }
 
 template < typename T >
-static void restrictT( const MeshCtx& m, const LevelGeom& gc, int Lc, void* coarse, const void* fine, int flag, hipStream_t st )
+static void restrictT( const MeshCtx& m, const LevelGeom& gc, int Lc, void* coarse, const void* fine, int flag, void* zero, hipStream_t st )
 {
-   const int nC      = m.mesh->nC();
-   const i64 strideF = cellStride( Lc + 1 );
+   const int nC = m.mesh->nC();
    // cell-interior coarse points are restricted whatever the flag (the reference's cell loop has no flag test,
    // P1toP1LinearRestriction.cpp:181-260)
-   if ( gc.nInteriorTiles > 0 )
-   {
-      const int nb = gc.nInteriorTiles * nC;
-      hipLaunchKernelGGL( ( kRestrictCell< T > ), dim3( xcdGrid( nb ) ), dim3( kBlock ), 0, st, gc.tiles, gc.interiorTile0,
-                          gc.nInteriorTiles, nC, Lc, gc.stride, strideF, (T*) coarse, (const T*) fine );
-   }
-   if ( gc.nChunks > 0 )
-      hipLaunchKernelGGL( ( kRestrictLower< T > ), dim3( ceilDiv( gc.nChunks, kBlock / 64 ) ), dim3( kBlock ), 0, st, gc.chunks,
-                          gc.nChunks, m.prims, m.entries, m.cellInfo, Lc, gc.stride, strideF, flag, (T*) coarse,
-                          (const T*) fine );
+   const int gL = gc.nChunks > 0 ? xcdGrid( ceilDiv( gc.nChunks, kBlock / 64 ) ) : 0, gC = xcdGrid( gc.nInteriorTiles * nC );
+   const i64 nZero = zero ? i64( nC ) * gc.stride : 0;
+   hipLaunchKernelGGL( ( kRestrict< T > ), dim3( gL + gC + ceilDiv( nZero, 4 * kBlock ) ), dim3( kBlock ), 0, st, gL, gC, gc.chunks, gc.nChunks,
+                       m.entries, m.cellInfo, gc.tiles, gc.interiorTile0, gc.nInteriorTiles, nC, Lc, gc.stride, cellStride( Lc + 1 ), flag,
+                       (T*) coarse, (const T*) fine, (T*) zero, nZero );
 }
 
 void launchRestrict( const MeshCtx& m, const LevelGeom& gc, int Lc, int dtype, void* coarse, const void* fine, int flag,
-                     hipStream_t st )
+                     hipStream_t st, void* zero )
 {
    if ( dtype == 8 )
-      restrictT< double >( m, gc, Lc, coarse, fine, flag, st );
+      restrictT< double >( m, gc, Lc, coarse, fine, flag, zero, st );
    else
-      restrictT< float >( m, gc, Lc, coarse, fine, flag, st );
+      restrictT< float >( m, gc, Lc, coarse, fine, flag, zero, st );
 }
 
 void launchProlongate( const MeshCtx& m, const LevelGeom& gf, int Lf, int dtype, void* fine, const void* coarse, int flag,

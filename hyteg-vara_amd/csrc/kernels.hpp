@@ -107,7 +107,8 @@ void launchInvDiag( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::Level&
 
 // grid transfer: restriction level Lc+1 -> Lc, prolongation Lf-1 -> Lf
 void launchRestrict( const MeshCtx& m, const LevelGeom& gc, int Lc, int dtype, void* coarse, const void* fine, int flag,
-                     hipStream_t st );
+                     hipStream_t st ,
+                     void* zero = nullptr );
 void launchProlongate( const MeshCtx& m, const LevelGeom& gf, int Lf, int dtype, void* fine, const void* coarse, int flag,
                        bool add, hipStream_t st );
 

@@ -334,19 +334,10 @@ __device__ __forceinline__ void bRestrictCell( int bid, const PlaneTile* __restr
    }
 }
 
-template < typename T >
-__global__ __launch_bounds__( kBlock ) void kRestrictCell( const PlaneTile* __restrict__ tiles, int tile0, int nTiles, int nC,
-                                                           int Lc, i64 strideC, i64 strideF, T* __restrict__ coarse,
-                                                           const T* __restrict__ fine )
-{
-   bRestrictCell< T >( int( blockIdx.x ), tiles, tile0, nTiles, nC, Lc, strideC, strideF, coarse, fine );
-}
-
 // Restriction, coarse points on macro-faces/-edges/-vertices: sum over the incident cells of the
 // in-cell fine neighbours, each scaled by 1 / (#cells sharing the fine point's primitive).
 template < typename T >
 __device__ __forceinline__ void bRestrictLower( int bid, const LowerChunk* __restrict__ chunks, int nChunks,
-                                                            const LowerPrim* __restrict__ prims,
                                                             const LowerEntry* __restrict__ entries,
                                                             const CellInfo* __restrict__ cinfo, int Lc, i64 strideC,
                                                             i64 strideF, int flag, T* __restrict__ coarse,
@@ -399,15 +390,29 @@ __device__ __forceinline__ void bRestrictLower( int bid, const LowerChunk* __res
    }
 }
 
+// One launch per restriction: blocks [0, gL) the points on faces, edges and vertices, whose chains of dependent loads take
+// longest, then [gL, gL + gC) the cell interiors, then `zero` (if not null) cleared, 4 kBlock values a block (the iterate
+// of the coarse level a cycle goes down to).
 template < typename T >
-__global__ __launch_bounds__( kBlock ) void kRestrictLower( const LowerChunk* __restrict__ chunks, int nChunks,
-                                                            const LowerPrim* __restrict__ prims,
-                                                            const LowerEntry* __restrict__ entries,
-                                                            const CellInfo* __restrict__ cinfo, int Lc, i64 strideC,
-                                                            i64 strideF, int flag, T* __restrict__ coarse,
-                                                            const T* __restrict__ fine )
+__global__ __launch_bounds__( kBlock ) void kRestrict( int gL, int gC, const LowerChunk* __restrict__ chunks, int nChunks,
+                                                       const LowerEntry* __restrict__ entries, const CellInfo* __restrict__ cinfo,
+                                                       const PlaneTile* __restrict__ tiles, int tile0, int nTiles, int nC, int Lc, i64 strideC,
+                                                       i64 strideF, int flag, T* __restrict__ coarse, const T* __restrict__ fine,
+                                                       T* __restrict__ zero, i64 nZero )
 {
-   bRestrictLower< T >( int( blockIdx.x ), chunks, nChunks, prims, entries, cinfo, Lc, strideC, strideF, flag, coarse, fine );
+   const int b = int( blockIdx.x );
+   if ( b < gL )
+      bRestrictLower< T >( b, chunks, nChunks, entries, cinfo, Lc, strideC, strideF, flag, coarse, fine );
+   else if ( b < gL + gC )
+      bRestrictCell< T >( b - gL, tiles, tile0, nTiles, nC, Lc, strideC, strideF, coarse, fine );
+   else
+   {
+      const i64 i0 = i64( b - gL - gC ) * 4 * kBlock + threadIdx.x;
+#pragma unroll
+      for ( int u = 0; u < 4; ++u )
+         if ( i0 + u * kBlock < nZero )
+            zero[i0 + u * kBlock] = T( 0 );
+   }
 }
 
 } // namespace hyg

@@ -356,23 +356,6 @@ LevelGeom& MeshCtx::geom( int L )
       g.nZSegs[k] = (int) v.size();
       g.zSegs[k]  = upload( v );
    }
-   {
-      // variable-coefficient sweep: rows y .. y+kElemRows-1, points x0 .. x0+61, planes z0 .. z1-1 of the closed cell
-      auto& v = g.eSegsHost;
-      v.clear();
-      i64 steps = 0;
-      for ( int y = 0; y <= N; y += kElemRows )
-         for ( int x0 = 0; x0 <= N - y; x0 += 62 )
-            steps += N - y - x0 + 1;
-      const int most  = int( std::max< i64 >( kZSegLeast, std::min< i64 >( kZSegChunk, steps * mesh->nC() / kElemWaves ) ) );
-      const int chunk = ec ? std::max( 2, std::min( 1024, std::atoi( ec ) ) ) : most;
-      for ( int z0 = 0; z0 <= N; z0 += chunk )
-         for ( int x0 = 0; x0 <= N - z0; x0 += 62 )
-            for ( int y = 0; y + x0 + z0 <= N; y += kElemRows )
-               v.push_back( { y, x0, z0, std::min( z0 + chunk, N - y - x0 + 1 ) } );
-      g.nESegs = (int) v.size();
-      g.eSegs  = upload( v );
-   }
    // P2 row pairs (y0, y0+1), y0 even: segment k holds the x values 124k .. 124k+123 (k = 0 from x = 1); the
    // pair has interior outputs while z <= N - 1 - x_first - max(y0, 1). Planes are chunked from z = 0 so every
    // segment starts on an even plane (plane 0 itself has no interior output).
@@ -454,6 +437,28 @@ MeshCtx::~MeshCtx()
    (void) hipFree( cellFaces );
    (void) hipFree( entries );
    (void) hipFree( cellInfo );
+}
+
+// Segments of the variable-coefficient sweep: rows y .. y+kElemRows-1, points x0 .. x0+61, planes z0 .. z1-1 of the closed cell.
+void MeshCtx::buildElemSegs( int L )
+{
+   LevelGeom& g = geom( L );
+   if ( g.eSegs )
+      return;
+   const int   N = 1 << L;
+   const char* ec = std::getenv( "HYG_ZCHUNK" );
+   i64         steps = 0;
+   for ( int y = 0; y <= N; y += kElemRows )
+      for ( int x0 = 0; x0 <= N - y; x0 += 62 )
+         steps += N - y - x0 + 1;
+   const int most  = int( std::max< i64 >( kZSegLeast, std::min< i64 >( kZSegChunk, steps * mesh->nC() / kElemWaves ) ) );
+   const int chunk = ec ? std::max( 2, std::min( 1024, std::atoi( ec ) ) ) : most;
+   for ( int z0 = 0; z0 <= N; z0 += chunk )
+      for ( int x0 = 0; x0 <= N - z0; x0 += 62 )
+         for ( int y = 0; y + x0 + z0 <= N; y += kElemRows )
+            g.eSegsHost.push_back( { y, x0, z0, std::min( z0 + chunk, N - y - x0 + 1 ) } );
+   g.nESegs = (int) g.eSegsHost.size();
+   g.eSegs  = upload( g.eSegsHost );
 }
 
 // Assemble the per-level stencil tables of the constant P1 Laplace operator.
@@ -566,6 +571,7 @@ void assembleP1DivKGrad( hyg_op_s& op )
       op.kPoly = upload( op.kPolyHost );
    for ( int L = op.minL; L <= op.maxL; ++L )
    {
+      op.mesh->ctx.buildElemSegs( L );
       hyg_op_s::Level& ol = op.levels[L];
       const int        N  = 1 << L;
       std::vector< ElemCell > ec( m.nC() );

@@ -78,6 +78,15 @@ __device__ __forceinline__ void storeStream( T* p, T v )
    __builtin_nontemporal_store( v, p );
 }
 
+// a pointer that is the same in every lane, in scalar registers (constant memory)
+template < typename T >
+__device__ __forceinline__ const __attribute__( ( address_space( 4 ) ) ) T* uniformPtr( const T* p )
+{
+   const uint64_t v = reinterpret_cast< uint64_t >( p );
+   const uint32_t lo = __builtin_amdgcn_readfirstlane( uint32_t( v ) ), hi = __builtin_amdgcn_readfirstlane( uint32_t( v >> 32 ) );
+   return (const __attribute__( ( address_space( 4 ) ) ) T*) ( ( uint64_t( hi ) << 32 ) | lo );
+}
+
 // ------------------------------------------------------------------ single-lane moves
 // returns `old` with lane `dst` replaced by lane `src` of v (src, dst wave-uniform)
 __device__ __forceinline__ double moveLane( double v, int src, int dst, double old )

@@ -15,35 +15,30 @@ struct PlaneRows
    T e[R][P];
 };
 
-// directions without an x shift and with x+1 (E group)
-constexpr int kDirU[7] = { 0, 3, 4, 7, 9, 11, 12 };
-constexpr int kDirE[4] = { 2, 6, 10, 13 };
-
 // one row of a stencil sweep: the 7 unshifted, 4 x-1 (W, NW, TW, BNW) and 4 x+1 (E, SE, TSE, BE)
-// terms for the P points of a lane; wu / we are the per-lane weights of the first point's
-// unshifted terms and of the E-group terms formed for the first point (see cellZ).
+// terms for the P points of a lane, with wave-uniform weights.
 template < typename T, int P >
-__device__ __forceinline__ void stencilRow( const T* w, const T* wu, const T* we, const T ( &bc )[P], const T ( &bn )[P],
+__device__ __forceinline__ void stencilRow( const T* w, const T ( &bc )[P], const T ( &bn )[P],
                                             const T ( &bs )[P], const T ( &cc )[P], const T ( &cs )[P], const T ( &ac )[P],
                                             const T ( &an )[P], T ( &ax )[P] )
 {
    if constexpr ( P == 1 )
    {
-      T a = wu[0] * bc[0];
-      a += wu[1] * bn[0];
-      a += wu[2] * bs[0];
-      a += wu[3] * cc[0];
-      a += wu[4] * cs[0];
-      a += wu[5] * ac[0];
-      a += wu[6] * an[0];
+      T a = w[0] * bc[0];
+      a += w[3] * bn[0];
+      a += w[4] * bs[0];
+      a += w[7] * cc[0];
+      a += w[9] * cs[0];
+      a += w[11] * ac[0];
+      a += w[12] * an[0];
       T sr = w[1] * bc[0];
       sr += w[5] * bn[0];
       sr += w[8] * cc[0];
       sr += w[14] * an[0];
-      T sl = we[0] * bc[0];
-      sl += we[1] * bs[0];
-      sl += we[2] * cs[0];
-      sl += we[3] * ac[0];
+      T sl = w[2] * bc[0];
+      sl += w[6] * bs[0];
+      sl += w[10] * cs[0];
+      sl += w[13] * ac[0];
       a += laneMove< kDppWaveShr1 >( sr );
       a += laneMove< kDppWaveShl1 >( sl );
       ax[0] = a;
@@ -52,17 +47,17 @@ __device__ __forceinline__ void stencilRow( const T* w, const T* wu, const T* we
    {
       // point 0: x-1 is point 1 of lane-1 (shifted), x+1 is point 1 of this lane;
       // point 1: x-1 is point 0 of this lane, x+1 is point 0 of lane+1 (shifted)
-      T a0 = wu[0] * bc[0];
-      a0 += wu[1] * bn[0];
-      a0 += wu[2] * bs[0];
-      a0 += wu[3] * cc[0];
-      a0 += wu[4] * cs[0];
-      a0 += wu[5] * ac[0];
-      a0 += wu[6] * an[0];
-      a0 += we[0] * bc[1];
-      a0 += we[1] * bs[1];
-      a0 += we[2] * cs[1];
-      a0 += we[3] * ac[1];
+      T a0 = w[0] * bc[0];
+      a0 += w[3] * bn[0];
+      a0 += w[4] * bs[0];
+      a0 += w[7] * cc[0];
+      a0 += w[9] * cs[0];
+      a0 += w[11] * ac[0];
+      a0 += w[12] * an[0];
+      a0 += w[2] * bc[1];
+      a0 += w[6] * bs[1];
+      a0 += w[10] * cs[1];
+      a0 += w[13] * ac[1];
       T a1 = w[0] * bc[1];
       a1 += w[3] * bn[1];
       a1 += w[4] * bs[1];
@@ -137,38 +132,28 @@ __device__ __forceinline__ void cellZ( int bid, const ZSeg* __restrict__ segs, i
       sb                 = ( ci.colour[0] * ( N % sorM ) ) % sorM;
    }
 
-   // x = 0 face (slot 2): the first point of lane 0 in the windows starting at a row start, with that
-   // face's one-sided weights. Its E-group terms are formed on lane 1 (P = 1, then shifted) or on
-   // lane 0 itself (P = 2), which therefore holds that face's E-group weights.
-   const CellFaceSlot fx   = cfs[4 * c + 2];
-   const bool         onX0 = faces && x0 == 1 && ( fx.bc & flag ) != 0;
-   T                  wu[7], we[4];
-   {
-      const T* wf = entryW + 16 * i64( onX0 ? fx.entry : 0 );
-#pragma unroll
-      for ( int k = 0; k < 7; ++k )
-         wu[k] = ( onX0 && lane == 0u ) ? wf[kDirU[k]] : w[kDirU[k]];
-#pragma unroll
-      for ( int k = 0; k < 4; ++k )
-         we[k] = ( onX0 && lane == ( P == 1 ? 1u : 0u ) ) ? wf[kDirE[k]] : w[kDirE[k]];
-   }
-   // diagonal face (slot 3): the row ends x = N-y-z of rows y0..y0+R-1 inside the output window
+   // The x = 0 face (slot 2) is the first point of lane 0 in the windows starting at a row start, the diagonal face (slot 3)
+   // the row ends x = N-y-z of rows y0..y0+R-1 inside the output window: second and third evaluations of the row with
+   // those faces' one-sided weights, read from the scalar cache where they are used. Per-lane weights for lane 0
+   // and the diagonal's held through the march took 118 vector registers for the FP64 apply instead of 88 (141 instead of 110 for
+   // a Chebyshev step); 24 cells: apply at level 8 400 -> 394 us, V(3,3) cycle from level 7 2.66 -> 2.62 ms.
+   typedef const T __attribute__( ( address_space( 4 ) ) ) CT;
+   const CellFaceSlot fx     = cfs[4 * c + 2];
+   const bool         onX0   = faces && x0 == 1 && ( fx.bc & flag ) != 0;
+   const CT*          wX0    = uniformPtr( entryW + 16 * i64( onX0 ? fx.entry : 0 ) );
    const CellFaceSlot fd     = cfs[4 * c + 3];
    const int          xeHi   = N - y0 - z0, xeLo = N - ( y0 + R - 1 ) - ( z1 - 1 );
    const bool         onDiag = faces && ( fd.bc & flag ) != 0 && xeHi >= x0 && xeLo <= x0 + WO - 1;
-   T                  wd[15], wdu[7], wde[4];
-   {
-      const T* wf = entryW + 16 * i64( onDiag ? fd.entry : 0 );
+   const CT*          wDiag  = uniformPtr( entryW + 16 * i64( onDiag ? fd.entry : 0 ) );
+   auto faceRow = [&]( const CT* q, const T ( &bc )[P], const T ( &bn )[P], const T ( &bs )[P], const T ( &cc )[P], const T ( &cs )[P],
+                       const T ( &ac )[P], const T ( &an )[P], T ( &ax )[P] ) {
+      asm volatile( "" : "+s"( q ) ); // not held through the march
+      T wf[NDIR];
 #pragma unroll
       for ( int d = 0; d < NDIR; ++d )
-         wd[d] = onDiag ? wf[d] : T( 0 );
-#pragma unroll
-      for ( int k = 0; k < 7; ++k )
-         wdu[k] = wd[kDirU[k]];
-#pragma unroll
-      for ( int k = 0; k < 4; ++k )
-         wde[k] = wd[kDirE[k]];
-   }
+         wf[d] = q[d];
+      stencilRow< T, P >( wf, bc, bn, bs, cc, cs, ac, an, ax );
+   };
    T f2v[R], dg[R][P]; // face partial sums gathered over the march
 #pragma unroll
    for ( int r = 0; r < R; ++r )
@@ -241,7 +226,7 @@ __device__ __forceinline__ void cellZ( int bid, const ZSeg* __restrict__ segs, i
          // plane z: C = row r+1, N = row r+2, S = row r; plane z+1: TC = row r+1, TS = row r;
          // plane z-1: BC = row r+1, BN = row r+2
          T ax[P];
-         stencilRow< T, P >( w, wu, we, Bp.r[r + 1], Bp.r[r + 2], Bp.r[r], C.r[r + 1], C.r[r], A.r[r + 1], A.r[r + 2], ax );
+         stencilRow< T, P >( w, Bp.r[r + 1], Bp.r[r + 2], Bp.r[r], C.r[r + 1], C.r[r], A.r[r + 1], A.r[r + 2], ax );
 #pragma unroll
          for ( int k = 0; k < P; ++k )
          {
@@ -256,13 +241,16 @@ __device__ __forceinline__ void cellZ( int bid, const ZSeg* __restrict__ segs, i
                bufStore( o1, r1, so, o * B );
          }
          if ( onX0 ) // the first point of lane 0 is the x = 0 face point of row y0+r, plane z
-            f2v[r] = moveLane( ax[0], 0, z - z0, f2v[r] );
+         {
+            T af[P];
+            faceRow( wX0, Bp.r[r + 1], Bp.r[r + 2], Bp.r[r], C.r[r + 1], C.r[r], A.r[r + 1], A.r[r + 2], af );
+            f2v[r] = moveLane( af[0], 0, z - z0, f2v[r] );
+         }
          const int dEnd = lastD + 1 - r - z; // window offset of the row end
          if ( onDiag && dEnd >= 0 && dEnd < 64 * P ) // (wave-uniform) the row end is in the window
          {
             T ad[P];
-            stencilRow< T, P >( wd, wdu, wde, Bp.r[r + 1], Bp.r[r + 2], Bp.r[r], C.r[r + 1], C.r[r], A.r[r + 1], A.r[r + 2],
-                                ad );
+            faceRow( wDiag, Bp.r[r + 1], Bp.r[r + 2], Bp.r[r], C.r[r + 1], C.r[r], A.r[r + 1], A.r[r + 2], ad );
 #pragma unroll
             for ( int k = 0; k < P; ++k )
                dg[r][k] = d0 + k == dEnd ? ad[k] : dg[r][k];

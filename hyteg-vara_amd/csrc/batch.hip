@@ -148,6 +148,21 @@ __global__ __launch_bounds__( kBlock ) void kBatchElem( const ElemTask< T >* __r
 }
 
 template < typename T, int MODE >
+__global__ __launch_bounds__( kBlock ) void kBatchElemPoints( const ElemTask< T >* __restrict__ tasks, int nTasks, int total )
+{
+   const int vb = int( blockIdx.x );
+   if ( vb >= total )
+      return;
+   const ElemTask< T >& t = tasks[findTask( tasks, nTasks, vb )];
+   const ElemArgs< T >& e = t.el;
+   const int            tA = elemTiles( e.L ), b = remapXcd( vb - t.first, e.nC * tA );
+   if ( b >= e.nC * tA )
+      return;
+   bElemApply< T, MODE, false >( b, e.L, tA, e.stride, e.cells, e.kb, e.cinfo, e.cfs, e.prims, e.entries, e.part, e.lowPart, e.dinv, e.flag, e.x,
+                                 e.in1, e.out0, e.out1, e.a );
+}
+
+template < typename T, int MODE >
 __global__ __launch_bounds__( kBlock ) void kBatchCombine( const CombineTask< T >* __restrict__ tasks, int nTasks, int total )
 {
    for ( int vb = int( blockIdx.x ); vb < total; vb += int( gridDim.x ) )
@@ -245,13 +260,15 @@ template < typename T >
 void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item >& items, int cfg )
 {
    constexpr bool   dbl = std::is_same< T, double >::value;
-   BatchPlan::Step  st{}, el{}, cb{};
+   BatchPlan::Step  st{}, el{}, ep{}, cb{};
    st.phase = BatchPlan::STENCIL;
    st.cfg   = cfg;
-   el.phase = BatchPlan::ELEM;
+   el.phase = ep.phase = BatchPlan::ELEM;
+   el.cfg   = 1; // the march; ep, cfg 0: a thread per point
+   ep.cfg   = 0;
    cb.phase = BatchPlan::COMBINE;
-   st.mode = el.mode = cb.mode = mode;
-   st.dtype = el.dtype = cb.dtype = dbl ? 8 : 4;
+   st.mode = el.mode = ep.mode = cb.mode = mode;
+   st.dtype = el.dtype = ep.dtype = cb.dtype = dbl ? 8 : 4;
    for ( const auto& it : items )
    {
       const MeshCtx&          m  = *it.m;
@@ -293,7 +310,10 @@ void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item 
          const ElemArgs< T >& e = u.el;
          u.kind                 = 1;
          u.el                   = elemArgs< T >( m, g, ol, it.L, c );
-         appendTask( el, u, elemBlocks( e ) );
+         if ( elemMarches( it.L, e.nC, dbl ? 8 : 4 ) )
+            appendTask( el, u, elemBlocks( e ) );
+         else
+            appendTask( ep, u, xcdGrid( e.nC * elemTiles( it.L ) ) );
          f.kind    = 0;
          f.part    = e.part;
          f.primInv = nullptr;
@@ -309,6 +329,7 @@ void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item 
    }
    plan.steps.push_back( std::move( st ) );
    plan.steps.push_back( std::move( el ) );
+   plan.steps.push_back( std::move( ep ) );
    plan.steps.push_back( std::move( cb ) );
 }
 
@@ -436,19 +457,23 @@ void launchStencilMode( const BatchPlan::Step& s, hipStream_t st )
    }
 }
 
+template < typename T, int MODE >
+void launchElemMode( const BatchPlan::Step& s, hipStream_t st )
+{
+   auto kf = s.cfg ? kBatchElem< T, MODE > : kBatchElemPoints< T, MODE >;
+   hipLaunchKernelGGL( kf, dim3( s.total ), dim3( kBlock ), 0, st, (const ElemTask< T >*) s.dev, s.nTasks, s.total );
+}
+
 template < typename T >
 void launchElemStep( const BatchPlan::Step& s, hipStream_t st )
 {
-   const dim3 g( s.total ), b( kBlock );
    switch ( s.mode )
    {
-   case MODE_APPLY: hipLaunchKernelGGL( ( kBatchElem< T, MODE_APPLY > ), g, b, 0, st, (const ElemTask< T >*) s.dev, s.nTasks, s.total ); break;
-   case MODE_RESIDUAL:
-      hipLaunchKernelGGL( ( kBatchElem< T, MODE_RESIDUAL > ), g, b, 0, st, (const ElemTask< T >*) s.dev, s.nTasks, s.total );
-      break;
-   case MODE_JACOBI: hipLaunchKernelGGL( ( kBatchElem< T, MODE_JACOBI > ), g, b, 0, st, (const ElemTask< T >*) s.dev, s.nTasks, s.total ); break;
-   case MODE_CHEB0: hipLaunchKernelGGL( ( kBatchElem< T, MODE_CHEB0 > ), g, b, 0, st, (const ElemTask< T >*) s.dev, s.nTasks, s.total ); break;
-   default: hipLaunchKernelGGL( ( kBatchElem< T, MODE_CHEBK > ), g, b, 0, st, (const ElemTask< T >*) s.dev, s.nTasks, s.total ); break;
+   case MODE_APPLY: launchElemMode< T, MODE_APPLY >( s, st ); break;
+   case MODE_RESIDUAL: launchElemMode< T, MODE_RESIDUAL >( s, st ); break;
+   case MODE_JACOBI: launchElemMode< T, MODE_JACOBI >( s, st ); break;
+   case MODE_CHEB0: launchElemMode< T, MODE_CHEB0 >( s, st ); break;
+   default: launchElemMode< T, MODE_CHEBK >( s, st ); break;
    }
 }
 

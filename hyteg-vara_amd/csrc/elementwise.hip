@@ -167,7 +167,7 @@ static void elemT( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, co
       hipLaunchKernelGGL( ( kElemApply< T, MODE, DIAG, false, true > ), dim3( xcdGrid( nC * tA ) ), dim3( kBlock ), 0, s, L, tA, g.stride,
                           ol.elem, kb, m.cellInfo, m.cellFaces, m.prims, m.entries, part, low, dv, c.flag, x, in1, out0, out1, T( c.a ),
                           nullptr, 0, dbl ? (const T*) ol.bw : (const T*) ol.bwF, nC * tA );
-   else if constexpr ( DIAG )
+   else if ( DIAG || !elemMarches( L, nC, dbl ? 8 : 4 ) )
       hipLaunchKernelGGL( ( kElemApply< T, MODE, DIAG > ), dim3( xcdGrid( nC * tA ) ), dim3( kBlock ), 0, s, L, tA, g.stride, ol.elem, kb,
                           m.cellInfo, m.cellFaces, m.prims, m.entries, part, low, dv, c.flag, x, in1, out0, out1, T( c.a ), nullptr, 0,
                           nullptr, nC * tA );

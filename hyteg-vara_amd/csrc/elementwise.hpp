@@ -189,10 +189,15 @@ __global__ __launch_bounds__( kBlock ) void kKBarPoly( int L, int tilesPerCell, 
 }
 
 // ------------------------------------------------------------------ 2. stencil application per cell
+// entry i of the element matrix of type t in the value type
+typedef const __attribute__( ( address_space( 4 ) ) ) ElemCell ElemCellAt;
+__device__ __forceinline__ double elemK( ElemCellAt* ec, int t, int i, double* ) { return ec->mt[t][i]; }
+__device__ __forceinline__ float  elemK( ElemCellAt* ec, int t, int i, float* ) { return ec->mtF[t][i]; }
+
 // Stencil weights W[d] (C W E N S NW SE TC TW TS TSE BC BN BE BNW) of lattice point (px, py, pz) of a macro-cell
 // from the coefficient integrals kc of its micro-cells (the incident ones that lie in the cell); DIAG: W[0] only.
 template < typename T, bool DIAG >
-__device__ __forceinline__ void elemWeights( const ElemCell& ec, const T* __restrict__ kc, int N, int px, int py, int pz, T W[NDIR] )
+__device__ __forceinline__ void elemWeights( ElemCellAt* ec, const T* __restrict__ kc, int N, int px, int py, int pz, T W[NDIR] )
 {
    // anchors p - o for the eight offsets o in {0,1}^3 (encoded x + 2y + 4z)
    int  aIdx[8], aLen[8];
@@ -218,18 +223,15 @@ __device__ __forceinline__ void elemWeights( const ElemCell& ec, const T* __rest
          const bool ok = aOk[o] && as + kMCMax[t] <= N;
          const T    kv = ok ? kc[t * aLen[o] + aIdx[o]] : T( 0 );
          if constexpr ( DIAG )
-            W[0] += kv * T( ec.mt[t][5 * k] );
+            W[0] += kv * elemK( ec, t, 5 * k, static_cast< T* >( nullptr ) );
          else
 #pragma unroll
             for ( int j = 0; j < 4; ++j )
-               W[kMCDir[t][k][j]] += kv * T( ec.mt[t][4 * k + j] );
+               W[kMCDir[t][k][j]] += kv * elemK( ec, t, 4 * k + j, static_cast< T* >( nullptr ) );
       }
 }
 
 // ------------------------------------------------------------------ 3. the operator, z-marching wavefronts
-__device__ __forceinline__ double elemK( const ElemCell& ec, int t, int i, double* ) { return ec.mt[t][i]; }
-__device__ __forceinline__ float  elemK( const ElemCell& ec, int t, int i, float* ) { return ec.mtF[t][i]; }
-
 // A "down" micro-cell is the point reflection of the "up" cell of its colour (p -> (1,1,1) - p up to a lattice step), so its
 // element matrix holds the same entries: the vertex of type 0, 1 or 2 that vertex v of type 3, 4 or 5 is mapped to.
 constexpr int kMCMirror[3][4] = { { 3, 0, 1, 2 }, { 2, 0, 1, 3 }, { 2, 3, 1, 0 } };
@@ -392,7 +394,7 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
    const CellFaceSlot f2 = p.cfs[4 * c + 2], f3 = p.cfs[4 * c + 3];
    const auto         rp2 = makeRsrc( p.part + i64( f2.block ) * NP * NP, unsigned( NP * NP * B ) );
    const auto         rp3 = makeRsrc( p.part + i64( f3.block ) * NP * NP, unsigned( NP * NP * B ) );
-   const ElemCell&    ec  = p.cells[c];
+   ElemCellAt*        ec  = uniformPtr( p.cells + c );
    T                  K[3][6];
    constexpr int      EA[6] = { 0, 0, 0, 1, 1, 2 }, EB[6] = { 1, 2, 3, 2, 3, 3 };
 #pragma unroll
@@ -658,7 +660,25 @@ int elemBlocks( const ElemArgs< T >& e )
    return xcdGrid( ( ( e.nSegs + 3 ) / 4 ) * e.nC );
 }
 
-// One thread per point of the closed macro-cell, for what is not done by the march above. DIAG: the diagonal entry instead of
+// blocks per cell with a thread per point
+__host__ __device__ constexpr int elemTiles( int L ) { return ( S3i( ( 1 << L ) + 1 ) + kBlock - 1 ) / kBlock; }
+
+// March (kElemSweep) or a thread per point (kElemApply)? The march reads each integral and value about once but fills 62-point
+// windows with rows of at most N + 1 points and walks its planes one after the other; threads gather 24 integrals and 15 values each,
+// most of them from cache, and pack their lanes whatever the length of the rows. Sweep with kept integrals, threads / march, us:
+// level 8, 24 cells FP64 1838 / 1393, FP32 1443 / 759, 6 cells 424 / 361, 365 / 195; level 7, 162 cells 1642 / 1507, 1294 / 819, 24
+// cells 250 / 251, 193 / 122, 6 cells 51 / 64, 49 / 43, 3 cells 32.4 / 38.5, 28.1 / 27.7, 1 cell 14.6 / 17.2, 12.2 / 13.9; level 6, 162
+// cells 234 / 332, 164 / 156, 24 cells 37 / 57, 32 / 39 (eight such problems in a batch 281 / 421, 221 / 226); level 5, 24 cells in a
+// batch of six 34 / 86, 30 / 54; level 4, 960 cells 42 / 172, 40 / 99; level 4, 3 cells 10.0 / 13.7, 10.2 / 13.1. In a batch a problem
+// takes the route that it takes alone, so that its results are the same.
+inline bool elemMarches( int L, int nC, int dtype )
+{
+   if ( dtype == 4 )
+      return L >= 8 || ( L == 7 && nC >= 3 ) || ( L == 6 && nC >= 100 );
+   return L >= 8 || ( L == 7 && nC >= 64 );
+}
+
+// One thread per point of the closed macro-cell. DIAG: the diagonal entry instead of
 // the product. BND: the points on the cell's faces, edges and vertices only, listed in bnd[0 .. nBnd) by their index in the
 // cell array (the surrogate operator does the interior points itself). STW: the point's stencil weights are read from wst
 // ([cell][direction][point], the blended operator) instead of assembled from the coefficient integrals.
@@ -699,7 +719,7 @@ __device__ __forceinline__ void bElemApply( int bid, int L, int tilesPerCell, i6
          W[d] = ( DIAG && d > 0 ) ? T( 0 ) : wc[i64( d ) * S3i( w )];
    }
    else
-      elemWeights< T, DIAG >( cells[c], kb + i64( c ) * 6 * S3i( N ), N, px, py, pz, W );
+      elemWeights< T, DIAG >( uniformPtr( cells + c ), kb + i64( c ) * 6 * S3i( N ), N, px, py, pz, W );
    const i64 q = i64( c ) * stride + cidx( w, px, py, pz );
    T         val;
    if constexpr ( DIAG )
@@ -710,9 +730,22 @@ __device__ __forceinline__ void bElemApply( int bid, int L, int tilesPerCell, i6
       const int tc = T2i( Wz ) - py, bc = T2i( Wz + 1 ) - py, nn = Wz - py;
       const int off[NDIR] = { 0, -1, 1, nn, -( nn + 1 ), nn - 1, -nn, tc, tc - 1, tc - nn, tc - nn + 1, -bc, -bc + nn + 1, -bc + 1, -bc + nn };
       val = T( 0 );
+      if constexpr ( STW )
+      {
 #pragma unroll
-      for ( int d = 0; d < NDIR; ++d )
-         val += W[d] * x[q + ( W[d] != T( 0 ) ? off[d] : 0 )];
+         for ( int d = 0; d < NDIR; ++d )
+            val += W[d] * x[q + ( W[d] != T( 0 ) ? off[d] : 0 )];
+      }
+      else
+      {
+         // The rows of the element matrices sum to zero: differences to the point, which lose less in FP32 than the weights'
+         // sum (error of a V-cycle of twelve problems against FP64 1.2e-7 instead of 3.0e-7) and need no centre weight. A direction of
+         // weight 0 is not looked at.
+         const T x0 = x[q];
+#pragma unroll
+         for ( int d = 1; d < NDIR; ++d )
+            val += W[d] * ( x[q + ( W[d] != T( 0 ) ? off[d] : 0 )] - x0 );
+      }
    }
    if ( slot == 0 )
    {

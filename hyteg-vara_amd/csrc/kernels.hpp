@@ -138,7 +138,7 @@ struct BatchPlan
    struct Step
    {
       int                 phase = 0, mode = 0, dtype = 8, nTasks = 0, total = 0;
-      int                 cfg   = 1; // sweep steps: cell-interior configuration (index of kCellRows / kCellDepth)
+      int                 cfg   = 1; // sweep steps: cell-interior configuration (index of kCellRows / kCellDepth); ELEM: 1 march, 0 thread per point
       std::vector< char > host;
       void*               dev = nullptr;
    };

@@ -55,7 +55,7 @@ __global__ __launch_bounds__( kBlock ) void kSurSample( int L, int nPts, int til
       return;
    const int N = 1 << L;
    double    W[NDIR];
-   elemWeights< double, false >( cells[c], kb + i64( c ) * 6 * S3i( N ), N, pts[3 * s], pts[3 * s + 1], pts[3 * s + 2], W );
+   elemWeights< double, false >( uniformPtr( cells + c ), kb + i64( c ) * 6 * S3i( N ), N, pts[3 * s], pts[3 * s + 1], pts[3 * s + 2], W );
    double* o = out + ( i64( c ) * nPts + s ) * NDIR;
 #pragma unroll
    for ( int d = 0; d < NDIR; ++d )

@@ -1,0 +1,66 @@
+"""What a rule of the dispatch must not cost: times of one call against another of the same run on the same device, so that no
+absolute figure is pinned. Every bound lies between the ratio measured with the rule and that of the one kernel for all sizes
+it replaced (both are given), and numbers of launches are counted in a captured graph."""
+import ctypes as C
+import os
+import time
+
+import pytest
+
+import oracle_lib as ol
+
+pytestmark = pytest.mark.gpu
+HIP = C.CDLL("libamdhip64.so")
+
+
+def us(call):
+    """Microseconds per call: the fastest of eight runs of about 10 ms."""
+    def run(n):
+        t0 = time.perf_counter()
+        for _ in range(n):
+            call()
+        HIP.hipDeviceSynchronize()
+        return (time.perf_counter() - t0) / n
+    run(2)
+    n = max(3, min(500, int(0.01 / max(run(3), 1e-7))))
+    return 1e6 * min(run(n) for _ in range(8))
+
+
+def shell(hyg, ntan):
+    return hyg.Mesh("shell", ntan, 2, 0.55, 1.0)
+
+
+def cell_points(mesh, L):
+    w = (1 << L) + 1
+    return int(mesh.info()[3]) * w * (w + 1) * (w + 2) // 6
+
+
+def apply_us(hyg, mesh, L, dt, modes, stored):
+    op = hyg.P1DivKGradOperator(mesh, L, L, 1.0, modes)
+    if stored:
+        op.store_local_matrices()
+    x, y = hyg.Function(mesh, L, L, dt), hyg.Function(mesh, L, L, dt)
+    t = us(lambda: op.apply(x, y, L))
+    print(L, dt, len(modes), stored, "%.1f us" % t, flush=True)
+    return t
+
+
+@pytest.mark.parametrize("dtype", ["F64", "F32"])
+def test_variable_coefficient_on_many_small_cells(hyg, dtype):
+    """960 cells at level 4 (rows of 17 points) against 24 cells at level 6, about as many points: 1.4 to 1.6 times the time per point with a
+    thread per point, 3 to 4 times with the march of 62-point windows; a batch of eight small shells 3 and 10 times."""
+    dt = getattr(hyg, dtype)
+    modes = ol.random_field(33, modes=8, kmax=3)
+    cube, big, small = hyg.Mesh("cube_24el.msh"), shell(hyg, 5), shell(hyg, 3)
+    ref = apply_us(hyg, cube, 6, dt, modes, True) / cell_points(cube, 6)
+    assert apply_us(hyg, big, 4, dt, modes, True) / cell_points(big, 4) <= 2.2 * ref
+    gs, xs, bs, ops = [], [], [], []
+    for _ in range(8):
+        op = hyg.P1DivKGradOperator(small, 0, 3, 1.0, modes)
+        op.store_local_matrices()
+        ops.append(op)
+        gs.append(hyg.GMG(op, 0, 3, dt))
+        xs.append(hyg.Function(small, 0, 3, dt))
+        bs.append(hyg.Function(small, 0, 3, dt))
+    batch = hyg.Batch(gs, xs, bs)
+    assert us(lambda: batch.apply(xs, bs)) / (8 * cell_points(small, 3)) <= 5.0 * ref

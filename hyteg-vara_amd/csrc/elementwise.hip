@@ -23,8 +23,9 @@
 namespace hyg {
 
 // ------------------------------------------------------------------ coefficient tables
-// Tables of one level, built once. axis[((c 3 + axis) N + n) MP + m]: e^(i phase) of mode m at n lattice steps along an axis
-// (axis 0: with the phase at the cell's vertex 0), MP modes with zeros behind the nModes given; mat: the matrix of kKBar in
+// Tables of one level, built once. axis[c 3 N MP + b N MP + ..]: e^(i phase) of mode m at n lattice steps along axis b
+// (axis 0: with the phase at the cell's vertex 0), at m N + n for axis 0 (lanes take consecutive n) and n MP + m for axes 1 and 2
+// (lanes take the same n, modes follow each other); MP modes with zeros behind the nModes given; mat: the matrix of kKBar in
 // the order in which its lanes hold it (step, tile, lane). Phases are reduced in turns before the sine is taken.
 template < typename T >
 __device__ void kbMatrix( const ElemCell& ec, const double* __restrict__ modes, int nModes, int i, T* __restrict__ mat )
@@ -63,7 +64,7 @@ __global__ __launch_bounds__( kBlock ) void kKBarTables( const ElemCell* __restr
    const int       i0 = int( blockIdx.y ) * kBlock + int( threadIdx.x ), step = int( gridDim.y ) * kBlock;
    for ( int i = i0; i < 3 * N * MP; i += step )
    {
-      const int m = i % MP, n = ( i / MP ) % N, b = i / ( MP * N );
+      const int b = i / ( MP * N ), r = i - b * MP * N, m = b == 0 ? r / N : r % MP, n = b == 0 ? r % N : r / MP;
       double    cs = 0.0, sn = 0.0;
       if ( m < nModes )
       {
@@ -85,6 +86,23 @@ __global__ __launch_bounds__( kBlock ) void kKBarTables( const ElemCell* __restr
 }
 
 // ------------------------------------------------------------------ launch
+// Coefficient integrals by matrix products (kKBar) or a thread per anchor (kKBarPoint)? The products are paid for 8, 32 or 64 modes
+// and for tiles of 16 anchors of a row, a thread for the modes there are, one after the other. Apply with n modes, thread / products,
+// us. Long rows, level 7 on 24 cells: FP32 n = 24 592 / 632, 28 652 / 634, 32 713 / 634, 64 1206 / 1579 (6 cells 168 / 189, 183 / 189,
+// 199 / 189); FP64 32 1103 / 1232, 16 788 / 1225. Shorter rows: level 6 on 24 cells FP32 32 125 / 131, level 5 on 240 cells FP64 32
+// 226 / 338, level 4 on 960 cells 174 / 312. Few anchors, where a thread's chain of modes is the whole time, FP64: level 3 on 24 cells
+// n = 4 17.7 / 17.0, 12 20.5 / 20.0, 24 24.7 / 19.9, 64 39.1 / 25.9; level 4 on 24 cells 24 26.0 / 26.7, 32 28.9 / 26.8; level 4 on 48
+// cells 32 29.5 / 31.5; level 3 on 162 cells 32 29.1 / 33.6; level 2 on 162 cells 24 26.1 / 23.1, 33 29.6 / 39.7.
+static bool kbOnMatrixCores( int n, int L, int nC, int dtype )
+{
+   if ( L >= 7 )
+      return dtype == 4 && n > 26 && n <= 32;
+   const i64 rows = ( i64( nC ) << L ) * ( ( 1 << L ) + 1 ) / 2; // of anchors
+   if ( L == 4 )
+      return rows <= 3300 && n > 24 && n <= 32;
+   return L <= 3 && n >= 3 && ( n <= 8 || n > 12 || L <= 2 ) && rows <= ( n <= 32 ? 1800 : 900 );
+}
+
 template < typename T >
 static void launchKBar( const hyg_op_s& op, int L, int nC, T* kb, hipStream_t s )
 {
@@ -97,11 +115,18 @@ static void launchKBar( const hyg_op_s& op, int L, int nC, T* kb, hipStream_t s 
       hipLaunchKernelGGL( ( kKBarPoly< T > ), dim3( nC * tK ), dim3( kBlock ), 0, s, L, tK, ol.elem, op.kPoly, op.kPolyDeg, kb );
       return;
    }
-   const int   rows   = nC * N * ceilDiv( N, kKBarRows ) >= 2048 ? kKBarRows : 16; // 2048: four blocks per CU and half of them empty
-   const int   chunks = ceilDiv( N, rows );
-   const auto* axis   = static_cast< const KbPair< T >* >( dbl ? ol.kbAxis : ol.kbAxisF );
-   const T*    mat    = dbl ? (const T*) ol.kbMat : (const T*) ol.kbMatF;
-   auto        kf     = kKBar< T, 32 >;
+   const auto* axis = static_cast< const KbPair< T >* >( dbl ? ol.kbAxis : ol.kbAxisF );
+   const T*    mat  = dbl ? (const T*) ol.kbMat : (const T*) ol.kbMatF;
+   if ( !kbOnMatrixCores( op.nModes, L, nC, dbl ? 8 : 4 ) )
+   {
+      const int tK = ceilDiv( S3i( N ), kBlock );
+      hipLaunchKernelGGL( ( kKBarPoint< T > ), dim3( nC * tK ), dim3( kBlock ), 0, s, N, tK, op.nModes, kbModes( op.nModes ), axis, mat,
+                          T( op.k0 ), kb );
+      return;
+   }
+   const int rows   = nC * N * ceilDiv( N, kKBarRows ) >= 2048 ? kKBarRows : 16; // 2048: four blocks per CU and half of them empty
+   const int chunks = ceilDiv( N, rows );
+   auto      kf     = kKBar< T, 32 >;
    switch ( kbModes( op.nModes ) )
    {
    case 8: kf = kKBar< T, 4 >; break;

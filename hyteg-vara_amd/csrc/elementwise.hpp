@@ -49,6 +49,9 @@ __device__ __forceinline__ f32x4 mma16( float a, float b, f32x4 c ) { return __b
 // lane group and slot within its tile of row i of a 16 x 16 result: FP64 results lie 4 rows apart, FP32 ones in sequence
 __device__ __forceinline__ void mmaRow( int i, int& g, int& r, double* ) { g = i & 3, r = i >> 2; }
 __device__ __forceinline__ void mmaRow( int i, int& g, int& r, float* ) { g = i >> 2, r = i & 3; }
+// and the other way round
+constexpr int mmaRowOf( int g, int r, double* ) { return 4 * r + g; }
+constexpr int mmaRowOf( int g, int r, float* ) { return 4 * g + r; }
 
 template < typename T >
 struct KbPair
@@ -89,7 +92,7 @@ __global__ __launch_bounds__( kBlock, S > 16 ? 1 : ( sizeof( T ) == 8 ? 2 : 3 ) 
 #pragma unroll
       for ( int s = 0; s < S; ++s )
       {
-         const KbPair< T > X = ax[min( x, N - 1 ) * MP + 2 * s + h], Z = ax[( 2 * N + z ) * MP + 2 * s + h];
+         const KbPair< T > X = ax[( 2 * s + h ) * N + min( x, N - 1 )], Z = ax[( 2 * N + z ) * MP + 2 * s + h];
          const T           re = X.re * Z.re - X.im * Z.im, im = X.re * Z.im + X.im * Z.re;
          a[s] = ( g & 1 ) ? im : re; // (X Z Y)'s real or imaginary part = a Y.re + d Y.im
          d[s] = ( g & 1 ) ? re : -im;
@@ -127,6 +130,55 @@ __global__ __launch_bounds__( kBlock, S > 16 ? 1 : ( sizeof( T ) == 8 ? 2 : 3 ) 
    }
 }
 static_assert( kMCMax[1] == kMCMax[2] && kMCMax[4] == kMCMax[5], "types handled alike by kKBar" );
+
+// The same integrals with a thread per anchor (consecutive anchors of the cell, whatever their rows), the matrix read with scalar
+// loads: per mode three table values, two complex products and 60 multiply-adds.
+template < typename T >
+__global__ __launch_bounds__( kBlock ) void kKBarPoint( int N, int tilesPerCell, int nModes, int MP, const KbPair< T >* __restrict__ axis,
+                                                        const T* __restrict__ mat, T k0, T* __restrict__ kb )
+{
+   typedef const T __attribute__( ( address_space( 4 ) ) ) CT;
+   const int c    = int( blockIdx.x ) / tilesPerCell;
+   const int s    = ( int( blockIdx.x ) - c * tilesPerCell ) * kBlock + int( threadIdx.x );
+   if ( s >= S3i( N ) )
+      return;
+   int x, y, z;
+   tetXYZ( N, s, x, y, z );
+   const KbPair< T >* ax = axis + i64( c ) * 3 * N * MP;
+   const CT*          mc = (const CT*) ( mat + i64( c ) * MP * 64 );
+   T                  g[30];
+#pragma unroll
+   for ( int k = 0; k < 30; ++k )
+      g[k] = T( 0 );
+   for ( int m = 0; m < nModes; ++m )
+   {
+      const KbPair< T > X = ax[m * N + x], Y = ax[( N + y ) * MP + m], Z = ax[( 2 * N + z ) * MP + m];
+      const T           re = X.re * Z.re - X.im * Z.im, im = X.re * Z.im + X.im * Z.re;
+      const T           cs = re * Y.re - im * Y.im, sn = re * Y.im + im * Y.re;
+      const CT*         a = mc + ( m >> 1 ) * 128 + ( m & 1 ) * 32;
+#pragma unroll
+      for ( int t = 0; t < 6; ++t )
+#pragma unroll
+         for ( int q = 0; q < 5; ++q )
+         {
+            // where kKBar holds point q of type t: group and slot
+            const int gr = t < 4 ? t : 2 * ( t - 4 ) + ( q < 3 ? 0 : 1 ), j = t < 4 ? q : ( q < 3 ? q + 5 : q + 2 );
+            const int o  = 64 * ( j >> 2 ) + mmaRowOf( gr, j & 3, static_cast< T* >( nullptr ) );
+            g[5 * t + q] = fma( cs, a[o], fma( sn, a[o + 16], g[5 * t + q] ) );
+         }
+   }
+   const int nx = N - y - z;
+   T*        o  = kb + i64( c ) * 6 * S3i( N ) + kbRow( N, y, z ) + x;
+#pragma unroll
+   for ( int t = 0; t < 6; ++t )
+   {
+      T v = T( 0 );
+#pragma unroll
+      for ( int q = 0; q < 5; ++q )
+         v += T( kQW6[q] ) * expT( g[5 * t + q] );
+      o[t * nx] = x + kMCMax[t] <= nx ? k0 * v : T( 0 ); // 0: the element is not in the cell
+   }
+}
 
 // The same integrals for a polynomial coefficient k(x) = sum_i poly[i] x^a y^b z^c over the monomials of degree <= deg
 // in the order of the reference's MonomialBasis3D (by total degree; within a degree by decreasing a, then b). One

@@ -64,3 +64,24 @@ def test_variable_coefficient_on_many_small_cells(hyg, dtype):
         bs.append(hyg.Function(small, 0, 3, dt))
     batch = hyg.Batch(gs, xs, bs)
     assert us(lambda: batch.apply(xs, bs)) / (8 * cell_points(small, 3)) <= 5.0 * ref
+
+
+@pytest.mark.parametrize("dtype", ["F64", "F32"])
+def test_coefficient_integrals_cost_the_modes_there_are(hyg, dtype):
+    """Padded to 32 or 64 modes, 12 modes take as long as 32 and 33 over twice as long; taken one by one 0.7 and 1.0 times."""
+    dt = getattr(hyg, dtype)
+    cube = hyg.Mesh("cube_24el.msh")
+    t = {n: apply_us(hyg, cube, 6, dt, ol.random_field(33, modes=n, kmax=8), False) for n in (12, 32, 33)}
+    assert t[12] <= 0.85 * t[32]
+    assert t[33] <= 1.3 * t[32]
+
+
+@pytest.mark.parametrize("dtype", ["F64", "F32"])
+def test_coefficient_integrals_on_many_small_cells(hyg, dtype):
+    """Tiles of 16 anchors of a row are mostly empty on rows of at most 16: 3 times the time per anchor of 24 cells at level 6, against
+    1.5 times with a thread per anchor."""
+    dt = getattr(hyg, dtype)
+    modes = ol.random_field(33, modes=32, kmax=8)
+    cube, big = hyg.Mesh("cube_24el.msh"), shell(hyg, 5)
+    ref = apply_us(hyg, cube, 6, dt, modes, False) / cell_points(cube, 6)
+    assert apply_us(hyg, big, 4, dt, modes, False) / cell_points(big, 4) <= 2.2 * ref

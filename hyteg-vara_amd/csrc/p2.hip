@@ -1184,7 +1184,8 @@ static void p2Variable( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int 
    const i64              kqs = p2KqStride( m, L ), ps = p2PartStride( m, L ), ls = p2LowStride( m, L );
    const int              flag = cs[0].flag;
    const P2Comps< T >     cp   = p2Comps< T >( cs, n );
-   if ( ol.p2s )
+   // a lattice of two intervals per edge has points on cell edges only
+   if ( N > 2 && ol.p2s )
    {
       // stored stencils
       const T*           sw = dbl ? (const T*) ol.p2s : (const T*) ol.p2sF;
@@ -1193,7 +1194,7 @@ static void p2Variable( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int 
       hipLaunchKernelGGL( kf, dim3( xcdGrid( nC * ct.start[8] ) ), dim3( kBlock ), 0, s, L, g.stride, ct, sw, cp, T( cs[0].a ), m.cellFaces, flag,
                           part, ps, nC );
    }
-   else
+   else if ( N > 2 )
       launchP2KQPoints< T >( L, nC, g.stride, el, kq, kqs, dv, cp, n, MODE, T( cs[0].a ), m.cellFaces, flag, part, ps, s );
    const int tB = ceilDiv( i64( p2EdgeVertexCount( N ) ) * kP2EvLanes, kBlock );
    hipLaunchKernelGGL( ( kP2KEdge< T > ), dim3( nC * tB ), dim3( kBlock ), 0, s, L, tB, g.stride, el, kq, kqs, m.p2tab, m.cellInfo, m.prims,

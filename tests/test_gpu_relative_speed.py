@@ -85,3 +85,27 @@ def test_coefficient_integrals_on_many_small_cells(hyg, dtype):
     cube, big = hyg.Mesh("cube_24el.msh"), shell(hyg, 5)
     ref = apply_us(hyg, cube, 6, dt, modes, False) / cell_points(cube, 6)
     assert apply_us(hyg, big, 4, dt, modes, False) / cell_points(big, 4) <= 2.2 * ref
+
+
+def launches(hyg, stream, op, x, y, L):
+    call = lambda: hyg.check(hyg.load().hyg_apply(op.h, x.h, y.h, L, hyg.INNER, hyg.REPLACE, stream))
+    call()
+    assert HIP.hipStreamSynchronize(stream) == 0
+    graph, n = C.c_void_p(), C.c_size_t()
+    assert HIP.hipStreamBeginCapture(stream, 1) == 0
+    call()
+    assert HIP.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert HIP.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+    HIP.hipGraphDestroy(graph)
+    return n.value
+
+
+@pytest.mark.parametrize("stored", [False, True])
+def test_variable_p2_level_0_has_no_launch_without_points(hyg, hip_stream, stored):
+    """Two intervals per cell edge: all points lie on cell edges (one launch) and are then combined (another)."""
+    mesh = hyg.Mesh("three_tets_with_two_joint_faces.msh")
+    op = hyg.P2DivKGradOperator(mesh, 0, 0, kind=1)
+    if stored:
+        op.store_local_matrices()
+    x, y = hyg.Function(mesh, 0, 0, space="p2"), hyg.Function(mesh, 0, 0, space="p2")
+    assert launches(hyg, hip_stream, op, x, y, 0) == 2

@@ -20,7 +20,7 @@
 // faces are whole planes/rows and are computed by faceFlat with coalesced loads. kFaceCombine adds
 // the partial sums of the two sides, applies the epilogue and writes every replica.
 //
-// Macro-edges and -vertices, and the face points of levels up to kDirectFaceLevel (lower): the lanes of a
+// Macro-edges and -vertices, and the face points where directFaces says so (lower): the lanes of a
 // point share its incident cells and gather their one-sided stencils.
 
 #include "sweep.hpp"
@@ -55,7 +55,7 @@ static void stencilT( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol,
    T*             out1 = (T*) c.out1;
    // 1. cell interiors with the one-sided sums of the x = 0 and diagonal faces, the one-sided sums
    // of the z = 0 and y = 0 faces, and macro-edges and -vertices: one launch
-   const int nFace = directFaces( g ) ? 0 : g.nChunks - g.firstFaceChunk;
+   const int nFace = directFaces( m, g ) ? 0 : g.nChunks - g.firstFaceChunk;
    SweepArgs< T > p = sweepArgs< T >( m, g, ol, L, c, cfg );
    const int      nLow = p.nChunks;
    const int gL = nLow > 0 ? xcdGrid( ceilDiv( nLow, kBlock / 64 ) ) : 0;

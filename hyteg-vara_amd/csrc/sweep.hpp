@@ -477,20 +477,26 @@ struct SweepArgs
    int                 faces = 1;
 };
 
-// Up to level 6 the face points are gathered from both cells in the sweep launch itself, like the edge points: two stencils
-// of scattered loads per point against a second launch (kFaceCombine, 4 us where it has next to nothing to do). One sweep
-// of 6 cells at level 5: 8.4 us with the second launch, 4.5 us without. A Chebyshev V-cycle from level 7 on 24 cells:
-// 2.89 ms with the line at level 4, 2.80 at 5, 2.73 at 6, 2.84 at 7; an apply at level 8 takes 0.40 ms with one-sided
-// sums and 0.50 ms with gathers, whose lines on the x = 0 and diagonal faces are fetched for one value each.
-constexpr int kDirectFaceLevel = 6;
-inline bool   directFaces( const LevelGeom& g ) { return g.L <= kDirectFaceLevel; }
+// Where face points are done. Gathered from both cells in the sweep launch itself, like the edge points, they cost two
+// stencils of scattered loads per point; as one-sided sums of the cells they cost a second launch (kFaceCombine, 4 us where it has
+// next to nothing to do). Gathered / summed, us: level 5, apply of 6 cells FP64 4.0 / 8.6, residual of 960 cells FP32 83 / 100;
+// level 6, residual of 6 cells FP64 8.4 / 11.9, of 24 cells FP32 18.1 / 17.2, FP64 apply 21.6 / 20.9, of 162 cells FP32 67 / 59, of
+// 960 cells FP32 495 / 354, FP64 791 / 642; level 7, 6 cells FP32 17.0 / 17.6, 8 cells 26.6 / 22.0, 24 cells 68 / 47. Rows of up to
+// 32 points share their lines with few others, so there the gather always wins; beyond, it loses once the cells have more face
+// points than the launch costs (24 cells at level 6: a Chebyshev V-cycle from level 7 takes 2.73 ms with gathers there, 2.80
+// with sums).
+constexpr i64 kDirectFacePoints = 200000;
+inline bool   directFaces( const MeshCtx& m, const LevelGeom& g )
+{
+   return g.L <= 5 || ( i64( 2 * m.mesh->nC() ) << ( 2 * g.L ) ) <= kDirectFacePoints;
+}
 
 // arguments of the sweep of one level of the constant operator
 template < typename T >
 SweepArgs< T > sweepArgs( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::Level& ol, int L, const StencilCall& c, int cfg )
 {
    constexpr bool dbl    = std::is_same< T, double >::value;
-   const bool     direct = directFaces( g );
+   const bool     direct = directFaces( m, g );
    SweepArgs< T > p;
    p.segs    = g.zSegs[cfg];
    p.nSegs   = g.nZSegs[cfg];

@@ -117,6 +117,7 @@ struct ZSeg
 // 3.06 / 3.12 ms; 3 and 2 planes are slower again than 4 (4.7 and 4.8 against 4.5 us with the face points in the launch).
 constexpr int kZSegChunk = 24;
 constexpr int kZSegLeast = 4;
+constexpr int kZSegFull  = 8; // level 7, 6 cells (3.6 planes for kZSegWaves): FP64 apply 21.8 us with 4 planes, 19.1 with 8, FP32 15.9, 15.6
 constexpr int kZSegWaves = 8192;
 // The variable-coefficient sweep: one row per wavefront (two rows share more loads and edge differences but halve the waves
 // in flight: 208 against 196 us for an FP32 sweep at level 7), and segments for four times the waves (6 planes at level 7

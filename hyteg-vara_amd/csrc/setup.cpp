@@ -328,12 +328,14 @@ LevelGeom& MeshCtx::geom( int L )
       const int R = kCellRows[k], WO = 64 * kCellPoints[k] - 2;
       auto&     v = g.zSegsHost[k];
       v.clear();
-      // planes per segment: as many as leave kZSegWaves wavefronts on the mesh, at most kZSegChunk
+      // planes per segment: as many as leave kZSegWaves wavefronts on the mesh, at most kZSegChunk, at least kZSegFull where the
+      // shortest segments would nearly give as many
       i64 steps = 0;
       for ( int y = 1; y <= N - 2; y += R )
          for ( int x0 = 1; x0 <= N - 2; x0 += WO )
             steps += std::max( 0, N - y - x0 );
-      const int most  = int( std::max< i64 >( kZSegLeast, std::min< i64 >( kZSegChunk, steps * mesh->nC() / kZSegWaves ) ) );
+      const i64 fill  = steps * mesh->nC() / kZSegWaves;
+      const int most  = int( std::min< i64 >( kZSegChunk, std::max< i64 >( fill < 3 ? kZSegLeast : kZSegFull, fill ) ) );
       const int chunk = ec ? std::max( 2, std::min( 1024, std::atoi( ec ) ) ) : most;
       auto      add = [&]( int y, int x0, int z0 ) {
          const int zEnd = N - y - x0 + 1;

@@ -138,7 +138,7 @@ __global__ __launch_bounds__( kBlock ) void kBatchSweep( const SweepTask< T >* _
 }
 
 template < typename T, int MODE >
-__global__ __launch_bounds__( kBlock ) void kBatchElem( const ElemTask< T >* __restrict__ tasks, int nTasks, int total )
+__global__ __launch_bounds__( kBlock, kElemOccupancy< T > ) void kBatchElem( const ElemTask< T >* __restrict__ tasks, int nTasks, int total )
 {
    const int vb = int( blockIdx.x );
    if ( vb >= total )

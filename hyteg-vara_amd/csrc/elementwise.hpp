@@ -368,6 +368,54 @@ __device__ __forceinline__ void elemStoreBoundary( int c, int N, int slot, int p
    lowPart[i64( e ) * NP + i] = val;
 }
 
+// The (type, node, node) entries of the element matrices that make up each stencil direction, in the order of elemWeights.
+struct ElemTerms
+{
+   int first[NDIR + 1] = {}, term[96] = {}; // term: type + 8 node + 32 other node
+};
+constexpr ElemTerms elemTermTable()
+{
+   ElemTerms tb;
+   int       n = 0;
+   for ( int d = 0; d < NDIR; ++d )
+   {
+      tb.first[d] = n;
+      for ( int t = 0; t < 6; ++t )
+         for ( int k = 0; k < 4; ++k )
+            for ( int j = 0; j < 4; ++j )
+               if ( kMCDir[t][k][j] == d )
+                  tb.term[n++] = t + 8 * k + 32 * j;
+   }
+   tb.first[NDIR] = n;
+   return tb;
+}
+static __constant__ ElemTerms kElemTerms = elemTermTable();
+
+// The operator's value (the cell's part of it) at one point as elemWeights and bElemApply form it, a direction of weight 0 not
+// looked at: what kElemSweep takes where its sums are not finite. Loops that are not unrolled, for few registers.
+template < typename T >
+__device__ __forceinline__ T elemValue( ElemCellAt* ec, const T* __restrict__ kc, const T* __restrict__ xc, int N, int px, int py, int pz )
+{
+   const T x0  = xc[cidx( N + 1, px, py, pz )];
+   T       val = T( 0 );
+#pragma unroll 1
+   for ( int d = 1; d < NDIR; ++d )
+   {
+      T w = T( 0 );
+#pragma unroll 1
+      for ( int i = kElemTerms.first[d]; i < kElemTerms.first[d + 1]; ++i )
+      {
+         const int e = kElemTerms.term[i], t = e & 7, k = ( e >> 3 ) & 3, j = e >> 5, o = kMCOff[t][k];
+         const int ax = px - ( o & 1 ), ay = py - ( ( o >> 1 ) & 1 ), az = pz - ( ( o >> 2 ) & 1 );
+         if ( ax >= 0 && ay >= 0 && az >= 0 && ax + ay + az + kMCMax[t] <= N )
+            w += kc[kbRow( N, ay, az ) + t * ( N - ay - az ) + ax] * elemK( ec, t, 4 * k + j, static_cast< T* >( nullptr ) );
+      }
+      const bool on = w != T( 0 );
+      val += w * ( xc[cidx( N + 1, px + ( on ? dirX( d ) : 0 ), py + ( on ? dirY( d ) : 0 ), pz + ( on ? dirZ( d ) : 0 ) )] - x0 );
+   }
+   return val;
+}
+
 template < typename T >
 struct ElemArgs
 {
@@ -410,6 +458,8 @@ struct ElemLayer
 // (64 B per point in FP64) where a thread per point gathered 39 values: level 7 on 24 cells (8.4 million points) 314 -> 242
 // us in FP64, FP32 Jacobi sweep 244 -> 140 us. Bound by the vector instructions of a step (180 FP32, of which 105 are the
 // edge products) at 55% of the lanes: rows of a tetrahedron end inside the 62-point windows.
+// A sum of differences turns an infinite value into NaN at points whose weight for it is 0 (and at the point itself): a plane with
+// a sum that is not finite stores nothing and is done again point by point behind the march (planes: one bit each).
 // Lanes outside a row, rows outside a plane and anchors outside the cell load 0 (the descriptor's range check), so they
 // add nothing; elements that stick out of the cell have kb = 0.
 // The arguments are read where they are used (ap, made opaque for the rare boundary rows): held in scalar registers through
@@ -550,6 +600,7 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
       elemStoreBoundary( c, N, classifySlot( N, px, y, z ), px, y, z, val, q->flag, q->cinfo, q->cfs, q->prims, q->entries, q->part,
                          q->lowPart );
    };
+   unsigned again = 0; // planes that are done again
    T vEdge[R] = {}; // values of the rows' points on the edge between local vertices 2 and 3 (x = 0 on the diagonal face)
    // one plane: `cur` holds layer z, `nxt` receives layer z+1; EDGE: the plane or a row of it lies on a face of the cell
    auto step = [&]( auto EDGE, ElemLayer< T, R >& cur, ElemLayer< T, R >& nxt ) {
@@ -579,6 +630,11 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
          const int y = y0 + r, xe = N - y - z; // row end
          if ( xe < x0 )
             continue; // (wave-uniform) nothing of this row in the window
+         if ( __builtin_expect( __ballot( !isfinite( Ax ) ) != 0, 0 ) )
+         {
+            again |= 1u << ( z - z0 );
+            continue;
+         }
          if constexpr ( EDGE.value )
             if ( y == 0 || z == 0 )
             {
@@ -669,10 +725,44 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
          if ( y0 + r > 0 && z > 0 && z >= z0 && z < z1 )
             boundary( y0 + r, vEdge[r] );
       }
+   if ( again != 0 )
+   {
+      ElemArgsAt< T > q = ap;
+      asm volatile( "" : "+s"( q ) );
+      for ( ; again != 0; again &= again - 1 )
+      {
+         z = z0 + __builtin_ctz( again );
+#pragma unroll 1
+         for ( int r = 0; r < R; ++r )
+         {
+            const int y = y0 + r;
+            if ( lane < 1 || lane > 62 || px > N - y - z )
+               continue;
+            const i64 cq  = i64( c ) * q->stride;
+            const T   val = elemValue( uniformPtr( q->cells + c ), q->kb + i64( c ) * 6 * S3i( N ), q->x + cq, N, px, y, z );
+            if ( classifySlot( N, px, y, z ) != 0 )
+               boundary( y, val );
+            else if ( q->flag & 1 )
+            {
+               const i64 o  = cq + cidx( N + 1, px, y, z );
+               const T   e  = kIn1 ? q->in1[o] : ( MODE == MODE_APPLY_ADD ? q->out0[o] : T( 0 ) );
+               T         q0 = T( 0 ), q1 = T( 0 );
+               epilogue< T, MODE >( val, q->x[o], e, e, kD ? q->dinv[o] : T( 0 ), q->a, q0, q1 );
+               q->out0[o] = q0;
+               if constexpr ( kTwo )
+                  q->out1[o] = q1;
+            }
+         }
+      }
+   }
 }
 
+// wavefronts per SIMD
+template < typename T >
+constexpr int kElemOccupancy = sizeof( T ) == 4 ? 6 : 3;
+
 template < typename T, int MODE, int R >
-__global__ __launch_bounds__( kBlock ) void kElemSweep( ElemArgs< T > p )
+__global__ __launch_bounds__( kBlock, kElemOccupancy< T > ) void kElemSweep( ElemArgs< T > p )
 {
    // p is the whole argument segment
    elemSweep< T, MODE, R >( int( blockIdx.x ), (ElemArgsAt< T >) __builtin_amdgcn_kernarg_segment_ptr() );

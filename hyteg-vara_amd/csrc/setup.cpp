@@ -441,7 +441,8 @@ MeshCtx::~MeshCtx()
    (void) hipFree( cellInfo );
 }
 
-// Segments of the variable-coefficient sweep: rows y .. y+kElemRows-1, points x0 .. x0+61, planes z0 .. z1-1 of the closed cell.
+// Segments of the variable-coefficient sweep: rows y .. y+kElemRows-1, points x0 .. x0+61, planes z0 .. z1-1 of the closed cell, at
+// most 32 (the sweep keeps a bit for each).
 void MeshCtx::buildElemSegs( int L )
 {
    LevelGeom& g = geom( L );
@@ -454,7 +455,7 @@ void MeshCtx::buildElemSegs( int L )
       for ( int x0 = 0; x0 <= N - y; x0 += 62 )
          steps += N - y - x0 + 1;
    const int most  = int( std::max< i64 >( kZSegLeast, std::min< i64 >( kZSegChunk, steps * mesh->nC() / kElemWaves ) ) );
-   const int chunk = ec ? std::max( 2, std::min( 1024, std::atoi( ec ) ) ) : most;
+   const int chunk = ec ? std::max( 2, std::min( 32, std::atoi( ec ) ) ) : most;
    for ( int z0 = 0; z0 <= N; z0 += chunk )
       for ( int x0 = 0; x0 <= N - z0; x0 += 62 )
          for ( int y = 0; y + x0 + z0 <= N; y += kElemRows )

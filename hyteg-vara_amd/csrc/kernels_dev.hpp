@@ -376,6 +376,18 @@ __device__ __forceinline__ void bRestrictLower( int bid, const LowerChunk* __res
 #pragma unroll
       for ( int d = 1; d < NDIR; ++d )
          s += T( 0.5 ) * g[d] * f[d];
+      if ( !isfinite( s ) )
+      {
+         // the point itself, read with weight 0 in place of neighbours outside the cell, makes an infinite value NaN: without them
+         s = T( 0 );
+#pragma unroll 1
+         for ( int d = 0; d < NDIR; ++d )
+         {
+            const int ax = 2 * qx + dirX( d ), ay = 2 * qy + dirY( d ), az = 2 * qz + dirZ( d );
+            if ( inCell( Nf, ax, ay, az ) )
+               s += ( d == 0 ? T( 1 ) : T( 0.5 ) ) * T( cf.invNC[classifySlot( Nf, ax, ay, az )] ) * fs[cidx( wf, ax, ay, az )];
+         }
+      }
       v += k0 + cl.sub < ch.nCells ? s : T( 0 );
    }
    v = chunkSum( v, cl );

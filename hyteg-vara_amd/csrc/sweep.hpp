@@ -413,6 +413,15 @@ __device__ __forceinline__ void lower( int bid, const LowerChunk* __restrict__ c
 #pragma unroll
       for ( int d = 0; d < NDIR; ++d )
          s += wv[d] * v[d];
+      if ( !isfinite( s ) )
+      {
+         // directions that lead out of the cell read the point itself with weight 0, which makes an infinite value NaN: without them
+         s = T( 0 );
+#pragma unroll 1
+         for ( int d = 0; d < NDIR; ++d )
+            if ( inCell( N, qx + dirX( d ), qy + dirY( d ), qz + dirZ( d ) ) )
+               s += wv[d] * xs[cidx( w, qx + dirX( d ), qy + dirY( d ), qz + dirZ( d ) )];
+      }
       Ax += k0 + cl.sub < ch.nCells ? s : T( 0 );
    }
    Ax = chunkSum( Ax, cl );

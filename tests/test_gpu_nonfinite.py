@@ -88,3 +88,28 @@ def test_variable_coefficient_residual_and_jacobi_with_infinite_values(hyg, dtyp
         fine = np.isfinite(res[1])
         assert not fine[ks].any() and (~fine).sum() <= 15 * len(ks), what
         assert np.abs(res[1][fine] - res[0][fine]).max() <= 1e-5 * np.abs(res[0]).max(), what
+
+
+@pytest.mark.parametrize("dtype", ["F64", "F32"])
+def test_constant_operator_and_restriction_at_the_point_itself(hyg, dtype):
+    """Lanes of face, edge and vertex points have no neighbours outside a cell; the point's own infinite value stays infinite."""
+    dt, L = getattr(hyg, dtype), 3
+    mesh = hyg.Mesh("cube_kuhn_6el.msh")
+    n, nc = mesh.ndofs(L), mesh.ndofs(L - 1)
+    op = hyg.P1ConstantOperator(mesh, L, L)
+    x, y = hyg.Function(mesh, L, L, dt), hyg.Function(mesh, L, L, dt)
+    r = hyg.Function(mesh, L - 1, L, dt)
+    xyz, _ = mesh.coords(L)
+    cxyz, _ = mesh.coords(L - 1)
+    for k in points(n, 6, 60):
+        v = np.zeros(n)
+        v[k] = np.inf
+        x.upload(L, v)
+        op.apply(x, y, L, hyg.ALL)
+        assert y.download(L)[k] == np.inf
+        r.upload(L, v)
+        r.restrict(L, hyg.ALL)
+        c = np.flatnonzero(np.abs(cxyz - xyz[k]).max(axis=1) < 1e-12)
+        if len(c):
+            assert r.download(L - 1)[c[0]] == np.inf
+    assert nc < n

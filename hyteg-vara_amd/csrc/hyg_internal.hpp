@@ -40,6 +40,18 @@ inline i64 cellStride( int L )
    const i64 w = ( i64( 1 ) << L ) + 1;
    return ( S3( w ) + 63 ) / 64 * 64;
 }
+// A value of a cell's array (N intervals per edge) that is always 0, behind its points: levels are cleared when they are created,
+// kernels write points only, and whole arrays are copied from one another. Read in place of points outside the cell, whose
+// weight is 0: the point itself in their place makes an infinite value NaN.
+__host__ __device__ inline int zeroValue( int N ) { return S3i( N + 1 ); }
+constexpr bool zeroValueFits()
+{
+   for ( i64 w = 2; w <= ( 1 << 12 ) + 1; w = 2 * w - 1 )
+      if ( w * ( w + 1 ) * ( w + 2 ) / 6 % 64 == 0 )
+         return false;
+   return true;
+}
+static_assert( zeroValueFits(), "cell arrays are longer than their points" );
 // values allocated after the last cell array of a level: row-window kernels read up to 128 values
 // past a cell's last point (and discard them)
 constexpr i64 kTailSlack = 256;

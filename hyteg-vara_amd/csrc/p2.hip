@@ -338,6 +338,35 @@ __global__ __launch_bounds__( kBlock ) void kP2KEdge( int L, int tilesPerCell, i
          }
       }
    }
+   // Infinite values: the gradients take differences of them. The sum of weights times values instead.
+   if ( !isfinite( val[0] ) || !isfinite( val[1] ) || !isfinite( val[2] ) )
+   {
+      val[0] = val[1] = val[2] = T( 0 );
+#pragma unroll 1
+      for ( int k = sub; k < ne; k += kP2EvLanes )
+      {
+         const int tl = tb->ent[cls][k], t = tl >> 4, l = tl & 15;
+         const int ax = ( px - tb->nd[t][l][0] ) >> 1, ay = ( py - tb->nd[t][l][1] ) >> 1, az = ( pz - tb->nd[t][l][2] ) >> 1;
+         if ( ax < 0 || ay < 0 || az < 0 || ax + ay + az + kMCMax[t] > Nc )
+            continue;
+         const T* kv = kq + i64( c * 6 + t ) * SA + cidx( Nc + 1, ax, ay, az );
+         T        m[kP2Moments], r[10];
+#pragma unroll
+         for ( int q = 0; q < kP2Moments; ++q )
+            m[q] = kv[i64( q ) * kqStride];
+         p2RowOf( l, m, el + ( c * 6 + t ) * kP2Moments, r );
+#pragma unroll
+         for ( int j = 0; j < 10; ++j )
+         {
+            const i64 o = cb + cidx( w, 2 * ax + tb->nd[t][j][0], 2 * ay + tb->nd[t][j][1], 2 * az + tb->nd[t][j][2] );
+            val[0] += r[j] * cp.x[0][o];
+            if ( nc > 1 )
+               val[1] += r[j] * cp.x[1][o];
+            if ( nc > 2 )
+               val[2] += r[j] * cp.x[2][o];
+         }
+      }
+   }
    const int e = ci.entry[slot];
    int       i = 0;
    if ( slot <= 10 )
@@ -851,6 +880,7 @@ __device__ __forceinline__ void p2StoredIntPt( int c, int s, int N, i64 stride, 
    p2RowStarts( N, px, py, pz, rb );
    const P2Inside in( N, px, py, pz );
    const i64      cb = i64( c ) * stride, q = cb + rb[2][2];
+   const unsigned bytes = unsigned( stride * i64( sizeof( T ) ) );
    T              val[NC];
 #pragma unroll
    for ( int k = 0; k < NC; ++k )
@@ -859,11 +889,13 @@ __device__ __forceinline__ void p2StoredIntPt( int c, int s, int N, i64 stride, 
    for ( int e = 0; e < off.n; ++e )
    {
       const T wt = ws[i64( e ) * nS];
-      // a node outside the cell has no weight: the point reads itself instead
-      const int o = in.has( off.d[e][0], off.d[e][1], off.d[e][2] ) ? rb[off.d[e][2] + 2][off.d[e][1] + 2] + off.d[e][0] : rb[2][2];
+      // a node outside the cell has no weight and reads 0 (the descriptor's range check)
+      const unsigned o = in.has( off.d[e][0], off.d[e][1], off.d[e][2] ) ?
+                             unsigned( rb[off.d[e][2] + 2][off.d[e][1] + 2] + off.d[e][0] ) * unsigned( sizeof( T ) ) :
+                             kDropOffset;
 #pragma unroll
       for ( int k = 0; k < NC; ++k )
-         val[k] += wt * ( cp.x[k] + cb )[unsigned( o )];
+         val[k] += wt * bufLoad< T >( makeRsrc( cp.x[k] + cb, bytes ), o, 0 );
    }
    if ( slot > 0 )
    {
@@ -900,8 +932,12 @@ __device__ __forceinline__ void p2StoredIntDispatch( int cls, int c, int s, int 
    else if constexpr ( CLS < 7 )
       p2StoredIntDispatch< T, MODE, CLS + 1, NC >( cls, c, s, N, stride, sw, cp, a, cfs, flag, part, partStride );
 }
+// Wavefronts per SIMD: a thread has to keep the loads of many nodes in flight. Left to itself the compiler takes 67 registers for
+// three FP64 components, in turn with their loads, and 62 for FP32 (three components, 960 cells at P2 level 4: 1119 and 678 us,
+// now 971 and 579; 240 cells at level 3 FP64 84, now below 75). One FP32 component is as fast without.
+constexpr int p2StoredWaves( int bytes, int nc, int none ) { return bytes == 8 ? ( nc > 1 ? 2 : 4 ) : ( nc > 1 ? 4 : none ); }
 template < typename T, int MODE, int NC >
-__global__ __launch_bounds__( kBlock ) void kP2StoredInt( int L, i64 stride, P2ClassTiles ct, const T* __restrict__ sw, P2Comps< T > cp,
+__global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( p2StoredWaves( sizeof( T ), NC, 1 ), p2StoredWaves( sizeof( T ), NC, 8 ) ) ) ) void kP2StoredInt( int L, i64 stride, P2ClassTiles ct, const T* __restrict__ sw, P2Comps< T > cp,
                                                           T a, const CellFaceSlot* __restrict__ cfs, int flag, T* __restrict__ part,
                                                           i64 partStride, int nC )
 {

@@ -128,8 +128,8 @@ __device__ __forceinline__ void p2KQIntPt( int c, int s, int N, i64 stride, cons
 #pragma unroll
    for ( int e = 0; e < off.n; ++e )
    {
-      // a node outside the cell has no weight: the point reads itself instead
-      const int o = in.has( off.d[e][0], off.d[e][1], off.d[e][2] ) ? rb[off.d[e][2] + 2][off.d[e][1] + 2] + off.d[e][0] : q;
+      // a node outside the cell has no weight
+      const int o = in.has( off.d[e][0], off.d[e][1], off.d[e][2] ) ? rb[off.d[e][2] + 2][off.d[e][1] + 2] + off.d[e][0] : zeroValue( N );
       // explicit fused multiply-adds: every component (and the single-component pass) rounds alike
       val[0] = fma( W[e], ( cp.x[0] + cb )[unsigned( o )], val[0] );
       if ( nc > 1 )

@@ -113,3 +113,25 @@ def test_constant_operator_and_restriction_at_the_point_itself(hyg, dtype):
         if len(c):
             assert r.download(L - 1)[c[0]] == np.inf
     assert nc < n
+
+
+@pytest.mark.parametrize("dtype", ["F64", "F32"])
+@pytest.mark.parametrize("stored", [False, True])
+def test_variable_p2_operator_at_the_point_itself(hyg, stored, dtype):
+    """A point on a cell face has stencil nodes outside the cell, of weight 0; its own infinite value stays infinite."""
+    dt, L = getattr(hyg, dtype), 2
+    mesh = hyg.Mesh("three_tets_with_two_joint_faces.msh")
+    n = mesh.ndofs(L + 1)
+    op = hyg.P2DivKGradOperator(mesh, L, L, kind=1)
+    if stored:
+        op.store_local_matrices()
+    x, y = (hyg.Function(mesh, L, L, dt, space="p2") for _ in range(2))
+    lost = []
+    for k in range(n):
+        v = np.zeros(n)
+        v[k] = np.inf
+        x.upload(L, v)
+        op.apply(x, y, L, hyg.ALL)
+        if y.download(L)[k] != np.inf:
+            lost.append(k)
+    assert not lost

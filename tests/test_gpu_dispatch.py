@@ -65,7 +65,8 @@ def test_face_points_in_the_sweep_and_from_one_sided_sums(hyg, name, L, dtype):
 @pytest.mark.parametrize("name,L", [("three_tets_with_two_joint_faces.msh", 0), ("three_tets_with_two_joint_faces.msh", 1),
                                     ("pyramid_tilted_4el.msh", 6), ("three_tets_with_two_joint_faces.msh", 7)])
 def test_variable_coefficient_sweep(hyg, name, L, dtype):
-    """The z-marching sweep: rows of one and of several 62-point windows, segments of 4 to 24 planes, every kind of point."""
+    """The sweep with a thread per point and, for FP32 at level 7, the march in segments of 4 planes: every kind of point. The inverse
+    diagonal is the library's own here (against the oracle: test_gpu_divkgrad.py, test_gpu_march.py)."""
     dt = getattr(hyg, dtype)
     modes = ol.random_field(33, modes=8, kmax=3)
     gm, om = hyg.Mesh(name), ol.Mesh(name)
@@ -100,7 +101,7 @@ def test_variable_coefficient_sweep(hyg, name, L, dtype):
 
 
 def test_points_do_not_see_values_that_are_not_their_neighbours(hyg):
-    """An infinite value reaches the points whose stencil holds it and no other (the lanes past a row end of the sweep)."""
+    """An infinite value stays within the stencil of its point (which neighbours of weight 0 do not see: test_gpu_nonfinite.py)."""
     L, name = 6, "tet_1el.msh"
     gm, om = hyg.Mesh(name), ol.Mesh(name)
     n = gm.ndofs(L)
@@ -124,8 +125,8 @@ def test_points_do_not_see_values_that_are_not_their_neighbours(hyg):
 @pytest.mark.parametrize("dtype", ["F64", "F32"])
 @pytest.mark.parametrize("nmodes,L", [(0, 1), (1, 3), (8, 5), (9, 2), (32, 6), (33, 4), (64, 5)])
 def test_coefficient_integrals_of_every_variant(hyg, nmodes, L, dtype):
-    """The matrix product behind k, by the number of modes (padded to 8, 32 or 64) and the length of rows (16-anchor tiles
-    and their remainders, blocks of 16 and 32 rows)."""
+    """The matrix product behind k by the number of modes (tables padded to 8, 32 or 64) and the length of rows; which of the two kernels
+    forms it: test_gpu_march.py."""
     dt = getattr(hyg, dtype)
     name = "pyramid_tilted_4el.msh"
     modes = ol.random_field(5, modes=nmodes, kmax=3) if nmodes else []

@@ -2,7 +2,6 @@
 absolute figure is pinned. Every bound lies between the ratio measured with the rule and that of the one kernel for all sizes
 it replaced (both are given), and numbers of launches are counted in a captured graph."""
 import ctypes as C
-import os
 import time
 
 import pytest

@@ -42,7 +42,6 @@ struct CombineTask
    int               kind, first;
    const LowerChunk* chunks;
    int               nChunks, firstFacePrim, L, flag;
-   const LowerPrim*  prims;
    const LowerEntry* entries;
    const T*          part;
    const T*          primInv;
@@ -66,7 +65,6 @@ struct TransferTask
    i64               strideF, strideC;
    const LowerChunk* chunks;
    int               nChunks;
-   const LowerPrim*  prims;
    const LowerEntry* entries;
    const CellInfo*   cinfo;
    T*                dst;
@@ -144,7 +142,7 @@ __global__ __launch_bounds__( kBlock, kElemOccupancy< T > ) void kBatchElem( con
    if ( vb >= total )
       return;
    const ElemTask< T >& t = tasks[findTask( tasks, nTasks, vb )];
-   elemSweep< T, MODE, kElemRows >( vb - t.first, (ElemArgsAt< T >) &t.el );
+   elemSweep< T, MODE >( vb - t.first, (ElemArgsAt< T >) &t.el );
 }
 
 template < typename T, int MODE >
@@ -170,10 +168,10 @@ __global__ __launch_bounds__( kBlock ) void kBatchCombine( const CombineTask< T 
       const CombineTask< T >& t = tasks[findTask( tasks, nTasks, vb )];
       const int               b = vb - t.first;
       if ( t.kind == 0 )
-         bFaceCombine< T, MODE >( b, t.chunks, t.nChunks, t.prims, t.entries, t.firstFacePrim, t.part, t.primInv, t.dinv, t.L,
+         bFaceCombine< T, MODE >( b, t.chunks, t.nChunks, t.entries, t.firstFacePrim, t.part, t.primInv, t.dinv, t.L,
                                   t.stride, t.flag, t.x, t.in1, t.out0, t.out1, t.a );
       else
-         bLowCombine< T, MODE >( b, t.chunks, t.nChunks, t.prims, t.entries, t.part, t.dinv, t.L, t.stride, t.flag, t.x, t.in1,
+         bLowCombine< T, MODE >( b, t.chunks, t.nChunks, t.entries, t.part, t.dinv, t.L, t.stride, t.flag, t.x, t.in1,
                                  t.out0, t.out1, t.a );
    }
 }
@@ -285,7 +283,6 @@ void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item 
       f.firstFacePrim = m.mesh->nV() + m.mesh->nE();
       f.L             = it.L;
       f.flag          = c.flag;
-      f.prims         = m.prims;
       f.entries       = m.entries;
       f.stride        = g.stride;
       f.x             = (const T*) c.x;
@@ -296,7 +293,7 @@ void addStencilT( BatchPlan& plan, int mode, const std::vector< BatchPlan::Item 
       if ( op.kind == 0 )
       {
          t.kind          = 0;
-         t.sw            = sweepArgs< T >( m, g, ol, it.L, c, cfg );
+         t.sw            = sweepArgs< T >( m, g, ol, it.L, c, cfg, directFaces( m, g ) );
          const int gL    = t.sw.nChunks > 0 ? xcdGrid( ceilDiv( t.sw.nChunks, kBlock / 64 ) ) : 0;
          appendTask( st, t, t.sw.gC + t.sw.gF + gL );
          f.kind    = 0;
@@ -355,7 +352,6 @@ void addRestrictT( BatchPlan& plan, const std::vector< BatchPlan::Transfer >& it
       t.strideF = cellStride( it.L + 1 );
       t.chunks  = gc.chunks;
       t.nChunks = gc.nChunks;
-      t.prims   = m.prims;
       t.entries = m.entries;
       t.cinfo   = m.cellInfo;
       t.dst     = (T*) it.dst;

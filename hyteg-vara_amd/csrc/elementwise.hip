@@ -8,12 +8,13 @@
 // ElemCell::mt) and kb_e = 6 sum_q w_q k(x_q) is the 5-point degree-3 quadrature of k over the
 // element divided by its volume (w = -2/15 at the centroid, 3/40 at the four points with barycentric
 // coordinates (1/2, 1/6, 1/6, 1/6)). Each apply
-//   1. evaluates kb_e for every micro-cell (kKBar): the log-coefficient at the 30 quadrature points of the six cell
-//      types of a lattice point is a matrix product of the modes' phase factors there with a constant matrix of
-//      their amplitudes and offsets (kKBarTables, once per level at operator creation), on the matrix cores;
-//   2. marches over the cubes of the anchor lattice plane by plane and adds the contributions of their six elements to
-//      the corners (kElemSweep); interior points get the epilogue, points on faces, edges and vertices store the cell's
-//      one-sided sum;
+//   1. evaluates kb_e for every micro-cell: the log-coefficient at the 30 quadrature points of the six cell types of a
+//      lattice point is a matrix product of the modes' phase factors there with a constant matrix of their amplitudes
+//      and offsets (kKBarTables, once per level at operator creation), with a thread per anchor (kKBarPoint) or on the
+//      matrix cores (kKBar);
+//   2. forms the product at every point of the closed cells, with a thread per point (kElemApply) or, on long rows, marching
+//      over the cubes of the anchor lattice plane by plane (kElemSweep); interior points get the epilogue, points on
+//      faces, edges and vertices store the cell's one-sided sum;
 //   3. adds the one-sided sums of face, edge and vertex points over their cells and writes every
 //      replica (kFaceCombine, kLowCombine).
 // The inverse diagonal (per point, since it depends on k) is built the same way at operator setup.
@@ -199,17 +200,17 @@ static void elemT( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, co
    else
    {
       const ElemArgs< T > e = elemArgs< T >( m, g, ol, L, c );
-      hipLaunchKernelGGL( ( kElemSweep< T, MODE, kElemRows > ), dim3( elemBlocks( e ) ), dim3( kBlock ), 0, s, e );
+      hipLaunchKernelGGL( ( kElemSweep< T, MODE > ), dim3( elemBlocks( e ) ), dim3( kBlock ), 0, s, e );
    }
    // 3. face, edge and vertex values
    const int nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
    if ( nFace > 0 )
       hipLaunchKernelGGL( ( kFaceCombine< T, MODE > ), dim3( xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) ), dim3( kBlock ), 0, s,
-                          g.chunks + g.firstFaceChunk, nFace, m.prims, m.entries, m.mesh->nV() + m.mesh->nE(), part, (const T*) nullptr,
+                          g.chunks + g.firstFaceChunk, nFace, m.entries, m.mesh->nV() + m.mesh->nE(), part, (const T*) nullptr,
                           dv, L, g.stride, c.flag, x, in1, out0, out1, T( c.a ) );
    if ( nLow > 0 )
       hipLaunchKernelGGL( ( kLowCombine< T, MODE > ), dim3( ceilDiv( nLow, kBlock / 64 ) ), dim3( kBlock ), 0, s, g.chunks, nLow,
-                          m.prims, m.entries, low, dv, L, g.stride, c.flag, x, in1, out0, out1, T( c.a ) );
+                          m.entries, low, dv, L, g.stride, c.flag, x, in1, out0, out1, T( c.a ) );
 }
 
 template < typename T >

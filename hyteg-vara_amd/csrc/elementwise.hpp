@@ -36,10 +36,10 @@ __device__ __forceinline__ int kbRow( int N, int y, int z ) { return 6 * ( S3i( 
 // slots 5..7), the last slot of groups 1 and 3 is empty. Columns: 16 anchors of a row.
 // A block takes rowsPer (32, or 16 where that leaves too few blocks) rows of a plane, each wave every fourth of them; per tile
 // of 16 anchors a wave holds X Z (2 values per step in registers) and walks its rows, whose Y is staged in LDS with the
-// constant matrix. (Waves on tiles of their own, whose rows are fewer at large x: 1570 us.)
-// 32 modes, level 7, 24 cells (8.6 million anchors): FP64 2180 -> 1130 us, FP32 814 -> 600 us against a thread per anchor with
-// a sincos per mode and the matrix read through the scalar cache. The FP64 time is that of 2 S matrix instructions (30 ns
-// each per SIMD, 600 us in all; 30 of 32 rows used) and of the 8 exponentials per lane, which use the same FP64 units.
+// constant matrix. (Waves on tiles of their own, whose rows are fewer at large x: 1570 us in FP64 at level 7 on 24 cells, against 1130.)
+// 32 modes, level 7, 24 cells (8.6 million anchors), FP32: apply 634 us, with a thread per anchor (kKBarPoint) 713. In FP64 the matrix
+// instructions (30 ns each per SIMD, 600 us in all) and the exponentials, which use the same units, take longer than that thread's
+// multiply-adds: 1231 against 1103. Where either is taken: kbOnMatrixCores.
 constexpr int kKBarRows = 32;
 
 typedef double f64x4 __attribute__( ( ext_vector_type( 4 ) ) );
@@ -443,28 +443,29 @@ struct ElemArgs
 template < typename T >
 using ElemArgsAt = const __attribute__( ( address_space( 4 ) ) ) ElemArgs< T >*;
 
-// What a wave loads for one cube layer z: kb of the six types of anchor rows y0-1 .. y0+R-1, and point rows y0-1 .. y0+R
-// of plane z+1.
-template < typename T, int R >
+// What a wave loads for one cube layer z: kb of the six types of anchor rows y-1 and y, and point rows y-1 .. y+1 of plane z+1.
+template < typename T >
 struct ElemLayer
 {
-   T k[R + 1][6];
-   T u[R + 2];
+   T k[2][6];
+   T u[3];
 };
 
-// All points of the closed cells. A wave owns R rows (y0 ..) and 62 points (x0 .., lanes 1..62) and marches z: layer z (the
-// cubes between planes z and z+1) gives its contributions to plane z, which completes it, and to plane z+1, which are
-// carried; corners at x+1 are moved by one lane shift per row. It reads the six kb of an anchor and each value about once
-// (64 B per point in FP64) where a thread per point gathered 39 values: level 7 on 24 cells (8.4 million points) 314 -> 242
-// us in FP64, FP32 Jacobi sweep 244 -> 140 us. Bound by the vector instructions of a step (180 FP32, of which 105 are the
-// edge products) at 55% of the lanes: rows of a tetrahedron end inside the 62-point windows.
+// All points of the closed cells. A wave owns a row y and 62 points (x0 .., lanes 1..62) and marches z: layer z (the cubes
+// between planes z and z+1 in the anchor rows y-1 and y) gives its contributions to plane z, which completes it, and to plane z+1,
+// which are carried; corners at x+1 are moved by one lane shift per row. A point costs 12 loads of kb and 3 of values (120 B in
+// FP64 requested, of which neighbouring rows find half in cache) and 14 edges of either cube (28 products with a difference), where
+// a thread per point gathers 24 kb and 15 values. Bound by the vector instructions of a step (180 FP32, of which 105 are the edge
+// products) at 55% of the lanes at level 7: rows of a tetrahedron end inside the 62-point windows. Two rows per wave share more
+// loads and edge differences but halve the waves in flight (FP32 sweep at level 7 on 24 cells 208 against 196 us, both with 24-plane
+// segments).
 // A sum of differences turns an infinite value into NaN at points whose weight for it is 0 (and at the point itself): a plane with
 // a sum that is not finite stores nothing and is done again point by point behind the march (planes: one bit each).
 // Lanes outside a row, rows outside a plane and anchors outside the cell load 0 (the descriptor's range check), so they
 // add nothing; elements that stick out of the cell have kb = 0.
 // The arguments are read where they are used (ap, made opaque for the rare boundary rows): held in scalar registers through
 // the march they spilled, 66 of 250 vector instructions per plane.
-template < typename T, int MODE, int R >
+template < typename T, int MODE >
 __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
 {
    const auto&    p    = *ap;
@@ -516,11 +517,11 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
       return bufLoad< T >( rx, unsigned( px ) < unsigned( n ) ? unsigned( px * B ) : kDropOffset, o );
    };
    // layer z: kb of the anchor rows and the point rows of plane z+1
-   auto loadLayer = [&]( ElemLayer< T, R >& Q, int z ) {
+   auto loadLayer = [&]( ElemLayer< T >& Q, int z ) {
       const int  W  = N - z; // anchors of row 0
       const auto rk = makeRsrc( kc + 6 * ( SN - S3i( W ) ), W > 0 ? unsigned( 6 * T2i( W ) * B ) : 0u );
 #pragma unroll
-      for ( int r = 0; r <= R; ++r )
+      for ( int r = 0; r < 2; ++r )
       {
          const int      y = y0 - 1 + r, n = y >= 0 ? max( 0, W - y ) : 0;
          const int      o  = n > 0 ? 6 * rowStart( W, y ) * B : 0;
@@ -530,60 +531,46 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
             Q.k[r][t] = bufLoad< T >( rk, vo, o + t * n * B );
       }
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
          Q.u[r] = loadU( y0 - 1 + r, z + 1 );
    };
-   T lo[R + 2], loX[R + 2]; // plane z: the rows and their values at x+1
-   T cn[R], cs[R];          // contributions of layer z-1 to plane z: at the anchor's x, and at x+1 (to be shifted)
-#pragma unroll
-   for ( int r = 0; r < R; ++r )
-      cn[r] = cs[r] = T( 0 );
+   T lo[3], loX[3]; // plane z: the rows and their values at x+1
+   T cn = T( 0 ), cs = T( 0 ); // contributions of layer z-1 to plane z: at the anchor's x, and at x+1 (to be shifted)
    // contributions of layer z: `first` forms only those to plane z+1
-   auto layer = [&]( const ElemLayer< T, R >& Q, const T ( &hiX )[R + 2], bool first, T ( &n )[R], T ( &s )[R] ) {
+   auto layer = [&]( const ElemLayer< T >& Q, const T ( &hiX )[3], bool first, T& n, T& s ) {
+      n  = cn;
+      s  = cs;
+      cn = cs = T( 0 );
 #pragma unroll
-      for ( int r = 0; r < R; ++r )
-      {
-         n[r]  = cn[r];
-         s[r]  = cs[r];
-         cn[r] = cs[r] = T( 0 );
-      }
-#pragma unroll
-      for ( int r = 0; r <= R; ++r )
+      for ( int r = 0; r < 2; ++r )
       {
          const T u[8] = { lo[r], loX[r], lo[r + 1], loX[r + 1], Q.u[r], hiX[r], Q.u[r + 1], hiX[r + 1] };
          T       q[8];
 #pragma unroll
          for ( int k = 0; k < 8; ++k )
             q[k] = T( 0 );
-         // anchor row y0-1+r: its y corners are point rows r-1 (if r > 0) and r (if r < R)
-         if ( first )
+         // the row's points are the upper y corners of anchor row y-1 and the lower ones of row y
+         if ( r == 0 )
          {
-            if ( r == 0 )
+            if ( first )
                cubeContributions< T, 0xc0 >( K, Q.k[r], u, q );
-            else if ( r == R )
+            else
+               cubeContributions< T, 0xcc >( K, Q.k[r], u, q );
+            n += q[2];
+            s += q[3];
+            cn += q[6];
+            cs += q[7];
+         }
+         else
+         {
+            if ( first )
                cubeContributions< T, 0x30 >( K, Q.k[r], u, q );
             else
-               cubeContributions< T, 0xf0 >( K, Q.k[r], u, q );
-         }
-         else if ( r == 0 )
-            cubeContributions< T, 0xcc >( K, Q.k[r], u, q );
-         else if ( r == R )
-            cubeContributions< T, 0x33 >( K, Q.k[r], u, q );
-         else
-            cubeContributions< T, 0xff >( K, Q.k[r], u, q );
-         if ( r > 0 )
-         {
-            n[r - 1] += q[0];
-            s[r - 1] += q[1];
-            cn[r - 1] += q[4];
-            cs[r - 1] += q[5];
-         }
-         if ( r < R )
-         {
-            n[r] += q[2];
-            s[r] += q[3];
-            cn[r] += q[6];
-            cs[r] += q[7];
+               cubeContributions< T, 0x33 >( K, Q.k[r], u, q );
+            n += q[0];
+            s += q[1];
+            cn += q[4];
+            cs += q[5];
          }
       }
    };
@@ -601,92 +588,77 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
                          q->lowPart );
    };
    unsigned again = 0; // planes that are done again
-   T vEdge[R] = {}; // values of the rows' points on the edge between local vertices 2 and 3 (x = 0 on the diagonal face)
-   // one plane: `cur` holds layer z, `nxt` receives layer z+1; EDGE: the plane or a row of it lies on a face of the cell
-   auto step = [&]( auto EDGE, ElemLayer< T, R >& cur, ElemLayer< T, R >& nxt ) {
-      T ein[R], edi[R];
-#pragma unroll
-      for ( int r = 0; r < R; ++r )
-      {
-         int            n;
-         const int      o  = rowU( y0 + r, z, n );
-         // lanes past the row end read what follows in the array (or 0 past its slack); their results are dropped
-         if constexpr ( kE )
-            ein[r] = bufLoad< T >( re, vx, o );
-         if constexpr ( kD )
-            edi[r] = bufLoad< T >( rd, vx, o );
-      }
+   T        vEdge = T( 0 ); // value of the row's point on the edge between local vertices 2 and 3 (x = 0 on the diagonal face)
+   // one plane: `cur` holds layer z, `nxt` receives layer z+1; EDGE: the row or the plane lies on a face of the cell
+   auto step = [&]( auto EDGE, ElemLayer< T >& cur, ElemLayer< T >& nxt ) {
+      int       cnt;
+      const int o = rowU( y0, z, cnt );
+      // lanes past the row end read what follows in the array (or 0 past its slack); their results are dropped
+      const T ein = kE ? bufLoad< T >( re, vx, o ) : T( 0 ), edi = kD ? bufLoad< T >( rd, vx, o ) : T( 0 );
       if ( z + 1 < z1 )
          loadLayer( nxt, z + 1 );
-      T hiX[R + 2], n[R], s[R];
+      T hiX[3], n, s;
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
          hiX[r] = laneMove< kDppWaveShl1 >( cur.u[r] );
       layer( cur, hiX, false, n, s );
-#pragma unroll
-      for ( int r = 0; r < R; ++r )
+      const T   Ax = n + laneMove< kDppWaveShr1 >( s );
+      const int xe = N - y0 - z; // row end
+      if ( xe >= x0 ) // (wave-uniform) something of the row in the window
       {
-         const T   Ax = n[r] + laneMove< kDppWaveShr1 >( s[r] );
-         const int y = y0 + r, xe = N - y - z; // row end
-         if ( xe < x0 )
-            continue; // (wave-uniform) nothing of this row in the window
          if ( __builtin_expect( __ballot( !isfinite( Ax ) ) != 0, 0 ) )
-         {
             again |= 1u << ( z - z0 );
-            continue;
-         }
-         if constexpr ( EDGE.value )
-            if ( y == 0 || z == 0 )
-            {
-               if ( mine && px <= xe )
-                  boundary( y, Ax );
-               continue;
-            }
-         int       cnt;
-         const int o  = rowU( y, z, cnt );
-         T         q0 = T( 0 ), q1 = T( 0 );
-         epilogue< T, MODE >( Ax, lo[r + 1], kE ? ein[r] : T( 0 ), kE ? ein[r] : T( 0 ), kD ? edi[r] : T( 0 ), a, q0, q1 );
-         const unsigned so = pIn < xe ? vx : kDropOffset;
-         bufStore( q0, r0, so, o );
-         if constexpr ( kTwo )
-            bufStore( q1, r1, so, o );
-         if ( xe > 0 )
+         else if ( EDGE.value && ( y0 == 0 || z == 0 ) )
          {
-            // face points: x = 0 and the row end
-            if ( on2 )
-               bufStore( Ax, rp2, v2, facePartIndex( 2, N, 0, y, z ) * B );
-            if ( on3 && xe <= x0 + 61 )
-               bufStore( Ax, rp3, mine && px == xe ? 0u : kDropOffset, facePartIndex( 3, N, xe, y, z ) * B );
+            if ( mine && px <= xe )
+               boundary( y0, Ax );
          }
          else
-            vEdge[r] = Ax;
+         {
+            T q0 = T( 0 ), q1 = T( 0 );
+            epilogue< T, MODE >( Ax, lo[1], ein, ein, edi, a, q0, q1 );
+            const unsigned so = pIn < xe ? vx : kDropOffset;
+            bufStore( q0, r0, so, o );
+            if constexpr ( kTwo )
+               bufStore( q1, r1, so, o );
+            if ( xe > 0 )
+            {
+               // face points: x = 0 and the row end
+               if ( on2 )
+                  bufStore( Ax, rp2, v2, facePartIndex( 2, N, 0, y0, z ) * B );
+               if ( on3 && xe <= x0 + 61 )
+                  bufStore( Ax, rp3, mine && px == xe ? 0u : kDropOffset, facePartIndex( 3, N, xe, y0, z ) * B );
+            }
+            else
+               vEdge = Ax;
+         }
       }
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
       {
          lo[r]  = cur.u[r];
          loX[r] = hiX[r];
       }
       ++z;
    };
-   ElemLayer< T, R > A, Bq;
+   ElemLayer< T > A, Bq;
    if ( z0 > 0 )
    {
-      T hiX[R + 2], n[R], s[R];
+      T hiX[3], n, s;
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
          lo[r] = loadU( y0 - 1 + r, z0 - 1 );
       loadLayer( Bq, z0 - 1 );
       loadLayer( A, z0 );
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
       {
          loX[r] = laneMove< kDppWaveShl1 >( lo[r] );
          hiX[r] = laneMove< kDppWaveShl1 >( Bq.u[r] );
       }
       layer( Bq, hiX, true, n, s );
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
       {
          lo[r]  = Bq.u[r];
          loX[r] = hiX[r];
@@ -695,14 +667,14 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
    else
    {
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
          lo[r] = loadU( y0 - 1 + r, 0 );
       loadLayer( A, 0 );
 #pragma unroll
-      for ( int r = 0; r < R + 2; ++r )
+      for ( int r = 0; r < 3; ++r )
          loX[r] = laneMove< kDppWaveShl1 >( lo[r] );
    }
-   // The general stores of the rows y = 0 and the plane z = 0 stay out of the main loop, whose scalar registers they would
+   // The general stores of the row y = 0 and the plane z = 0 stay out of the main loop, whose scalar registers they would
    // spill.
    if ( y0 == 0 || z0 == 0 )
       do
@@ -718,13 +690,11 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
       step( std::false_type(), Bq, A );
    }
    if ( x0 == 0 && lane == 1 )
-#pragma unroll
-      for ( int r = 0; r < R; ++r )
-      {
-         z = N - y0 - r;
-         if ( y0 + r > 0 && z > 0 && z >= z0 && z < z1 )
-            boundary( y0 + r, vEdge[r] );
-      }
+   {
+      z = N - y0;
+      if ( y0 > 0 && z > 0 && z >= z0 && z < z1 )
+         boundary( y0, vEdge );
+   }
    if ( again != 0 )
    {
       ElemArgsAt< T > q = ap;
@@ -732,26 +702,21 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
       for ( ; again != 0; again &= again - 1 )
       {
          z = z0 + __builtin_ctz( again );
-#pragma unroll 1
-         for ( int r = 0; r < R; ++r )
+         if ( lane < 1 || lane > 62 || px > N - y0 - z )
+            continue;
+         const i64 cq  = i64( c ) * q->stride;
+         const T   val = elemValue( uniformPtr( q->cells + c ), q->kb + i64( c ) * 6 * S3i( N ), q->x + cq, N, px, y0, z );
+         if ( classifySlot( N, px, y0, z ) != 0 )
+            boundary( y0, val );
+         else if ( q->flag & 1 )
          {
-            const int y = y0 + r;
-            if ( lane < 1 || lane > 62 || px > N - y - z )
-               continue;
-            const i64 cq  = i64( c ) * q->stride;
-            const T   val = elemValue( uniformPtr( q->cells + c ), q->kb + i64( c ) * 6 * S3i( N ), q->x + cq, N, px, y, z );
-            if ( classifySlot( N, px, y, z ) != 0 )
-               boundary( y, val );
-            else if ( q->flag & 1 )
-            {
-               const i64 o  = cq + cidx( N + 1, px, y, z );
-               const T   e  = kIn1 ? q->in1[o] : ( MODE == MODE_APPLY_ADD ? q->out0[o] : T( 0 ) );
-               T         q0 = T( 0 ), q1 = T( 0 );
-               epilogue< T, MODE >( val, q->x[o], e, e, kD ? q->dinv[o] : T( 0 ), q->a, q0, q1 );
-               q->out0[o] = q0;
-               if constexpr ( kTwo )
-                  q->out1[o] = q1;
-            }
+            const i64 o  = cq + cidx( N + 1, px, y0, z );
+            const T   e  = kIn1 ? q->in1[o] : ( MODE == MODE_APPLY_ADD ? q->out0[o] : T( 0 ) );
+            T         q0 = T( 0 ), q1 = T( 0 );
+            epilogue< T, MODE >( val, q->x[o], e, e, kD ? q->dinv[o] : T( 0 ), q->a, q0, q1 );
+            q->out0[o] = q0;
+            if constexpr ( kTwo )
+               q->out1[o] = q1;
          }
       }
    }
@@ -761,11 +726,11 @@ __device__ __forceinline__ void elemSweep( int bid, ElemArgsAt< T > ap )
 template < typename T >
 constexpr int kElemOccupancy = sizeof( T ) == 4 ? 6 : 3;
 
-template < typename T, int MODE, int R >
+template < typename T, int MODE >
 __global__ __launch_bounds__( kBlock, kElemOccupancy< T > ) void kElemSweep( ElemArgs< T > p )
 {
    // p is the whole argument segment
-   elemSweep< T, MODE, R >( int( blockIdx.x ), (ElemArgsAt< T >) __builtin_amdgcn_kernarg_segment_ptr() );
+   elemSweep< T, MODE >( int( blockIdx.x ), (ElemArgsAt< T >) __builtin_amdgcn_kernarg_segment_ptr() );
 }
 
 // arguments of the sweep of one level, and its blocks

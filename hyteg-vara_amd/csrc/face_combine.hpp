@@ -9,7 +9,6 @@ namespace hyg {
 
 template < typename T, int MODE >
 __device__ __forceinline__ void bFaceCombine( int bid, const LowerChunk* __restrict__ chunks, int nChunks,
-                                                          const LowerPrim* __restrict__ prims,
                                                           const LowerEntry* __restrict__ entries, int firstFacePrim,
                                                           const T* __restrict__ part, const T* __restrict__ primInv,
                                                           const T* __restrict__ dinvArr, int L,
@@ -55,14 +54,13 @@ __device__ __forceinline__ void bFaceCombine( int bid, const LowerChunk* __restr
 
 template < typename T, int MODE >
 __global__ __launch_bounds__( kBlock ) void kFaceCombine( const LowerChunk* __restrict__ chunks, int nChunks,
-                                                          const LowerPrim* __restrict__ prims,
                                                           const LowerEntry* __restrict__ entries, int firstFacePrim,
                                                           const T* __restrict__ part, const T* __restrict__ primInv,
                                                           const T* __restrict__ dinvArr, int L,
                                                           i64 stride, int flag, const T* __restrict__ x,
                                                           const T* __restrict__ in1, T* __restrict__ out0, T* __restrict__ out1, T a )
 {
-   bFaceCombine< T, MODE >( int( blockIdx.x ), chunks, nChunks, prims, entries, firstFacePrim, part, primInv, dinvArr, L, stride, flag, x, in1, out0, out1, a );
+   bFaceCombine< T, MODE >( int( blockIdx.x ), chunks, nChunks, entries, firstFacePrim, part, primInv, dinvArr, L, stride, flag, x, in1, out0, out1, a );
 }
 
 // colour of point (i, j) of a macro-face, -edge or -vertex in the multi-colour SOR ordering: the sum over the
@@ -80,7 +78,7 @@ __device__ __forceinline__ int sorColour( const CellInfo* __restrict__ cinfo, co
 // points of colour sorK, in place, every replica
 template < typename T >
 __global__ __launch_bounds__( kBlock ) void kFaceCombineSor( const LowerChunk* __restrict__ chunks, int nChunks,
-                                                             const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
+                                                             const LowerEntry* __restrict__ entries,
                                                              int firstFacePrim, const T* __restrict__ part, const T* __restrict__ primInv,
                                                              const CellInfo* __restrict__ cinfo, int sorK, int sorM, int L, i64 stride,
                                                              int flag, T* __restrict__ x, const T* __restrict__ b, T a )
@@ -145,7 +143,7 @@ __device__ __forceinline__ void tetXYZ( int w, int s, int& x, int& y, int& z )
 // ------------------------------------------------------------------ edges and vertices: combine
 template < typename T, int MODE >
 __device__ __forceinline__ void bLowCombine( int bid, const LowerChunk* __restrict__ chunks, int nChunks,
-                                                         const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
+                                                         const LowerEntry* __restrict__ entries,
                                                          const T* __restrict__ lowPart, const T* __restrict__ dinv, int L,
                                                          i64 stride, int flag, const T* __restrict__ x, const T* __restrict__ in1,
                                                          T* __restrict__ out0, T* __restrict__ out1, T a )
@@ -189,12 +187,12 @@ __device__ __forceinline__ void bLowCombine( int bid, const LowerChunk* __restri
 
 template < typename T, int MODE >
 __global__ __launch_bounds__( kBlock ) void kLowCombine( const LowerChunk* __restrict__ chunks, int nChunks,
-                                                         const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
+                                                         const LowerEntry* __restrict__ entries,
                                                          const T* __restrict__ lowPart, const T* __restrict__ dinv, int L,
                                                          i64 stride, int flag, const T* __restrict__ x, const T* __restrict__ in1,
                                                          T* __restrict__ out0, T* __restrict__ out1, T a )
 {
-   bLowCombine< T, MODE >( int( blockIdx.x ), chunks, nChunks, prims, entries, lowPart, dinv, L, stride, flag, x, in1, out0, out1, a );
+   bLowCombine< T, MODE >( int( blockIdx.x ), chunks, nChunks, entries, lowPart, dinv, L, stride, flag, x, in1, out0, out1, a );
 }
 
 // 1 / d of every value (0 stays 0: padding and unused slots)

@@ -131,11 +131,8 @@ constexpr int kZSegChunk = 24;
 constexpr int kZSegLeast = 4;
 constexpr int kZSegFull  = 8; // level 7, 6 cells (3.6 planes for kZSegWaves): FP64 apply 21.8 us with 4 planes, 19.1 with 8, FP32 15.9, 15.6
 constexpr int kZSegWaves = 8192;
-// The variable-coefficient sweep: one row per wavefront (two rows share more loads and edge differences but halve the waves
-// in flight: 208 against 196 us for an FP32 sweep at level 7), and segments for four times the waves (6 planes at level 7
-// on 24 cells: with 4 / 6 / 8 / 12 / 16 / 24 planes that sweep takes 188 / 181 / 180 / 182 / 186 / 196 us, a batched cycle
-// of 12 problems of levels 4 to 6 4.42 / 4.43 / 4.51 / 4.82 / 5.00 / 5.42 ms).
-constexpr int kElemRows  = 1;
+// The variable-coefficient march: segments for four times the waves of the constant sweep (6 planes at level 7 on 24 cells: with 4 /
+// 6 / 8 / 12 / 16 / 24 planes the FP32 sweep takes 188 / 181 / 180 / 182 / 186 / 196 us).
 constexpr int kElemWaves = 32768;
 // P2 constant operator, z-marching row pairs: a wavefront computes rows y0 (even) and y0+1 of a segment of
 // kP2ZSeg x values (x0 = kP2ZSeg k - 2 + 2 lane, lanes 0 and 63 halo) over planes [z0, z1), z0 even; the

@@ -15,10 +15,10 @@
 // cell's one-sided sum for kFaceCombine / kLowCombine, exactly as the P1 elementwise operator does.
 //
 // Variable coefficient (P2ElementwiseOperator< p2_div_k_grad_affine_q4 >, P2ElementwiseOperator.cpp:100-310):
-// the element matrix of micro-cell e of type t is sum_q k_e,q M_t,q with the 11 quadrature-point matrices
-// M_t,q = w_q |det J| grad phi(l_q) grad phi(l_q)^T of the cell's type t (affine map: the same for every
-// micro-cell of that type) and the coefficient k_e,q at the quadrature points, evaluated once at operator
-// setup (kP2KQ). A point assembles the rows it needs on the fly.
+// a row of the element matrix of micro-cell e of type t is a short combination of the ten moments of k against
+// lambda_a lambda_b on e (11-point rule, formed once at operator setup by kP2KQ) and the ten products
+// |det J| grad lambda_a . grad lambda_b of the cell's type t (affine map: the same for every micro-cell of that type;
+// p2_common.hpp). A point assembles the rows it needs on the fly, or they are summed once into its stored stencil.
 #include "p2_common.hpp"
 
 #include <utility>
@@ -1164,8 +1164,7 @@ static i64 p2LowStride( const MeshCtx& m, int L ) { return i64( m.entriesHost.si
 // Face, edge and vertex points of up to three components (one per grid row) from their partial sums, one launch
 template < typename T, int MODE >
 __global__ __launch_bounds__( kBlock ) void kP2Combine( int gF, const LowerChunk* __restrict__ chunks, int nLow, int nFace,
-                                                        const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
-                                                        int firstFacePrim, const T* __restrict__ part, i64 partStride,
+                                                        const LowerEntry* __restrict__ entries, int firstFacePrim, const T* __restrict__ part, i64 partStride,
                                                         const T* __restrict__ low, i64 lowStride, const T* __restrict__ dinv, int L, i64 stride,
                                                         int flag, P2Comps< T > cp, T a )
 {
@@ -1175,10 +1174,10 @@ __global__ __launch_bounds__( kBlock ) void kP2Combine( int gF, const LowerChunk
    T*        out0 = k == 0 ? cp.out0[0] : ( k == 1 ? cp.out0[1] : cp.out0[2] );
    T*        out1 = k == 0 ? cp.out1[0] : ( k == 1 ? cp.out1[1] : cp.out1[2] );
    if ( b < gF )
-      bFaceCombine< T, MODE >( b, chunks + nLow, nFace, prims, entries, firstFacePrim, part + i64( k ) * partStride, (const T*) nullptr, dinv, L,
+      bFaceCombine< T, MODE >( b, chunks + nLow, nFace, entries, firstFacePrim, part + i64( k ) * partStride, (const T*) nullptr, dinv, L,
                                stride, flag, x, in1, out0, out1, a );
    else
-      bLowCombine< T, MODE >( b - gF, chunks, nLow, prims, entries, low + i64( k ) * lowStride, dinv, L, stride, flag, x, in1, out0, out1, a );
+      bLowCombine< T, MODE >( b - gF, chunks, nLow, entries, low + i64( k ) * lowStride, dinv, L, stride, flag, x, in1, out0, out1, a );
 }
 template < typename T >
 static P2Comps< T > p2Comps( const StencilCall* cs, int n )
@@ -1200,7 +1199,7 @@ static void p2Combines( const MeshCtx& m, const LevelGeom& g, int L, const Stenc
    const int nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
    const int gF   = nFace > 0 ? xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) : 0;
    hipLaunchKernelGGL( ( kP2Combine< T, MODE > ), dim3( gF + ceilDiv( nLow, kBlock / 64 ), n ), dim3( kBlock ), 0, s, gF, g.chunks, nLow, nFace,
-                       m.prims, m.entries, m.mesh->nV() + m.mesh->nE(), part, p2PartStride( m, L ), low, p2LowStride( m, L ), dv, L, g.stride,
+                       m.entries, m.mesh->nV() + m.mesh->nE(), part, p2PartStride( m, L ), low, p2LowStride( m, L ), dv, L, g.stride,
                        cs[0].flag, p2Comps< T >( cs, n ), T( cs[0].a ) );
 }
 
@@ -1355,7 +1354,7 @@ void launchP2Vector( const MeshCtx& m, LevelGeom& g, const hyg_op_s& op, int L, 
       cs[0].mode == MODE_APPLY ? p2Variable< float, MODE_APPLY >( m, g, op, L, cs, n, s ) : p2Variable< float, MODE_APPLY_ADD >( m, g, op, L, cs, n, s );
 }
 
-// coefficient values of every micro-cell at its 11 quadrature points (variable-coefficient P2 operator)
+// moments of the coefficient of every micro-cell (variable-coefficient P2 operator)
 void launchP2Coefficients( const MeshCtx& m, const hyg_op_s& op, int L, hipStream_t s )
 {
    const hyg_op_s::Level& ol = op.levels[L];

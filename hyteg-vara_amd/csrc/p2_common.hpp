@@ -68,7 +68,7 @@ struct P2Comps
 };
 
 // Stored stencils (setup) and the on-the-fly apply: the stencil of a point is the sum, over the micro-cells that have
-// it as node l (on the cell's side of face F for a face point), of row l of sum_q k_q M_{t,q}, keyed by the offset to
+// it as node l (on the cell's side of face F for a face point), of row l of its element matrix, keyed by the offset to
 // the other node.
 constexpr int p2OffsetIndex( const P2StencilOffsets& o, int dx, int dy, int dz )
 {
@@ -76,22 +76,6 @@ constexpr int p2OffsetIndex( const P2StencilOffsets& o, int dx, int dy, int dz )
       if ( o.d[e][0] == dx && o.d[e][1] == dy && o.d[e][2] == dz )
          return e;
    return -1;
-}
-// offset index of node j seen from node l of micro-cell type t, for points of class CLS (face F)
-struct P2OffsetTable
-{
-   int e[6][10][10] = {};
-};
-constexpr P2OffsetTable p2OffsetTable( int cls, int f )
-{
-   P2OffsetTable          tb;
-   const P2StencilOffsets off = p2StencilOffsets( cls, f );
-   for ( int t = 0; t < 6; ++t )
-      for ( int l = 0; l < 10; ++l )
-         for ( int j = 0; j < 10; ++j )
-            tb.e[t][l][j] = p2OffsetIndex( off, p2NodeOffset( t, j, 0 ) - p2NodeOffset( t, l, 0 ), p2NodeOffset( t, j, 1 ) - p2NodeOffset( t, l, 1 ),
-                                           p2NodeOffset( t, j, 2 ) - p2NodeOffset( t, l, 2 ) );
-   return tb;
 }
 constexpr int kP2MaxPairs = 24; // micro-cells of a point: 24 at vertex nodes, fewer in the edge-midpoint classes
 

@@ -441,7 +441,7 @@ MeshCtx::~MeshCtx()
    (void) hipFree( cellInfo );
 }
 
-// Segments of the variable-coefficient sweep: rows y .. y+kElemRows-1, points x0 .. x0+61, planes z0 .. z1-1 of the closed cell, at
+// Segments of the variable-coefficient sweep: row y, points x0 .. x0+61, planes z0 .. z1-1 of the closed cell, at
 // most 32 (the sweep keeps a bit for each).
 void MeshCtx::buildElemSegs( int L )
 {
@@ -451,14 +451,14 @@ void MeshCtx::buildElemSegs( int L )
    const int   N = 1 << L;
    const char* ec = std::getenv( "HYG_ZCHUNK" );
    i64         steps = 0;
-   for ( int y = 0; y <= N; y += kElemRows )
+   for ( int y = 0; y <= N; ++y )
       for ( int x0 = 0; x0 <= N - y; x0 += 62 )
          steps += N - y - x0 + 1;
    const int most  = int( std::max< i64 >( kZSegLeast, std::min< i64 >( kZSegChunk, steps * mesh->nC() / kElemWaves ) ) );
    const int chunk = ec ? std::max( 2, std::min( 32, std::atoi( ec ) ) ) : most;
    for ( int z0 = 0; z0 <= N; z0 += chunk )
       for ( int x0 = 0; x0 <= N - z0; x0 += 62 )
-         for ( int y = 0; y + x0 + z0 <= N; y += kElemRows )
+         for ( int y = 0; y + x0 + z0 <= N; ++y )
             g.eSegsHost.push_back( { y, x0, z0, std::min( z0 + chunk, N - y - x0 + 1 ) } );
    g.nESegs = (int) g.eSegsHost.size();
    g.eSegs  = upload( g.eSegsHost );
@@ -866,10 +866,10 @@ void assembleP2Const( hyg_op_s& op )
    }
 }
 
-// P2ElementwiseOperator< p2_div_k_grad_affine_q4 >: per lattice level and per cell and type the 11 quadrature-point
-// matrices w_q |det J| grad phi(l_q) grad phi(l_q)^T of the micro-cells of level lattice-1, the cell geometry
-// for evaluating the coefficient, and the buffers (coefficient values, partial sums, inverse diagonal) filled
-// on the device.
+// P2ElementwiseOperator< p2_div_k_grad_affine_q4 >: per lattice level and per cell and type the ten products
+// |det J| grad lambda_a . grad lambda_b of the micro-cells of level lattice-1, the cell geometry for evaluating the
+// coefficient, and the buffers (ten moments of the coefficient per micro-cell, partial sums, inverse diagonal) filled on the
+// device.
 void assembleP2DivKGrad( hyg_op_s& op )
 {
    const MeshCtx& mc = op.mesh->ctx;

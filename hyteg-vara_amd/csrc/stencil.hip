@@ -55,8 +55,9 @@ static void stencilT( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol,
    T*             out1 = (T*) c.out1;
    // 1. cell interiors with the one-sided sums of the x = 0 and diagonal faces, the one-sided sums
    // of the z = 0 and y = 0 faces, and macro-edges and -vertices: one launch
-   const int nFace = directFaces( m, g ) ? 0 : g.nChunks - g.firstFaceChunk;
-   SweepArgs< T > p = sweepArgs< T >( m, g, ol, L, c, cfg );
+   const bool     direct = directFaces( m, g );
+   const int      nFace  = direct ? 0 : g.nChunks - g.firstFaceChunk;
+   SweepArgs< T > p      = sweepArgs< T >( m, g, ol, L, c, cfg, direct );
    const int      nLow = p.nChunks;
    const int gL = nLow > 0 ? xcdGrid( ceilDiv( nLow, kBlock / 64 ) ) : 0;
    if ( p.gC + p.gF + gL > 0 )
@@ -77,7 +78,7 @@ static void stencilT( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol,
    // 2. face values from the partial sums
    if ( nFace > 0 )
       hipLaunchKernelGGL( ( kFaceCombine< T, MODE > ), dim3( xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) ), dim3( kBlock ), 0, s,
-                          g.chunks + g.firstFaceChunk, nFace, m.prims, m.entries, m.mesh->nV() + m.mesh->nE(), part, pi,
+                          g.chunks + g.firstFaceChunk, nFace, m.entries, m.mesh->nV() + m.mesh->nE(), part, pi,
                           (const T*) nullptr, L, g.stride, c.flag, x, in1, out0, out1, T( c.a ) );
 }
 
@@ -95,33 +96,16 @@ static void sorT( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol, int
    const int      nLow = g.firstFaceChunk, nFace = g.nChunks - g.firstFaceChunk;
    T*             part = dbl ? (T*) ol.facePart : (T*) ol.facePartF;
    const T*       pi   = dbl ? (const T*) ol.primInv : (const T*) ol.primInvF;
-   SweepArgs< T > p;
-   p.segs    = g.zSegs[cfg];
-   p.nSegs   = g.nZSegs[cfg];
-   p.nC      = m.mesh->nC();
-   p.L       = L;
-   p.flag    = flag;
-   p.stride  = g.stride;
-   p.cellSt  = dbl ? (const T*) ol.cellSt : (const T*) ol.cellStF;
-   p.cfs     = m.cellFaces;
-   p.entryW  = dbl ? (const T*) ol.entryW : (const T*) ol.entryWF;
-   p.primInv = pi;
-   p.part    = part;
-   p.x       = (const T*) xv;
-   p.in1     = (const T*) bv;
-   p.out0    = (T*) xv;
-   p.out1    = (T*) xv;
-   p.a       = T( relax );
-   p.items   = g.flatItems;
-   p.nItems  = nFace > 0 ? g.nFlatItems : 0;
-   p.chunks  = g.chunks;
-   p.nChunks = nLow;
-   p.prims   = m.prims;
-   p.entries = m.entries;
-   p.gC      = p.nSegs > 0 ? xcdGrid( ( ( p.nSegs + 3 ) / 4 ) * p.nC ) : 0;
-   p.gF      = p.nItems > 0 ? xcdGrid( ceilDiv( p.nItems, 4 ) ) : 0;
-   p.cinfo   = m.cellInfo;
-   p.sorM    = m.nColours;
+   StencilCall    c;
+   c.flag = flag;
+   c.x    = xv;
+   c.in1  = bv;
+   c.out0 = xv;
+   c.out1 = xv;
+   c.a    = relax;
+   SweepArgs< T > p = sweepArgs< T >( m, g, ol, L, c, cfg, false );
+   p.cinfo = m.cellInfo;
+   p.sorM  = m.nColours;
    const int gL = nLow > 0 ? xcdGrid( ceilDiv( nLow, kBlock / 64 ) ) : 0;
    for ( int q = 0; q < m.nColours; ++q )
    {
@@ -130,7 +114,7 @@ static void sorT( const MeshCtx& m, LevelGeom& g, const hyg_op_s::Level& ol, int
          hipLaunchKernelGGL( ( kSweep< T, MODE_SOR, 2, 1, 2 > ), dim3( p.gC + p.gF + gL ), dim3( kBlock ), 0, s, p );
       if ( nFace > 0 )
          hipLaunchKernelGGL( ( kFaceCombineSor< T > ), dim3( xcdGrid( ceilDiv( nFace, kBlock / 64 ) ) ), dim3( kBlock ), 0, s,
-                             g.chunks + g.firstFaceChunk, nFace, m.prims, m.entries, m.mesh->nV() + m.mesh->nE(), part, pi,
+                             g.chunks + g.firstFaceChunk, nFace, m.entries, m.mesh->nV() + m.mesh->nE(), part, pi,
                              m.cellInfo, p.sorK, p.sorM, L, g.stride, flag, (T*) xv, (const T*) bv, T( relax ) );
    }
 }

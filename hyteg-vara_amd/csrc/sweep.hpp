@@ -374,7 +374,7 @@ __device__ __forceinline__ void faceFlat( int bid, const int4* __restrict__ item
 // lane are unconditional and independent and issue back to back.
 template < typename T, int MODE >
 __device__ __forceinline__ void lower( int bid, const LowerChunk* __restrict__ chunks, int nChunks,
-                                                    const LowerPrim* __restrict__ prims, const LowerEntry* __restrict__ entries,
+                                                    const LowerEntry* __restrict__ entries,
                                                     const T* __restrict__ entryW, const T* __restrict__ primInv, int L,
                                                     i64 stride, int flag, const T* __restrict__ x, const T* __restrict__ in1,
                                                     T* __restrict__ out0, T* __restrict__ out1, T a, const CellInfo* __restrict__ cinfo,
@@ -476,7 +476,6 @@ struct SweepArgs
    int                 nItems;
    const LowerChunk*   chunks;
    int                 nChunks;
-   const LowerPrim*    prims;
    const LowerEntry*   entries;
    int                 gC, gF;
    const CellInfo*     cinfo = nullptr; // multi-colour SOR: cell colours, the colour of this pass and their number
@@ -500,12 +499,11 @@ inline bool   directFaces( const MeshCtx& m, const LevelGeom& g )
    return g.L <= 5 || ( i64( 2 * m.mesh->nC() ) << ( 2 * g.L ) ) <= kDirectFacePoints;
 }
 
-// arguments of the sweep of one level of the constant operator
+// arguments of the sweep of one level of the constant operator; direct: face points in the launch itself
 template < typename T >
-SweepArgs< T > sweepArgs( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::Level& ol, int L, const StencilCall& c, int cfg )
+SweepArgs< T > sweepArgs( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::Level& ol, int L, const StencilCall& c, int cfg, bool direct )
 {
-   constexpr bool dbl    = std::is_same< T, double >::value;
-   const bool     direct = directFaces( m, g );
+   constexpr bool dbl = std::is_same< T, double >::value;
    SweepArgs< T > p;
    p.segs    = g.zSegs[cfg];
    p.nSegs   = g.nZSegs[cfg];
@@ -527,7 +525,6 @@ SweepArgs< T > sweepArgs( const MeshCtx& m, const LevelGeom& g, const hyg_op_s::
    p.nItems  = direct ? 0 : g.nFlatItems;
    p.chunks  = g.chunks;
    p.nChunks = direct ? g.nChunks : g.firstFaceChunk;
-   p.prims   = m.prims;
    p.entries = m.entries;
    p.gC      = p.nSegs > 0 ? xcdGrid( ( ( p.nSegs + 3 ) / 4 ) * p.nC ) : 0;
    p.gF      = p.nItems > 0 ? xcdGrid( ceilDiv( p.nItems, 4 ) ) : 0;
@@ -544,7 +541,7 @@ __device__ __forceinline__ void bSweep( int b, const SweepArgs< T >& p )
    else if ( b < p.gC + p.gF )
       faceFlat< T >( b - p.gC, p.items, p.nItems, p.L, p.stride, p.cfs, p.entryW, p.part, p.flag, p.x );
    else
-      lower< T, MODE >( b - p.gC - p.gF, p.chunks, p.nChunks, p.prims, p.entries, p.entryW, p.primInv, p.L, p.stride, p.flag,
+      lower< T, MODE >( b - p.gC - p.gF, p.chunks, p.nChunks, p.entries, p.entryW, p.primInv, p.L, p.stride, p.flag,
                         p.x, p.in1, p.out0, p.out1, p.a, p.cinfo, p.sorK, p.sorM );
 }
 
